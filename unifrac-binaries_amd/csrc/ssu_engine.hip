@@ -2,6 +2,7 @@
 // buffer management and the per-method kernel sequence.
 #include "ssu_engine.hpp"
 #include "ssu_kernels.hpp"
+#include "ssu_tiles.hpp"
 #include "ssu_tune.hpp"
 
 #include <hip/hip_runtime.h>
@@ -476,6 +477,15 @@ struct PlanImpl {
     bool bits = false;
     uint32_t ldb = 0;
     std::vector<uint32_t> block_order;  // pair blocks / Gram tiles in launch order
+    // pair tiles over the dense nodes (FP32 weighted): the work list of the full
+    // matrix, a stripe selection's, and the output bands'
+    bool tiled = false;
+    uint32_t n_dense_max = 0;        // the most dense nodes an execution can have
+    TileSet tset, tset_run;
+    struct TileBand { uint32_t unit0, n_units, per_xcd, split0, n_split; };
+    std::vector<TileBand> tile_bands;
+    std::vector<uint32_t> udense;    // bit q: not in urare (the dense nodes of blocked embeddings)
+    bool upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std::string* err);
     // shared-node pair blocks of 32 x 64 samples (FP32 operands, and generalized on
     // either), else 64 x 64 (FP64 weighted)
     bool rect() const { return sparse && (!spec.fp64 || gen); }
@@ -544,7 +554,8 @@ struct PlanImpl {
     DevMem d_knodes, d_klen, d_klen_sum, d_len_all, d_E, d_C, d_U, d_Cu, d_S, d_Spart, d_masks, d_visits, d_order, d_Pt, d_digits, d_chunks, d_G, d_col, d_out,
         d_faith, d_stripes, d_smask, d_dmask, d_pc, d_pidx, d_pval, d_walked, d_rows, d_rcount, d_roff, d_rbsum,
         d_sp_node, d_sp_len, d_umasks, d_B, d_poff, d_pcnt, d_obsum, d_Ssp, d_out2, d_pspmax, d_urare, d_close,
-        d_ridx, d_order_run, d_order_band, d_vdense, d_vrows, d_vlen, d_tau, d_kidx, d_H, d_pcv, d_nbound;
+        d_ridx, d_dlist, d_units, d_split, d_units_run, d_split_run, d_units_band, d_split_band, d_tws, d_udense,
+        d_order_run, d_order_band, d_vdense, d_vrows, d_vlen, d_tau, d_kidx, d_H, d_pcv, d_nbound;
 
     hipStream_t own_st = nullptr;    // created with the plan; st may point at a caller's stream
     // per-execution inputs and output (nullptr: the plan's own table data / totals / result)
@@ -790,9 +801,23 @@ bool PlanImpl::split_weighted(std::string* err) {
     split_thr = thr;
     split_slots = (uint32_t)std::max<uint64_t>(slots, 1);
     urare.assign((K + 31) / 32, 0u);
-    for (uint32_t q = 0; q < K; ++q)
-        if (cnt[q] < thr) urare[q >> 5] |= 1u << (q & 31);
-    return upload(d_urare, urare, st, err);   // (a member: the host copy outlives the upload)
+    udense.assign((K + 31) / 32, 0u);
+    n_dense_max = 0;
+    for (uint32_t q = 0; q < K; ++q) {
+        (cnt[q] < thr ? urare : udense)[q >> 5] |= 1u << (q & 31);
+        n_dense_max += cnt[q] >= thr;
+    }
+    // (members: the host copies outlive the uploads)
+    return upload(d_urare, urare, st, err) && upload(d_udense, udense, st, err);
+}
+
+bool PlanImpl::upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std::string* err) {
+    static const std::vector<TileUnit> none(1, TileUnit{TILE_NONE, 0u});
+    if (!upload(units, t.units.empty() ? none : t.units, st, err) ||
+        !upload(split, t.split.empty() ? none : t.split, st, err))
+        return false;
+    SSU_HIP(hipStreamSynchronize(st));   // (read until here)
+    return true;
 }
 
 // VAW on the shared-node path: nodes held by fewer than theta * n samples of the
@@ -1222,7 +1247,8 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
     }
     // 16 x 16 super-tiles of 64-sample blocks, 6 x 6 of 128-sample Gram tiles:
     // about the number of blocks (tiles) resident on one XCD
-    if (ok && P.sparse) {
+    P.tiled = P.sparse && !P.gen && !spec.fp64;
+    if (ok && P.sparse && !P.tiled) {
         P.block_order = P.rect() ? rect_block_order(P.n) : upper_block_order((P.n + 63) / 64, 16);
         ok = upload(P.d_order, P.block_order, P.st, err);
     }
@@ -1234,6 +1260,17 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
     if (ok && P.gram) ok = P.split_gram(err);   // builds the Gram columns (narrowed when it splits)
     if (ok && P.gram && P.col_node.empty() && !P.build_gram_columns()) ok = false;
     if (ok && P.sparse) ok = P.split_weighted(err);
+    if (ok && P.tiled) {
+        const uint32_t K = (uint32_t)P.knodes.size();
+        if (!P.split_thr) {   // no split: every node is dense
+            P.n_dense_max = K;
+            std::vector<uint32_t> all(K + 1, K);
+            for (uint32_t q = 0; q < K; ++q) all[q + 1] = q;
+            ok = upload(P.d_dlist, all, P.st, err) && hipStreamSynchronize(P.st) == hipSuccess;
+        }
+        P.tset = tile_set(P.n, TILE_ROWS_W, P.n_dense_max, TILE_RESIDENT);
+        ok = ok && P.upload_tiles(P.tset, P.d_units, P.d_split, err);
+    }
     if (ok && P.vsplit) ok = P.split_vaw(err);
     step("occupancy split");
     if (ok && P.gram && P.Kp)
@@ -1352,6 +1389,9 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             SSU_HIP(launch_bits_smask(P.d_smask.as<uint32_t>(), P.d_B.as<uint32_t>(), P.ldb,
                                       P.d_sp_node.as<int32_t>(), Ks, npan, P.st));
     }
+    if (P.tiled && ((split && !P.d_dlist.ensure(((size_t)K + 1) * sizeof(uint32_t), err)) ||
+                    !P.d_tws.ensure(std::max<size_t>(P.tset.slots * TILE_SLOT_W, 1), err)))
+        return false;
     // one embedding block (E holds every sample): the postings of the FP32 split take their
     // values from E, and the gather skips the operand rows of nodes that are never dense
     const bool skip_rare = split && gather && single && !s.vaw && P.d_urare.p;
@@ -1373,8 +1413,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                        P.d_Spart.as<double>(), shared ? P.d_masks.as<uint32_t>() : nullptr,
                                        split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
-                                       skip_rare ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u));
+                                       split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled));
             if (gather && s.vaw)
                 SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
                                            (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st));
@@ -1417,6 +1457,10 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.out2 = P.gen || vsplit ? P.d_out2.p : nullptr;
         b.pspmax = P.gen ? P.d_pspmax.as<double>() : nullptr;
         b.band = P.band;
+        if (P.tiled) {
+            b.dlist = P.d_dlist.as<uint32_t>();
+            if (!skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
+        }
         if (vsplit) {
             const bool unw = s.method == Method::unweighted || s.method == Method::unweighted_unnormalized;
             b.vaw = s.method == Method::generalized ? 3 : unw ? 2 : 1;
@@ -1508,6 +1552,47 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         }
         SSU_HIP(combine(0, P.n));
         SSU_HIP(P.mark(4));
+    } else if (P.tiled) {
+        TileArgs a{};
+        a.U = P.d_U.p;
+        a.ldn = P.ldn;
+        a.dlist = P.d_dlist.as<uint32_t>();
+        a.n = P.n;
+        a.S = P.S_ptr();
+        a.normalized = s.method == Method::weighted_normalized;
+        a.out = P.out_ptr();
+        a.add_partial = split;
+        a.ws = P.d_tws.as<double>();
+        const uint32_t nbands = P.banded_run ? (uint32_t)P.band_ev.size() : 1;
+        if (P.banded_run && nbands > 1) {
+            SSU_HIP(hipEventRecord(P.band_go, P.st));
+            SSU_HIP(hipStreamWaitEvent(P.band_st2, P.band_go, 0));
+        }
+        for (uint32_t k = 0; k < nbands; ++k) {
+            hipStream_t bs = P.st;
+            if (P.banded_run) {
+                const PlanImpl::TileBand& tb = P.tile_bands[k];
+                a.units = P.d_units_band.as<TileUnit>() + tb.unit0;
+                a.n_units = tb.n_units;
+                a.per_xcd = tb.per_xcd;
+                a.split = P.d_split_band.as<TileUnit>() + tb.split0;
+                a.n_split = tb.n_split;
+                if (k & 1) bs = P.band_st2;
+            } else {
+                const TileSet& t = P.band_all ? P.tset : P.tset_run;
+                a.units = (P.band_all ? P.d_units : P.d_units_run).as<TileUnit>();
+                a.n_units = (uint32_t)t.units.size();
+                a.per_xcd = t.per_xcd;
+                a.split = (P.band_all ? P.d_split : P.d_split_run).as<TileUnit>();
+                a.n_split = (uint32_t)t.split.size();
+            }
+            SSU_HIP(launch_tiles_w32(a, bs));
+            if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
+        }
+        if (P.banded_run && nbands > 1)   // the later work on st reads every band
+            SSU_HIP(hipStreamWaitEvent(P.st, P.band_ev[(nbands - 2) | 1], 0));   // the last band on band_st2
+        SSU_HIP(P.mark(3));
+        SSU_HIP(P.mark(4));
     } else if (P.sparse) {
         SparseArgs a{};
         a.U = s.fp64 ? P.d_E.p : P.d_U.p;
@@ -1541,8 +1626,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             }
             if (P.gen && s.fp64) SSU_HIP(launch_pairs_gen64(a, s.alpha, split ? P.d_out2.p : nullptr, bs));
             else if (P.gen) SSU_HIP(launch_pairs_gen32(a, (float)s.alpha, split ? P.d_out2.p : nullptr, bs));
-            else if (s.fp64) SSU_HIP(launch_pairs_sparse(true, a, bs));
-            else SSU_HIP(launch_pairs_sparse32(a, bs));
+            else SSU_HIP(launch_pairs_sparse(true, a, bs));
             if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
         }
         if (P.banded_run && nbands > 1)   // the later work on st reads every band
@@ -1654,7 +1738,7 @@ bool Plan::refines() const { return p_->refine_on; }
 // samples; Gram: 128-sample tile rows, band 0 holding every diagonal tile).
 bool PlanImpl::prepare_bands(std::string* err) {
     if (!band_ev.empty()) return true;
-    const uint32_t ei = gram ? GRAM_BM : (rect() ? 32 : 64);
+    const uint32_t ei = gram ? GRAM_BM : tiled ? TILE_ROWS_W : (rect() ? 32 : 64);
     const uint32_t nbi = (n + ei - 1) / ei;
     // the Gram path's bands are cheaper to compute than to copy: more, smaller ones
     // (16 bands measured 27.0 ms against 28.1 ms for 10 at 16,384 samples; the
@@ -1672,9 +1756,18 @@ bool PlanImpl::prepare_bands(std::string* err) {
     for (uint32_t k = 0; k <= nb; ++k) cut[k] = (uint32_t)std::llround(nbi * wsum[k] / wsum[nb]);
     for (uint32_t k = 1; k <= nb; ++k) cut[k] = std::max(cut[k], cut[k - 1]);   // (monotone; empty bands allowed)
     std::vector<uint32_t> ord;
+    TileSet tb;
     band_off.assign(1, 0u);
     band_row0.clear();
+    tile_bands.clear();
     for (uint32_t k = 0; k < nb; ++k) {
+        if (tiled) {
+            const TileSet t = tile_subset(tset, [&](uint32_t bi, uint32_t) { return bi >= cut[k] && bi < cut[k + 1]; });
+            tile_bands.push_back({(uint32_t)tb.units.size(), (uint32_t)t.units.size(), t.per_xcd,
+                                  (uint32_t)tb.split.size(), (uint32_t)t.split.size()});
+            tb.units.insert(tb.units.end(), t.units.begin(), t.units.end());
+            tb.split.insert(tb.split.end(), t.split.begin(), t.split.end());
+        }
         for (uint32_t bij : block_order) {
             const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
             const bool in_band = bi >= cut[k] && bi < cut[k + 1];
@@ -1684,6 +1777,7 @@ bool PlanImpl::prepare_bands(std::string* err) {
         band_row0.push_back(std::min(n, cut[k] * ei));
     }
     band_row0.push_back(n);
+    if (tiled && !upload_tiles(tb, d_units_band, d_split_band, err)) return false;
     if (!upload(d_order_band, ord.empty() ? std::vector<uint32_t>{0u} : ord, st, err)) return false;
     SSU_HIP(hipStreamSynchronize(st));   // `ord` is read until here
     if (!copy_st) SSU_HIP(hipStreamCreateWithFlags(&copy_st, hipStreamNonBlocking));
@@ -1700,7 +1794,8 @@ bool Plan::execute_to_host(void* host, std::string* err) {
     // paths write their output in one final pass)
     static const bool off = getenv("SSU_OUT_BANDS") && atoi(getenv("SSU_OUT_BANDS")) == 0;
     const bool gram_bands = P.gram && P.Kp;   // (no Gram columns: one fill, nothing to band)
-    if (off || !(P.sparse || gram_bands) || !P.band_all || P.n < 4096 || P.block_order.empty())
+    if (off || !(P.sparse || gram_bands) || !P.band_all || P.n < 4096 ||
+        (P.tiled ? P.tset.units.empty() : P.block_order.empty()))
         return execute(err) && copy_matrix(host, err);
     if (!P.prepare_bands(err)) return false;
     const size_t es = P.spec.fp64 ? sizeof(double) : sizeof(float);
@@ -1765,12 +1860,20 @@ bool Plan::set_stripes(uint32_t start, uint32_t stop, std::string* err) {
         P.band = GapBand();
         P.band_all = true;
         P.run_order.clear();
+        P.tset_run = TileSet();
         return true;
     }
     P.band = stripe_band(P.n, start, stop);
     P.band_all = false;
     // the blocks / tiles of the kernel's order that hold a selected pair
     P.run_order.clear();
+    if (P.tiled) {
+        P.tset_run = tile_subset(P.tset, [&](uint32_t bi, uint32_t bj) {
+            return P.band.meets_tile(bi * TILE_ROWS_W, std::min(P.n, (bi + 1) * TILE_ROWS_W), bj * TILE_COLS,
+                                     std::min(P.n, (bj + 1) * TILE_COLS));
+        });
+        return P.upload_tiles(P.tset_run, P.d_units_run, P.d_split_run, err);
+    }
     uint32_t ei = 0, ej = 0;   // block edges (rows, columns)
     if (P.gram) ei = ej = GRAM_BM;
     else if (P.sparse && !P.rect()) ei = ej = 64;
@@ -1929,6 +2032,11 @@ uint64_t Plan::kernel_terms() const {
     const PlanImpl& P = *p_;
     const uint64_t K = P.knodes.size();
     if (P.gram) return (uint64_t)P.order_used().size() * GRAM_BM * GRAM_BM * (uint64_t)P.Kp;
+    if (P.tiled) {
+        uint32_t nd = 0;
+        if (!P.d_dlist.p || hipMemcpy(&nd, P.d_dlist.p, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess) return 0;
+        return (P.band_all ? P.tset : P.tset_run).tiles * TILE_ROWS_W * TILE_COLS * nd;
+    }
     if (P.sparse) {
         // visited nodes per block, times the pairs a block evaluates
         const size_t nbi = P.rect() ? (P.n + 31) / 32 : (P.n + 63) / 64, nbj = (P.n + 63) / 64;
@@ -1961,6 +2069,7 @@ double Plan::split_theta() const {
     if (P.gram) return P.gsplit_slots ? P.split_theta : 0.0;
     return P.split_thr ? (double)P.split_thr / std::max<uint32_t>(P.n, 1) : 0.0;
 }
+// (the names of the paths; programs compare them)
 const char* Plan::main_kernel() const {
     if (p_->gram) return "k_gram_i8r";
     if (p_->sparse)

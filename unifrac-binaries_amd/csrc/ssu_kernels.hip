@@ -8,6 +8,7 @@
 //                 (src/unifrac_task_impl.hpp formulas), FP32 with FP64 merges or FP64
 //   Faith PD      src/unifrac.cpp:362-387, same FP64 summation order
 #include "ssu_kernels.hpp"
+#include "ssu_tiles.hpp"
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -187,7 +188,8 @@ __global__ void __launch_bounds__(256) k_bits_paths(uint32_t* __restrict__ B, ui
 
 // Segmented pass over the processed rows: blockIdx.y owns rows [k0, k1), k0 a
 // multiple of 32.  Per thread (sample s) and row r, e = E[knodes[r]][s]:
-//   GATHER: U[r][s] = (float)e
+//   GATHER: U[r][s] = (float)e; rare rows (bit r of rare_u) only with write_rare;
+//           with scale_u the other rows hold (float)(klen[r] * e)
 //   SUMS:   Spart[seg][s] = sum_{r in seg} klen[r] * e', increasing r, where e'
 //           is e as the pair kernels see it ((float)e when GATHER, else e)
 //   MASKS:  bit (r % 32) of masks[panel][r / 32] = any e > 0 over the 32
@@ -203,7 +205,8 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums(float* __restrict__
                                                              const int32_t* __restrict__ knodes,
                                                              const double* __restrict__ klen, uint32_t K,
                                                              uint32_t rows_per_seg, uint32_t n_valid,
-                                                             const uint32_t* __restrict__ skip_u) {
+                                                             const uint32_t* __restrict__ rare_u, int write_rare,
+                                                             int scale_u) {
     const size_t s = (size_t)blockIdx.x * EMB_THREADS + threadIdx.x;
     if (s >= lde) return;
     const bool real = s < n_valid;   // columns past the last sample never enter a mask
@@ -217,7 +220,8 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums(float* __restrict__
         double e = E[(size_t)knodes[r] * lde + s];
         if constexpr (GATHER) {
             const float f = (float)e;
-            if (!skip_u || !((skip_u[r >> 5] >> (r & 31)) & 1u)) U[(size_t)r * ldu + col0 + s] = f;
+            const bool rare = rare_u && ((rare_u[r >> 5] >> (r & 31)) & 1u);
+            if (!rare || write_rare) U[(size_t)r * ldu + col0 + s] = scale_u && !rare ? (float)(klen[r] * e) : f;
             e = (double)f;
         }
         if constexpr (SUMS) acc += klen[r] * e;
@@ -269,7 +273,8 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums2(float* __restrict_
                                                               const int32_t* __restrict__ knodes,
                                                               const double* __restrict__ klen, uint32_t K,
                                                               uint32_t rows_per_seg, uint32_t n_valid,
-                                                              const uint32_t* __restrict__ skip_u) {
+                                                              const uint32_t* __restrict__ rare_u, int write_rare,
+                                                              int scale_u) {
     const size_t s = 2 * ((size_t)blockIdx.x * EMB_THREADS + threadIdx.x);   // samples s, s + 1
     const size_t wave0 = s & ~(size_t)127;            // the wave's first sample
     if (wave0 >= lde) return;                         // (whole waves only)
@@ -293,8 +298,12 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums2(float* __restrict_
         }
         if constexpr (GATHER) {
             const float f0 = (float)e0, f1 = (float)e1;
-            if (in && (!skip_u || !((skip_u[r >> 5] >> (r & 31)) & 1u)))
-                *reinterpret_cast<float2*>(U + (size_t)r * ldu + col0 + s) = make_float2(f0, f1);
+            const bool rare = rare_u && ((rare_u[r >> 5] >> (r & 31)) & 1u);   // (uniform)
+            if (in && (!rare || write_rare)) {
+                float2 x = make_float2(f0, f1);
+                if (scale_u && !rare) x = make_float2((float)(klen[r] * e0), (float)(klen[r] * e1));
+                *reinterpret_cast<float2*>(U + (size_t)r * ldu + col0 + s) = x;
+            }
             e0 = (double)f0;
             e1 = (double)f1;
         }
@@ -1525,16 +1534,6 @@ __device__ __forceinline__ void pairs_sparse32_body(const V* __restrict__ U, con
         }
 }
 
-template <class TOut>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_pairs_sparse32(
-        const float* __restrict__ U, size_t ldn, const double* __restrict__ len, const uint32_t* __restrict__ masks,
-        uint32_t Kw, uint32_t n, const double* __restrict__ S, int normalized, TOut* __restrict__ out,
-        uint32_t* __restrict__ visits, const uint32_t* __restrict__ order, uint32_t n_blocks, uint32_t per_xcd,
-        const uint32_t* __restrict__ dmask, int add_partial) {
-    pairs_sparse32_body<TOut, false>(U, nullptr, ldn, len, masks, Kw, n, S, normalized, out, visits, order, n_blocks,
-                                     per_xcd, dmask, add_partial, 0.0f, nullptr);
-}
-
 // generalized: numerator and denominator summed directly (two accumulator sets, 2 waves per SIMD)
 template <class TOut, bool HALF = false>
 __global__ void __launch_bounds__(64) k_pairs_gen32(
@@ -2736,25 +2735,26 @@ template <bool G, bool S, bool M>
 static void gather_sums_t(dim3 grid, hipStream_t st, float* U, size_t ldu, uint32_t col0, double* Spart,
                           uint32_t* masks, uint32_t Kw, uint32_t* smask, const double* E, size_t lde,
                           const int32_t* knodes, const double* klen, uint32_t K, uint32_t rps, uint32_t n_valid,
-                          const uint32_t* skip_u) {
+                          const uint32_t* rare_u, bool write_rare, bool scale_u) {
     // two samples per thread where the layout allows 16-byte loads (SSU_GATHER2=0: one)
     static const bool two_ok = !(getenv("SSU_GATHER2") && atoi(getenv("SSU_GATHER2")) == 0);
     if (two_ok && lde % 2 == 0 && col0 % 2 == 0 && ldu % 2 == 0) {
         const dim3 g2(grid1(lde / 2, EMB_THREADS), grid.y);
         hipLaunchKernelGGL((k_gather_sums2<G, S, M>), g2, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart, masks, Kw,
-                           smask, E, lde, knodes, klen, K, rps, n_valid, skip_u);
+                           smask, E, lde, knodes, klen, K, rps, n_valid, rare_u, (int)write_rare, (int)scale_u);
         return;
     }
     hipLaunchKernelGGL((k_gather_sums<G, S, M>), grid, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart, masks, Kw,
-                       smask, E, lde, knodes, klen, K, rps, n_valid, skip_u);
+                       smask, E, lde, knodes, klen, K, rps, n_valid, rare_u, (int)write_rare, (int)scale_u);
 }
 
 hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* masks, uint32_t* smask,
                               const double* E, size_t lde, uint32_t col0, const int32_t* knodes, const double* klen,
-                              uint32_t K, uint32_t n, hipStream_t st, const uint32_t* skip_u, uint32_t rps_fixed) {
+                              uint32_t K, uint32_t n, hipStream_t st, const uint32_t* rare_u, uint32_t rps_fixed, bool write_rare, bool scale_u) {
     if (masks && (lde % 64 || col0 % 64)) return hipErrorInvalidValue;
     if (rps_fixed % 32) return hipErrorInvalidValue;
     if (smask && !masks) return hipErrorInvalidValue;
+    if (scale_u && !klen) return hipErrorInvalidValue;
     if (col0 >= n) return hipSuccess;
     const uint32_t cnt = (uint32_t)std::min<size_t>(lde, n - col0);   // real samples in this block
     if (!K) {
@@ -2772,13 +2772,13 @@ hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, ui
     const dim3 grid(cb, segs);
     const int key = (U ? 4 : 0) | (S ? 2 : 0) | (masks ? 1 : 0);
     switch (key) {
-    case 7: gather_sums_t<true, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 6: gather_sums_t<true, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 5: gather_sums_t<true, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 4: gather_sums_t<true, false, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 3: gather_sums_t<false, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 2: gather_sums_t<false, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
-    case 1: gather_sums_t<false, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, skip_u); break;
+    case 7: gather_sums_t<true, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 6: gather_sums_t<true, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 5: gather_sums_t<true, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 4: gather_sums_t<true, false, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 3: gather_sums_t<false, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 2: gather_sums_t<false, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 1: gather_sums_t<false, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
     case 0: return hipSuccess;
     default: return hipErrorInvalidValue;
     }
@@ -2877,13 +2877,6 @@ std::vector<uint32_t> rect_block_order(uint32_t n) {
     return order;
 }
 
-template <class TOut>
-static void pairs_sparse32_t(uint32_t grid, hipStream_t st, const SparseArgs& a, uint32_t per_xcd) {
-    hipLaunchKernelGGL((k_pairs_sparse32<TOut>), dim3(grid), dim3(64), 0, st, (const float*)a.U, a.ldn, a.len, a.masks,
-                       a.Kw, a.n, a.S, (int)a.normalized, (TOut*)a.out, a.visits, a.order, a.n_blocks, per_xcd,
-                       a.dmask, (int)(a.dmask != nullptr));
-}
-
 static bool sparse_args_ok(const SparseNodesArgs& a) {
     // posting slots are addressed with 32-bit offsets (bytes included)
     const bool common = a.dmask && a.smask && a.pc && a.pidx && a.poff && a.len && a.rows && a.rcount && a.roff &&
@@ -2905,6 +2898,8 @@ hipError_t launch_sparse_lists(const SparseNodesArgs& a, hipStream_t st) {
         const uint32_t nb = (uint32_t)((a.K + SCAN_BLOCK - 1) / SCAN_BLOCK);
         hipLaunchKernelGGL(k_node_split, dim3(gk), dim3(64), 0, st, a.dmask, a.pcnt, a.smask, a.K, a.npan, a.thr,
                            a.fixed_dense);
+        if (a.dlist)
+            if (const hipError_t e = launch_dense_list(a.dlist, a.dmask, a.K, st)) return e;
         hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(SCAN_T), 0, st, a.obsum, a.pcnt, (size_t)a.K);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(SCAN_T), 0, st, a.obsum, nb);
         hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(SCAN_T), 0, st, a.poff, a.pcnt, a.obsum, (size_t)a.K, nb);
@@ -3110,18 +3105,6 @@ hipError_t launch_pairs_gen64(const SparseArgs& a, double alpha, void* out2, hip
     hipLaunchKernelGGL(k_pairs_gen64, dim3(per_xcd * N_XCDS), dim3(64), 0, st, (const double*)a.U, a.rows, a.ldn,
                        a.len, a.masks, a.Kw, a.n, (double*)a.out, (double*)out2, a.visits, a.order, a.n_blocks,
                        per_xcd, a.dmask, (int)(a.dmask != nullptr), alpha);
-    return hipGetLastError();
-}
-
-hipError_t launch_pairs_sparse32(const SparseArgs& a, hipStream_t st) {
-    if (a.ldn % S3_BJ) return hipErrorInvalidValue;
-    const uint32_t nbi = (a.n + S3_BI - 1) / S3_BI, nbj = (a.n + S3_BJ - 1) / S3_BJ;
-    if (!nbi) return hipSuccess;
-    if ((size_t)nbj * S3_BJ > a.ldn || nbi > 65535 || !a.order) return hipErrorInvalidValue;
-    if (!a.n_blocks) return hipSuccess;   // a stripe selection without a block here
-    const uint32_t per_xcd = (a.n_blocks + N_XCDS - 1) / N_XCDS;
-    if (a.out_fp64) pairs_sparse32_t<double>(per_xcd * N_XCDS, st, a, per_xcd);
-    else pairs_sparse32_t<float>(per_xcd * N_XCDS, st, a, per_xcd);
     return hipGetLastError();
 }
 

@@ -122,15 +122,17 @@ hipError_t launch_bits_smask(uint32_t* smask, const uint32_t* B, uint32_t ldb, c
 //   masks (if non-null; lde, col0 multiples of 64): [ldn/32][ceil(K/32)] words, bit r%32 of
 //     word r/32 of panel p set iff some sample of p*32..p*32+31 has u_rs > 0;
 //   smask (if non-null, with masks): [ldn/32][K] words, bit s%32 of smask[s/32][r] = u_rs > 0;
-//   skip_u (optional, [ceil(K/32)] words): rows r with bit r set are not written to U (S and
-//     the masks still see their FP32-rounded values).
+//   rare_u (optional, [ceil(K/32)] words): rows r with bit r set are not written to U (S and
+//     the masks still see their FP32-rounded values), unless write_rare;
+//   scale_u: U[r] = (float)(klen[r] * E[knodes[r]]) instead (one rounding), the rare rows excepted.
 uint32_t gather_segments(uint32_t K, size_t ldn);
 //   rps_fixed (optional, a multiple of 32): rows per segment, in place of the
 //     default that depends on lde (S then depends on a sample's column alone).
 hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* masks, uint32_t* smask,
                               const double* E,
                               size_t lde, uint32_t col0, const int32_t* knodes, const double* klen, uint32_t K,
-                              uint32_t n, hipStream_t st, const uint32_t* skip_u = nullptr, uint32_t rps_fixed = 0);
+                              uint32_t n, hipStream_t st, const uint32_t* rare_u = nullptr, uint32_t rps_fixed = 0,
+                              bool write_rare = false, bool scale_u = false);
 // rows per segment that depends on K alone (for launch_gather_sums)
 uint32_t fixed_rows_per_segment(uint32_t K);
 // Faith PD: out[s] = sum over all non-root nodes k in postorder of (E[k][s] > 0) * len[k]
@@ -269,6 +271,8 @@ struct SparseNodesArgs {
     double* gram = nullptr; // unweighted: the Gram tiles of launch_gram_i8
     uint32_t n_pad = 0;     // their padded edge
     GapBand band;           // rows walk (and write) only the columns of selected pairs (G(a, a) always)
+    // optional: the dense nodes of this execution, dlist[0] = their number, then their indices
+    uint32_t* dlist = nullptr;
     // dense nodes fixed in advance ([ceil(K/32)] words, in place of the occupancy test)
     const uint32_t* fixed_dense = nullptr;
     // VAW (1: weighted values, 2: presence, 3: generalized, 0 <= alpha <= 1): numerator shares
@@ -310,11 +314,9 @@ size_t row_list_scan_blocks(uint32_t n, uint32_t K);
 // super-tile by super-tile; kernels walk it in XCD-contiguous runs.
 std::vector<uint32_t> upper_block_order(uint32_t nb, uint32_t super);
 hipError_t launch_pairs_sparse(bool in_fp64, const SparseArgs& a, hipStream_t st);
-// FP32 operands: 32 x 64 blocks (32-sample row panel pi <= 2 pj + 1, 64-sample
-// column panel pj), FP32 terms merged into FP64; `order` = rect_block_order(n)
-// and visits is [ceil(n/32)][ceil(n/64)].
+// 32 x 64 blocks (32-sample row panel pi <= 2 pj + 1, 64-sample column panel pj):
+// `order` = rect_block_order(n) and visits is [ceil(n/32)][ceil(n/64)].
 std::vector<uint32_t> rect_block_order(uint32_t n);
-hipError_t launch_pairs_sparse32(const SparseArgs& a, hipStream_t st);
 // generalized (FP32, 0 <= alpha <= 1) on the same blocks: numerator and denominator summed
 // directly over the nodes either panel holds; with dmask, adds the posting-list shares in
 // out (numerator) and out2 (denominator)

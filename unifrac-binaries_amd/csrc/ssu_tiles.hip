@@ -1,0 +1,376 @@
+// Pair tiles over the dense nodes (gfx950).
+//
+// Every dense node is held by a sizeable share of the samples, so every pair
+// block visits it: the kernels are dense contractions with |x_i - x_j| in
+// place of the product, which no matrix instruction forms.  They are laid out
+// like a vector-ALU GEMM: 128 columns per tile, four waves of (rows / 2) x 64
+// pairs, a lane holding groups of four rows and four columns 32 apart, so that
+// its operands are ds_read_b128 of 8 distinct contiguous 16-byte pieces (no
+// bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
+// to LDS by global_load_lds, 16 bytes per lane, a stage of nodes ahead.
+#include "ssu_tiles.hpp"
+
+#include <algorithm>
+
+namespace ssu {
+
+namespace {
+
+constexpr uint32_t N_XCDS = 8;
+
+#define SSU_GLOBAL(p) ((const __attribute__((address_space(1))) void*)(p))
+#define SSU_LDS(p) ((__attribute__((address_space(3))) void*)(p))
+
+// nodes [a, b) of part p of np: whole stages of eb nodes
+__device__ __forceinline__ void part_range(uint32_t nd, uint32_t eb, uint32_t p, uint32_t np, uint32_t& a, uint32_t& b) {
+    const uint32_t st = (nd + eb - 1) / eb;
+    a = (uint32_t)((uint64_t)st * p / np) * eb;
+    b = min(nd, (uint32_t)((uint64_t)st * (p + 1) / np) * eb);
+    a = min(a, nd);
+}
+
+// ------------------------------------------------------------------ terms
+//
+// An operation says what a lane holds and how a node's values enter a pair:
+//   V        operand type; FP32 sums are merged into FP64 every MERGE nodes
+//   RL       rows a lane holds (8, or 4 with two sums per pair), so a tile has 16 RL rows
+//   EB       nodes per LDS stage (two stages are resident)
+//   TWO      a denominator is summed beside the numerator
+//   LEN      the node's length is staged too (otherwise U's rows are scaled by it)
+constexpr uint32_t MERGE = 64;
+
+// FP32 weighted: |l u - l v|, two full-rate instructions
+struct OpW32 {
+    typedef float V;
+    static constexpr int RL = 8, EB = 16;
+    static constexpr bool TWO = false, LEN = false;
+    static __device__ __forceinline__ void term(float u, float v, float, float& num, float&) {
+        num += __builtin_fabsf(u - v);
+    }
+    // d from the tile's sum x and the rare nodes' share of it
+    static __device__ __forceinline__ double distance(double x, double share, double tot, bool normalized) {
+        x += share;
+        x = x < 0.0 ? 0.0 : x;   // the share's rounding can undershoot 0; NaN (empty samples) passes
+        return normalized ? x / tot : x;
+    }
+};
+
+template <class OP> struct Shape {
+    typedef typename OP::V V;
+    static constexpr uint32_t ROWS = 16 * OP::RL;               // of a tile: two waves of 8 RL
+    static constexpr uint32_t WAVE_ROWS = 8 * OP::RL;
+    static constexpr uint32_t NODE = ROWS + TILE_COLS;          // staged values of a node
+    static constexpr uint32_t PAIRS = OP::RL * 8;               // of a lane
+    static constexpr bool MIXED = sizeof(V) == 4;
+    // row of the lane's q-th row in its wave's rows, column of its q-th column in its wave's 64 columns
+    static __device__ __forceinline__ uint32_t row_at(uint32_t li, uint32_t q) { return (q >> 2) * 32 + li * 4 + (q & 3); }
+    static __device__ __forceinline__ uint32_t col_at(uint32_t lj, uint32_t q) { return (q >> 2) * 32 + lj * 4 + (q & 3); }
+};
+
+// four consecutive values of LDS (one 16-byte read, or two)
+template <class V> __device__ __forceinline__ void read4(V (&x)[4], const V* p) {
+    typedef __attribute__((ext_vector_type(16 / sizeof(V)))) V vec;
+    constexpr int N = 16 / sizeof(V);
+#pragma unroll
+    for (int h = 0; h < 4 / N; ++h) {
+        const vec v = reinterpret_cast<const vec*>(p)[h];
+#pragma unroll
+        for (int z = 0; z < N; ++z) x[h * N + z] = v[z];
+    }
+}
+
+// the distance of pair i < j, written to both triangles
+template <class OP>
+__device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j, double x) {
+    typedef typename OP::V V;
+    V* out = (V*)g.out;
+    const double share = g.add_partial ? (double)out[i * g.n + j] : 0.0;   // the rare nodes', from the posting walk
+    const double d = OP::distance(x, share, g.normalized ? g.S[i] + g.S[j] : 0.0, g.normalized);
+    out[i * g.n + j] = (V)d;
+    out[j * g.n + i] = (V)d;
+}
+
+template <class OP>
+__global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
+    typedef Shape<OP> SH;
+    typedef typename OP::V V;
+    constexpr int RL = OP::RL;
+    constexpr uint32_t EB = OP::EB;
+    const uint32_t seq = (blockIdx.x % N_XCDS) * g.per_xcd + blockIdx.x / N_XCDS;
+    if (seq >= g.n_units) return;
+    const uint32_t bij = g.units[seq].bij, part = g.units[seq].part;
+    if (bij == TILE_NONE) return;
+    const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
+    __shared__ __attribute__((aligned(16))) V sv[2][EB][SH::NODE];   // a node: its rows, then its columns
+    __shared__ V sl[2][EB];
+
+    const uint32_t nd = g.dlist[0];
+    const uint32_t np = (part & 63u) + 1;
+    uint32_t ka, kb;
+    part_range(nd, EB, (part >> 6) & 63u, np, ka, kb);
+
+    V num[RL][8];
+    double num64[SH::MIXED ? RL : 1][SH::MIXED ? 8 : 1];
+#pragma unroll
+    for (int r = 0; r < RL; ++r)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            num[r][c] = V(0);
+            if constexpr (SH::MIXED) num64[r][c] = 0.0;
+        }
+
+    // wave w stages nodes w, w + 4, ..: 16 bytes per lane, rows then columns
+    constexpr uint32_t VEC = 16 / sizeof(V), RLANES = SH::ROWS / VEC, CLANES = TILE_COLS / VEC;
+    const V* U = (const V*)g.U;
+    const uint32_t* dl = g.dlist + 1;
+    const uint32_t i0 = bi * SH::ROWS, j0 = bj * TILE_COLS;
+    // the rows of the wave's nodes of the stage after the next one to be loaded, read ahead of their use
+    uint32_t row_next[EB / 4];
+    V len_next = V(0);
+    auto index = [&](uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t e = 0; e < EB / 4; ++e) row_next[e] = dl[min(k0 + wave + 4 * e, kb - 1)];
+        if (g.rows) {
+#pragma unroll
+            for (uint32_t e = 0; e < EB / 4; ++e) row_next[e] = (uint32_t)g.rows[row_next[e]];
+        }
+        if constexpr (OP::LEN) len_next = threadIdx.x < EB ? (V)g.len[dl[min(k0 + threadIdx.x, kb - 1)]] : V(0);
+    };
+    // stages nodes k0 .. (those past the end are zeros, which add nothing) and reads the indices of the next ones
+    auto stage = [&](int buf, uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t e = 0; e < EB / 4; ++e) {
+            const uint32_t ee = wave + 4 * e;
+            const V* u = U + (size_t)row_next[e] * g.ldn;
+            V* to = &sv[buf][ee][0];
+            if constexpr (RLANES + CLANES <= 64) {
+                const V* src = u + (lane < RLANES ? i0 + lane * VEC : j0 + (lane - RLANES) * VEC);
+                if (RLANES + CLANES == 64 || lane < RLANES + CLANES)
+                    __builtin_amdgcn_global_load_lds(SSU_GLOBAL(src), SSU_LDS(to), 16, 0, 0);
+            } else {
+                static_assert(CLANES == 64 && RLANES <= 64, "a node is staged by one or two instructions");
+                if (RLANES == 64 || lane < RLANES)
+                    __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + i0 + lane * VEC), SSU_LDS(to), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + j0 + lane * VEC), SSU_LDS(to + SH::ROWS), 16, 0, 0);
+            }
+        }
+        if constexpr (OP::LEN) if (threadIdx.x < EB) sl[buf][threadIdx.x] = len_next;
+        if (k0 + EB < kb) index(k0 + EB);
+    };
+    auto node = [&](int buf, uint32_t e) __attribute__((always_inline)) {
+        V a[RL / 4][4], b[2][4];
+#pragma unroll
+        for (int h = 0; h < RL / 4; ++h) read4(a[h], &sv[buf][e][wr + 32 * h + li * 4]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) read4(b[h], &sv[buf][e][SH::ROWS + wc + 32 * h + lj * 4]);
+        const V l = OP::LEN ? sl[buf][e] : V(0);
+        V none = V(0);
+#pragma unroll
+        for (int r = 0; r < RL; ++r)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) OP::term(a[r >> 2][r & 3], b[c >> 2][c & 3], l, num[r][c], none);
+    };
+    auto merge = [&]() __attribute__((always_inline)) {
+        if constexpr (SH::MIXED) {
+#pragma unroll
+            for (int r = 0; r < RL; ++r)
+#pragma unroll
+                for (int c = 0; c < 8; ++c) { num64[r][c] += (double)num[r][c]; num[r][c] = V(0); }
+        }
+    };
+
+    if (ka < kb) {   // uniform
+        index(ka);
+        stage(0, ka);
+        __syncthreads();
+        int buf = 0;
+        uint32_t span = 0;
+        for (uint32_t k0 = ka; k0 < kb; k0 += EB) {
+            if (k0 + EB < kb) stage(buf ^ 1, k0 + EB);
+            else if (k0 + EB > kb) {   // (uniform) the last, partial stage: its missing nodes zero
+                for (uint32_t q = (kb - k0) * SH::NODE + threadIdx.x; q < EB * SH::NODE; q += 256)
+                    (&sv[buf][0][0])[q] = V(0);
+                __syncthreads();
+            }
+#pragma unroll
+            for (uint32_t e = 0; e < EB; ++e) node(buf, e);
+            span += EB;
+            if (span == MERGE) { merge(); span = 0; }
+            __syncthreads();
+            buf ^= 1;
+        }
+        merge();
+    }
+
+    if (np > 1) {   // this part's sums to its slot, [pair of the lane][thread], for k_tiles_finish
+        double* w = g.ws + (size_t)(part >> 12) * (SH::PAIRS * 256) + threadIdx.x;
+#pragma unroll
+        for (int r = 0; r < RL; ++r)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if constexpr (SH::MIXED) w[(r * 8 + c) * 256] = num64[r][c];
+                else w[(r * 8 + c) * 256] = num[r][c];
+            }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < RL; ++r)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const size_t i = i0 + wr + SH::row_at(li, r), j = j0 + wc + SH::col_at(lj, c);
+            double x;
+            if constexpr (SH::MIXED) x = num64[r][c];
+            else x = num[r][c];
+            if (i < j && j < g.n) write_pair<OP>(g, i, j, x);
+            else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
+        }
+}
+
+// The tiles cut into parts: the parts' sums in order, then the distances.
+// blockIdx.y: one of the lane's rows.
+template <class OP>
+__global__ void __launch_bounds__(256) k_tiles_finish(TileArgs g) {
+    typedef Shape<OP> SH;
+    typedef typename OP::V V;
+    const uint32_t bij = g.split[blockIdx.x].bij, part = g.split[blockIdx.x].part;
+    const uint32_t bi = bij >> 16, bj = bij & 0xffffu, np = (part & 63u) + 1, r = blockIdx.y;
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
+    const double* w = g.ws + (size_t)(part >> 12) * (SH::PAIRS * 256) + threadIdx.x;
+    double x[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) x[c] = 0.0;
+#pragma unroll 2
+    for (uint32_t p = 0; p < np; ++p)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) x[c] += w[(size_t)p * (SH::PAIRS * 256) + (r * 8 + c) * 256];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const size_t i = bi * SH::ROWS + wr + SH::row_at(li, r), j = bj * TILE_COLS + wc + SH::col_at(lj, c);
+        if (i < j && j < g.n) write_pair<OP>(g, i, j, x[c]);
+        else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
+    }
+}
+
+// ------------------------------------------------------------------ dense list
+// One workgroup: a thread counts the bits of its run of words, an exclusive sum
+// over the threads gives its first place, then it writes its nodes.
+constexpr uint32_t DL_T = 1024;
+__global__ void __launch_bounds__(DL_T) k_dense_list(uint32_t* __restrict__ dlist, const uint32_t* __restrict__ dmask,
+                                                     uint32_t Kw) {
+    __shared__ uint32_t wsum[DL_T / 64];
+    const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const uint32_t per = (Kw + DL_T - 1) / DL_T;
+    const uint32_t a = min(Kw, t * per), b = min(Kw, a + per);
+    uint32_t c = 0;
+    for (uint32_t q = a; q < b; ++q) c += __popc(dmask[q]);
+    uint32_t incl = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d, 64);
+        if ((int)lane >= d) incl += y;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    for (uint32_t q = 0; q < DL_T / 64; ++q) {
+        before += q < w ? wsum[q] : 0u;
+        total += wsum[q];
+    }
+    if (t == 0) dlist[0] = total;
+    uint32_t* o = dlist + 1 + before + incl - c;
+    for (uint32_t q = a; q < b; ++q)
+        for (uint32_t m = dmask[q]; m; m &= m - 1) *o++ = q * 32 + (uint32_t)(__ffs(m) - 1);
+}
+
+}  // namespace
+
+// ------------------------------------------------------------------ work lists
+
+// Each XCD gets an equal run of tiles.  Whole rounds of `resident` tiles stay
+// whole; the tiles left over, which would leave most of the XCD idle for one
+// more round, are cut into np parts over the nodes, np the cheapest of
+// ceil(left * np / resident) rounds of 1 / np of a tile each plus the cost of
+// writing and reading the parts' sums.
+TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes, uint32_t resident) {
+    TileSet t;
+    const uint32_t nbi = (n + rows - 1) / rows, nbj = (n + TILE_COLS - 1) / TILE_COLS;
+    // 1024 x 1024 samples per super-tile: about the tiles resident on one XCD
+    const uint32_t SI = std::max<uint32_t>(1, 1024 / rows), SJ = 1024 / TILE_COLS;
+    std::vector<uint32_t> order;
+    for (uint32_t si = 0; si < nbi; si += SI)
+        for (uint32_t sj = 0; sj < nbj; sj += SJ)
+            for (uint32_t bi = si; bi < std::min(nbi, si + SI); ++bi)
+                for (uint32_t bj = sj; bj < std::min(nbj, sj + SJ); ++bj)
+                    if ((bj + 1) * TILE_COLS > bi * rows) order.push_back(bi << 16 | bj);   // (with the diagonal)
+    t.tiles = order.size();
+    // a part is at least 64 nodes; writing and reading one costs about as much as 24 nodes' terms
+    const uint32_t most = std::max<uint32_t>(1, std::min<uint32_t>(TILE_MAX_PARTS, max_nodes / 64));
+    const double part_cost = max_nodes ? 24.0 / max_nodes : 1.0;
+    std::vector<std::vector<TileUnit>> xcd(N_XCDS);
+    size_t at = 0;
+    for (uint32_t x = 0; x < N_XCDS; ++x) {
+        const size_t end = order.size() * (x + 1) / N_XCDS, count = end - at;
+        const size_t left = count % resident, whole = count - left;
+        uint32_t np = 1;
+        double best = left ? 1.0 : 0.0;
+        for (uint32_t q = 2; q <= most && left; ++q) {
+            const double cost = (double)((left * q + resident - 1) / resident) * (1.0 / q + part_cost);
+            if (cost < 0.97 * best) { best = cost; np = q; }
+        }
+        for (size_t k = 0; k < count; ++k) {
+            const uint32_t bij = order[at + k];
+            if (k < whole || np == 1) { xcd[x].push_back({bij, 0u}); continue; }
+            t.split.push_back({bij, t.slots << 12 | (np - 1)});
+            for (uint32_t p = 0; p < np; ++p) xcd[x].push_back({bij, (t.slots + p) << 12 | p << 6 | (np - 1)});
+            t.slots += np;
+        }
+        at = end;
+        t.per_xcd = std::max<uint32_t>(t.per_xcd, (uint32_t)xcd[x].size());
+    }
+    for (auto& v : xcd) {
+        v.resize(t.per_xcd, TileUnit{TILE_NONE, 0u});
+        t.units.insert(t.units.end(), v.begin(), v.end());
+    }
+    return t;
+}
+
+TileSet tile_subset(const TileSet& full, const std::function<bool(uint32_t, uint32_t)>& keep) {
+    TileSet t;
+    auto in = [&](const TileUnit& u) { return u.bij != TILE_NONE && keep(u.bij >> 16, u.bij & 0xffffu); };
+    for (const TileUnit& u : full.units)
+        if (in(u)) {
+            t.units.push_back(u);
+            t.tiles += ((u.part >> 6) & 63u) == 0;
+        }
+    for (const TileUnit& u : full.split)
+        if (in(u)) t.split.push_back(u);
+    t.per_xcd = (uint32_t)((t.units.size() + N_XCDS - 1) / N_XCDS);
+    t.slots = full.slots;
+    return t;
+}
+
+// ------------------------------------------------------------------ launchers
+
+hipError_t launch_dense_list(uint32_t* dlist, const uint32_t* dmask, uint32_t K, hipStream_t st) {
+    if (!dlist || (K && !dmask)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_dense_list, dim3(1), dim3(DL_T), 0, st, dlist, dmask, (K + 31) / 32);
+    return hipGetLastError();
+}
+
+template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_t st) {
+    constexpr uint32_t rows = Shape<OP>::ROWS;
+    if (!a.n || !a.n_units) return hipSuccess;   // (a selection without a tile here)
+    if (!a.U || !a.dlist || !a.out || !a.units || (a.normalized && !a.S) || a.ldn % TILE_COLS || a.ldn < a.n ||
+        a.ldn % rows || (a.n + rows - 1) / rows > 65535 || (a.n_split && (!a.split || !a.ws)) || (OP::LEN && !a.len))
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_tiles<OP>, dim3(a.per_xcd * N_XCDS), dim3(256), 0, st, a);
+    if (a.n_split) hipLaunchKernelGGL(k_tiles_finish<OP>, dim3(a.n_split, OP::RL), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_tiles_w32(const TileArgs& a, hipStream_t st) { return launch_tiles<OpW32>(a, st); }
+
+}  // namespace ssu

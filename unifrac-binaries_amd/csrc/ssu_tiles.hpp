@@ -1,0 +1,72 @@
+// Pair tiles over the dense nodes of the shared-node path: the work list
+// (tiles of the upper triangle, some of them cut into parts over the nodes)
+// and the launchers.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <functional>
+#include <vector>
+
+namespace ssu {
+
+constexpr uint32_t TILE_COLS = 128;     // columns of every tile; its rows depend on the kernel
+constexpr uint32_t TILE_MAX_PARTS = 64;
+
+// One workgroup's work: part p of np of the tile of rows bi * rows .., columns
+// bj * TILE_COLS ..  Parts of one tile hold consecutive workspace slots.
+struct TileUnit {
+    uint32_t bij;    // bi << 16 | bj; TILE_NONE: nothing
+    uint32_t part;   // slot << 12 | p << 6 | (np - 1)
+};
+constexpr uint32_t TILE_NONE = 0xffffffffu;
+
+// The tiles of an n x n upper triangle in launch order.  Workgroups go to the 8
+// XCDs round robin; unit q of XCD x is units[x * per_xcd + q], so that each XCD
+// walks a run of neighbouring tiles and shares their operand rows in its L2.
+struct TileSet {
+    std::vector<TileUnit> units;
+    std::vector<TileUnit> split;   // the tiles cut into parts: bij, first slot << 12 | (np - 1)
+    uint32_t per_xcd = 0;
+    uint32_t slots = 0;            // workspace slots used (parts of cut tiles)
+    uint64_t tiles = 0;
+};
+// rows: tile rows (a divisor or multiple of TILE_COLS); max_nodes: an upper
+// bound on the dense nodes; resident: workgroups one XCD holds at a time.
+TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes, uint32_t resident);
+// those of `full` that keep(bi, bj) selects, cut as in `full` (so that a tile's
+// sums do not depend on the selection)
+TileSet tile_subset(const TileSet& full, const std::function<bool(uint32_t, uint32_t)>& keep);
+
+struct TileArgs {
+    const void* U;            // operand rows
+    const int32_t* rows;      // FP64: operand row of processed node r (nullptr: r itself)
+    size_t ldn;               // their stride, a multiple of TILE_COLS
+    const double* len;        // [K] lengths (FP64 operands)
+    const uint32_t* dlist;    // dlist[0] = dense nodes, then their processed-node indices
+    uint32_t n;
+    const double* S;          // per-sample sums
+    bool normalized;
+    void* out;                // n x n, the operand's type
+    bool add_partial;         // out[i * n + j], i < j, holds the rare nodes' share
+    double* ws;               // workspace slots of rows * TILE_COLS doubles
+    const TileUnit* units;
+    uint32_t n_units, per_xcd;
+    const TileUnit* split;
+    uint32_t n_split;
+};
+constexpr uint32_t TILE_ROWS_W = 128;      // rows per tile of the weighted kernels
+constexpr size_t TILE_SLOT_W = size_t(TILE_ROWS_W) * TILE_COLS * sizeof(double);   // bytes of one workspace slot
+constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD (32 CUs) holds at 2 waves per SIMD
+
+// FP32 weighted: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
+// share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (U's rows are scaled)
+hipError_t launch_tiles_w32(const TileArgs& a, hipStream_t st);
+
+// dlist from the dense mask ([ceil(K / 32)] words): dlist[0] = their number,
+// then the set bits in increasing order
+hipError_t launch_dense_list(uint32_t* dlist, const uint32_t* dmask, uint32_t K, hipStream_t st);
+
+}  // namespace ssu

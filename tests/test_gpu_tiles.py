@@ -11,7 +11,8 @@ from conftest import rel_err
 pytestmark = pytest.mark.gpu
 
 TOL = {"fp32": 1e-6, "fp64": 1e-11}
-OPS = [("weighted_normalized", {}), ("weighted_unnormalized", {})]
+OPS = [("weighted_normalized", {}), ("weighted_unnormalized", {}), ("weighted_normalized_fp64", {}),
+       ("weighted_unnormalized_fp64", {})]
 
 
 @pytest.fixture(scope="module", autouse=True)

@@ -477,7 +477,7 @@ struct PlanImpl {
     bool bits = false;
     uint32_t ldb = 0;
     std::vector<uint32_t> block_order;  // pair blocks / Gram tiles in launch order
-    // pair tiles over the dense nodes (FP32 weighted): the work list of the full
+    // pair tiles over the dense nodes (weighted): the work list of the full
     // matrix, a stripe selection's, and the output bands'
     bool tiled = false;
     uint32_t n_dense_max = 0;        // the most dense nodes an execution can have
@@ -486,9 +486,6 @@ struct PlanImpl {
     std::vector<TileBand> tile_bands;
     std::vector<uint32_t> udense;    // bit q: not in urare (the dense nodes of blocked embeddings)
     bool upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std::string* err);
-    // shared-node pair blocks of 32 x 64 samples (FP32 operands, and generalized on
-    // either), else 64 x 64 (FP64 weighted)
-    bool rect() const { return sparse && (!spec.fp64 || gen); }
     // stripe selection (set_stripes): the pairs computed, and the blocks / tiles
     // holding one (run_order, on the device in d_order_run; empty: block_order)
     GapBand band;
@@ -1245,11 +1242,10 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
         for (size_t q = 0; q < ls.size(); ++q) ls[q] = spec.fp64 ? P.klen_d[q] : (double)P.klen_f[q];
         ok = upload(P.d_klen_sum, ls, P.st, err);
     }
-    // 16 x 16 super-tiles of 64-sample blocks, 6 x 6 of 128-sample Gram tiles:
-    // about the number of blocks (tiles) resident on one XCD
-    P.tiled = P.sparse && !P.gen && !spec.fp64;
+    // 6 x 6 super-tiles of 128-sample Gram tiles: about the number of tiles resident on one XCD
+    P.tiled = P.sparse && !P.gen;
     if (ok && P.sparse && !P.tiled) {
-        P.block_order = P.rect() ? rect_block_order(P.n) : upper_block_order((P.n + 63) / 64, 16);
+        P.block_order = rect_block_order(P.n);
         ok = upload(P.d_order, P.block_order, P.st, err);
     }
     if (ok && P.gram) {
@@ -1414,7 +1410,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                        split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
                                        split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled));
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled && gather));
             if (gather && s.vaw)
                 SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
                                            (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st));
@@ -1459,7 +1455,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.band = P.band;
         if (P.tiled) {
             b.dlist = P.d_dlist.as<uint32_t>();
-            if (!skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
+            if (gather && !skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
         }
         if (vsplit) {
             const bool unw = s.method == Method::unweighted || s.method == Method::unweighted_unnormalized;
@@ -1554,7 +1550,9 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         SSU_HIP(P.mark(4));
     } else if (P.tiled) {
         TileArgs a{};
-        a.U = P.d_U.p;
+        a.U = s.fp64 ? P.d_E.p : P.d_U.p;
+        a.rows = s.fp64 ? P.d_knodes.as<int32_t>() : nullptr;
+        a.len = P.d_klen_sum.as<double>();
         a.ldn = P.ldn;
         a.dlist = P.d_dlist.as<uint32_t>();
         a.n = P.n;
@@ -1586,7 +1584,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                 a.split = (P.band_all ? P.d_split : P.d_split_run).as<TileUnit>();
                 a.n_split = (uint32_t)t.split.size();
             }
-            SSU_HIP(launch_tiles_w32(a, bs));
+            SSU_HIP(launch_tiles_weighted(s.fp64, a, bs));
             if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
         }
         if (P.banded_run && nbands > 1)   // the later work on st reads every band
@@ -1624,9 +1622,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                 a.n_blocks = P.band_off[k + 1] - P.band_off[k];
                 if (k & 1) bs = P.band_st2;
             }
-            if (P.gen && s.fp64) SSU_HIP(launch_pairs_gen64(a, s.alpha, split ? P.d_out2.p : nullptr, bs));
-            else if (P.gen) SSU_HIP(launch_pairs_gen32(a, (float)s.alpha, split ? P.d_out2.p : nullptr, bs));
-            else SSU_HIP(launch_pairs_sparse(true, a, bs));
+            if (s.fp64) SSU_HIP(launch_pairs_gen64(a, s.alpha, split ? P.d_out2.p : nullptr, bs));
+            else SSU_HIP(launch_pairs_gen32(a, (float)s.alpha, split ? P.d_out2.p : nullptr, bs));
             if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
         }
         if (P.banded_run && nbands > 1)   // the later work on st reads every band
@@ -1738,7 +1735,7 @@ bool Plan::refines() const { return p_->refine_on; }
 // samples; Gram: 128-sample tile rows, band 0 holding every diagonal tile).
 bool PlanImpl::prepare_bands(std::string* err) {
     if (!band_ev.empty()) return true;
-    const uint32_t ei = gram ? GRAM_BM : tiled ? TILE_ROWS_W : (rect() ? 32 : 64);
+    const uint32_t ei = gram ? GRAM_BM : tiled ? TILE_ROWS_W : 32;   // (generalized: 32 x 64 pair blocks)
     const uint32_t nbi = (n + ei - 1) / ei;
     // the Gram path's bands are cheaper to compute than to copy: more, smaller ones
     // (16 bands measured 27.0 ms against 28.1 ms for 10 at 16,384 samples; the
@@ -1876,7 +1873,6 @@ bool Plan::set_stripes(uint32_t start, uint32_t stop, std::string* err) {
     }
     uint32_t ei = 0, ej = 0;   // block edges (rows, columns)
     if (P.gram) ei = ej = GRAM_BM;
-    else if (P.sparse && !P.rect()) ei = ej = 64;
     else if (P.sparse) { ei = 32; ej = 64; }
     for (uint32_t bij : P.block_order) {
         const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
@@ -2039,14 +2035,14 @@ uint64_t Plan::kernel_terms() const {
     }
     if (P.sparse) {
         // visited nodes per block, times the pairs a block evaluates
-        const size_t nbi = P.rect() ? (P.n + 31) / 32 : (P.n + 63) / 64, nbj = (P.n + 63) / 64;
+        const size_t nbi = (P.n + 31) / 32, nbj = (P.n + 63) / 64;
         if (!nbj || !P.d_visits.p) return 0;
         std::vector<uint32_t> v(nbi * nbj);
         if (hipMemcpy(v.data(), P.d_visits.p, v.size() * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
             return 0;
         uint64_t sum = 0;
         for (uint32_t bij : P.order_used()) sum += v[(size_t)(bij >> 16) * nbj + (bij & 0xffffu)];
-        return sum * (P.rect() ? 32 * 64 : 64 * 64);
+        return sum * (32 * 64);
     }
     // dense tiles: 128 x 128 for weighted / plain unweighted, 64 x 64 for generalized and VAW
     const bool small = P.spec.vaw || P.spec.method == Method::generalized;

@@ -1153,23 +1153,10 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
         }
 }
 
-// ------------------------------------------------------ sparse weighted path
+// ------------------------------------------------------ generalized pair blocks
 //
-// Weighted UniFrac through the minimum:  |u - v| = u + v - 2 min(u, v), so
-//   sum_k l_k |u_ik - u_jk| = S_i + S_j - 2 M_ij,   M_ij = sum_k l_k min(u_ik, u_jk),
-// with S the per-sample sums.  min(u, v) is zero unless both samples hold the
-// node, so a 64x64 block of pairs only visits the nodes present in both of its
-// sample panels: the AND of the two panels' node masks.  One wavefront owns one
-// block; each lane keeps an 8x8 register tile of FP64 accumulators (v_min_f64
-// and v_fma_f64 issue at the same rate as their FP32 forms on this GPU).
-
-// v_min_f64 without the NaN-quieting canonicalisation the compiler adds for
-// operands it cannot see produced (here: LDS loads of staged values)
-__device__ __forceinline__ double vmin_f64(double a, double b) {
-    double r;
-    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
+// 32 x 64 blocks of pairs that only visit the nodes present in one of their
+// sample panels: the OR of the panels' node masks.
 
 // Compacts the set bits of the wave's 64 mask words (lane l holds word l) into
 // list[], in increasing order of l * 32 + bit; returns their number (uniform).
@@ -1192,145 +1179,11 @@ __device__ __forceinline__ uint32_t build_list(uint16_t* list, uint32_t word, ui
     return total;
 }
 
-constexpr uint32_t SP_B = 64;        // block edge in samples
 constexpr uint32_t SP_WORDS = 64;    // mask words (32 nodes each) per list chunk
-// Staging: the 8 values a lane reads for its rows (or columns) are contiguous;
-// groups of 8 sit SP_GS doubles (80 bytes) apart so that the 8 distinct
-// 16-byte reads of one ds_read_b128 pass fall in different LDS banks.
-constexpr uint32_t SP_GS = 10;
-constexpr uint32_t SP_HALF = 8 * SP_GS;   // offset of the column panel in a staged node
-// nodes per step; two steps are in flight in registers while one is consumed
-template <class TIn> struct SpStep { static constexpr uint32_t EB = sizeof(TIn) == 4 ? 8 : 4; };
 
 // Blocks are numbered so that each XCD (workgroups go to the XCDs round robin)
-// walks a contiguous run of `order` (upper_block_order): the blocks resident
+// walks a contiguous run of `order` (rect_block_order): the blocks resident
 // on one XCD then share their sample panels in that XCD's L2.
-
-template <class TIn, class TOut>
-__global__ void __launch_bounds__(64) k_pairs_sparse(const TIn* __restrict__ U, const int32_t* __restrict__ rows,
-                                                     size_t ldn, const double* __restrict__ len,
-                                                     const uint32_t* __restrict__ masks, uint32_t Kw, uint32_t n,
-                                                     const double* __restrict__ S, int normalized,
-                                                     TOut* __restrict__ out, uint32_t* __restrict__ visits,
-                                                     const uint32_t* __restrict__ order, uint32_t n_blocks,
-                                                     uint32_t per_xcd, const uint32_t* __restrict__ dmask,
-                                                     int add_partial) {
-    constexpr uint32_t EB = SpStep<TIn>::EB;
-    const uint32_t seq = (blockIdx.x % N_XCDS) * per_xcd + blockIdx.x / N_XCDS;
-    if (seq >= n_blocks) return;
-    const uint32_t bij = order[seq];
-    const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
-    uint32_t visited = 0;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t li = lane >> 3, lj = lane & 7;
-
-    __shared__ uint16_t list[SP_WORDS * 32];
-    __shared__ __attribute__((aligned(16))) double sv[EB][2 * SP_HALF];
-    __shared__ double sl[EB];
-
-    double acc[8][8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[r][c] = 0.0;
-
-    const uint32_t* mI = masks + (size_t)(2 * bi) * Kw;   // two 32-sample panels per side
-    const uint32_t* mJ = masks + (size_t)(2 * bj) * Kw;
-    const size_t offI = (size_t)bi * SP_B + lane, offJ = (size_t)bj * SP_B + lane;
-    const uint32_t slot = (lane >> 3) * SP_GS + (lane & 7);   // where this lane stages its sample
-
-    for (uint32_t w0 = 0; w0 < Kw; w0 += SP_WORDS) {
-        // active nodes of this chunk, in increasing order, as offsets from w0*32
-        const uint32_t w = w0 + lane;
-        uint32_t word = w < Kw ? ((mI[w] | mI[Kw + w]) & (mJ[w] | mJ[Kw + w])) : 0u;
-        if (dmask && w < Kw) word &= dmask[w];   // the other nodes come from the posting-list kernel
-        const uint32_t total = build_list(list, word, lane);
-        visited += total;
-        const uint32_t base = w0 * 32;
-        // lane e < EB resolves node t0 + e; its panel rows land in registers.
-        // The loads are unconditional (row 0 stands in past the list end and
-        // is masked out at staging), so the compiler can wait for one step's
-        // loads while the other step's stay in flight.
-        TIn pA[EB], qA[EB], pB[EB], qB[EB];
-        double lA = 0.0, lB = 0.0;
-        uint64_t vA = 0, vB = 0;   // which of the step's EB nodes are real
-        auto fetch = [&](TIn (&p)[EB], TIn (&q)[EB], double& l, uint64_t& valid, uint32_t t0)
-                         __attribute__((always_inline)) {
-            const uint32_t idx = t0 + lane;
-            const bool real = lane < EB && idx < total;
-            int32_t row = 0;
-            l = 0.0;
-            if (real) {
-                const uint32_t r = base + list[idx];
-                // FP32 operand rows are the processed rows themselves; only FP64
-                // operands read the embedding through rows[]
-                if constexpr (sizeof(TIn) == 8) row = rows[r];
-                else row = (int32_t)r;
-                l = len[r];
-            }
-            valid = __ballot(real);
-#pragma unroll
-            for (uint32_t e = 0; e < EB; ++e) {
-                const size_t off = (size_t)__builtin_amdgcn_readlane(row, e) * ldn;
-                p[e] = U[off + offI];
-                q[e] = U[off + offJ];
-            }
-        };
-        auto step = [&](TIn (&p)[EB], TIn (&q)[EB], double& l, uint64_t& valid, uint32_t t_next)
-                        __attribute__((always_inline)) {
-#pragma unroll
-            for (uint32_t e = 0; e < EB; ++e) {
-                const bool on = (valid >> e) & 1;
-                sv[e][slot] = on ? (double)p[e] : 0.0;
-                sv[e][SP_HALF + slot] = on ? (double)q[e] : 0.0;
-            }
-            if (lane < EB) sl[lane] = l;
-            __syncthreads();
-            if (t_next < total) fetch(p, q, l, valid, t_next);   // two steps ahead of its use
-#pragma unroll 2
-            for (uint32_t e = 0; e < EB; ++e) {
-                double a[8], b[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) a[r] = sv[e][li * SP_GS + r];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) b[c] = sv[e][SP_HALF + lj * SP_GS + c];
-                const double ln = sl[e];
-#pragma unroll
-                for (int r = 0; r < 8; ++r)
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) acc[r][c] = __builtin_fma(vmin_f64(a[r], b[c]), ln, acc[r][c]);
-            }
-            __syncthreads();
-        };
-        if (total) fetch(pA, qA, lA, vA, 0);
-        if (total > EB) fetch(pB, qB, lB, vB, EB);
-        for (uint32_t t0 = 0; t0 < total; t0 += 2 * EB) {
-            step(pA, qA, lA, vA, t0 + 2 * EB);
-            if (t0 + EB >= total) break;
-            step(pB, qB, lB, vB, t0 + 3 * EB);
-        }
-    }
-
-    if (visits && lane == 0) visits[(size_t)bi * ((n + SP_B - 1) / SP_B) + bj] = visited;
-    const size_t i0 = (size_t)bi * SP_B + li * 8, j0 = (size_t)bj * SP_B + lj * 8;
-#pragma unroll
-    for (int r = 0; r < 8; ++r)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const size_t i = i0 + r, j = j0 + c;
-            // the i < j lane writes both entries (so the partial it reads is its own)
-            if (i >= n || j >= n || i > j) continue;
-            if (i == j) { out[i * n + i] = (TOut)0; continue; }
-            double m = acc[r][c];
-            if (add_partial) m += (double)out[i * n + j];   // the sparse nodes' share, from k_pairs_rows
-            const double tot = S[i] + S[j];
-            double x = tot - 2.0 * m;
-            x = x < 0.0 ? 0.0 : x;   // rounding can undershoot 0; NaN (empty samples) passes
-            const double d = normalized ? x / tot : x;
-            out[i * n + j] = (TOut)d;
-            out[j * n + i] = (TOut)d;
-        }
-}
 
 // FP32 operands: 32 x 64 blocks of pairs (rows: a 32-sample panel, columns:
 // a 64-sample panel), one wavefront each, a 4 x 8 tile per lane.  The kernel
@@ -2848,13 +2701,6 @@ hipError_t launch_pairs(PairOp op, bool fp64, const PairArgs& a, hipStream_t st)
     return fp64 ? launch_pairs_prec<double>(op, a, st) : launch_pairs_prec<float>(op, a, st);
 }
 
-template <class TIn, class TOut>
-static void pairs_sparse_t(uint32_t grid, hipStream_t st, const SparseArgs& a, uint32_t per_xcd) {
-    hipLaunchKernelGGL((k_pairs_sparse<TIn, TOut>), dim3(grid), dim3(64), 0, st, (const TIn*)a.U, a.rows, a.ldn, a.len,
-                       a.masks, a.Kw, a.n, a.S, (int)a.normalized, (TOut*)a.out, a.visits, a.order, a.n_blocks,
-                       per_xcd, a.dmask, (int)(a.dmask != nullptr));
-}
-
 std::vector<uint32_t> upper_block_order(uint32_t nb, uint32_t super) {
     std::vector<uint32_t> order;
     order.reserve((size_t)nb * (nb + 1) / 2);
@@ -3105,25 +2951,6 @@ hipError_t launch_pairs_gen64(const SparseArgs& a, double alpha, void* out2, hip
     hipLaunchKernelGGL(k_pairs_gen64, dim3(per_xcd * N_XCDS), dim3(64), 0, st, (const double*)a.U, a.rows, a.ldn,
                        a.len, a.masks, a.Kw, a.n, (double*)a.out, (double*)out2, a.visits, a.order, a.n_blocks,
                        per_xcd, a.dmask, (int)(a.dmask != nullptr), alpha);
-    return hipGetLastError();
-}
-
-hipError_t launch_pairs_sparse(bool in_fp64, const SparseArgs& a, hipStream_t st) {
-    if (a.ldn % SP_B) return hipErrorInvalidValue;
-    const uint32_t nb = (a.n + SP_B - 1) / SP_B;
-    if (!nb) return hipSuccess;
-    if ((size_t)nb * SP_B > a.ldn || nb > 65535 || a.n_blocks > nb * (nb + 1) / 2 || !a.order)
-        return hipErrorInvalidValue;
-    if (!a.n_blocks) return hipSuccess;   // a stripe selection without a block here
-    const uint32_t per_xcd = (a.n_blocks + N_XCDS - 1) / N_XCDS;
-    const uint32_t grid = per_xcd * N_XCDS;
-    if (in_fp64) {
-        if (a.out_fp64) pairs_sparse_t<double, double>(grid, st, a, per_xcd);
-        else pairs_sparse_t<double, float>(grid, st, a, per_xcd);
-    } else {
-        if (a.out_fp64) pairs_sparse_t<float, double>(grid, st, a, per_xcd);
-        else pairs_sparse_t<float, float>(grid, st, a, per_xcd);
-    }
     return hipGetLastError();
 }
 

@@ -201,10 +201,7 @@ struct PairArgs {
 };
 hipError_t launch_pairs(PairOp op, bool fp64, const PairArgs& a, hipStream_t st);
 
-// Weighted (normalized or not).  FP64 (launch_pairs_sparse): d_ij = S_i + S_j -
-// 2 sum_k l_k min(u_ik, u_jk), visiting per 64x64 block only the nodes whose
-// bit is set in both panels' masks.  FP32 (launch_pairs_sparse32): sum_k l_k
-// |u_ik - u_jk| itself over the nodes either panel holds; S normalises.
+// Generalized pair blocks (launch_pairs_gen32 / gen64).
 struct SparseArgs {
     const void* U;          // node rows, float (row r) or double (row rows[r])
     const int32_t* rows;    // nullptr: identity
@@ -313,7 +310,6 @@ size_t row_list_scan_blocks(uint32_t n, uint32_t K);
 // The upper-triangle blocks (bi <= bj < nb) as bi << 16 | bj, super x super
 // super-tile by super-tile; kernels walk it in XCD-contiguous runs.
 std::vector<uint32_t> upper_block_order(uint32_t nb, uint32_t super);
-hipError_t launch_pairs_sparse(bool in_fp64, const SparseArgs& a, hipStream_t st);
 // 32 x 64 blocks (32-sample row panel pi <= 2 pj + 1, 64-sample column panel pj):
 // `order` = rect_block_order(n) and visits is [ceil(n/32)][ceil(n/64)].
 std::vector<uint32_t> rect_block_order(uint32_t n);

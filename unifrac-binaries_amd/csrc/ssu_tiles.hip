@@ -4,9 +4,9 @@
 // block visits it: the kernels are dense contractions with |x_i - x_j| in
 // place of the product, which no matrix instruction forms.  They are laid out
 // like a vector-ALU GEMM: 128 columns per tile, four waves of (rows / 2) x 64
-// pairs, a lane holding groups of four rows and four columns 32 apart, so that
-// its operands are ds_read_b128 of 8 distinct contiguous 16-byte pieces (no
-// bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
+// pairs, a lane holding its rows and columns in groups of 16 bytes, a group
+// apart from the next lane's, so that its operands are ds_read_b128 of 8
+// distinct contiguous pieces (no bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
 // to LDS by global_load_lds, 16 bytes per lane, a stage of nodes ahead.
 #include "ssu_tiles.hpp"
 
@@ -39,7 +39,12 @@ __device__ __forceinline__ void part_range(uint32_t nd, uint32_t eb, uint32_t p,
 //   LEN      the node's length is staged too (otherwise U's rows are scaled by it)
 constexpr uint32_t MERGE = 64;
 
-// FP32 weighted: |l u - l v|, two full-rate instructions
+// FP32 weighted: |l u - l v|, two instructions at the full FP32 rate (register
+// operands only: an SGPR operand halves it, as do min, max and v_sad_u32).
+// Bound by VALU issue: 16,384 samples x 9,790 dense nodes in 44.9 ms, 2.94e13
+// terms/s of the 3.1e13 that sub + add reach in registers at two waves per SIMD;
+// 32 x 64 pairs per wave with lengths in the term, three LDS reads for 32 terms,
+// took 70.4 ms.
 struct OpW32 {
     typedef float V;
     static constexpr int RL = 8, EB = 16;
@@ -55,6 +60,27 @@ struct OpW32 {
     }
 };
 
+// FP64 weighted: M = sum of l min(u, v), of which the distance is S_i + S_j - 2 M
+// (u, v >= 0; v_min_f64 without the NaN quieting the compiler adds for values it
+// does not see produced).  Bound by FP64 issue (half the FP32 rate): 3,001
+// samples x 3,700 dense nodes in 1.62 ms, against 2.66 ms in 64 x 64 blocks of one
+// wave; 131 samples 0.37 -> 0.04 ms, the parts filling the device.
+struct OpW64 {
+    typedef double V;
+    static constexpr int RL = 8, EB = 8;
+    static constexpr bool TWO = false, LEN = true;
+    static __device__ __forceinline__ void term(double u, double v, double l, double& num, double&) {
+        double m;
+        asm("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(u), "v"(v));
+        num = __builtin_fma(m, l, num);
+    }
+    static __device__ __forceinline__ double distance(double m, double share, double tot, bool normalized) {
+        double x = tot - 2.0 * (m + share);
+        x = x < 0.0 ? 0.0 : x;
+        return normalized ? x / tot : x;
+    }
+};
+
 template <class OP> struct Shape {
     typedef typename OP::V V;
     static constexpr uint32_t ROWS = 16 * OP::RL;               // of a tile: two waves of 8 RL
@@ -62,22 +88,20 @@ template <class OP> struct Shape {
     static constexpr uint32_t NODE = ROWS + TILE_COLS;          // staged values of a node
     static constexpr uint32_t PAIRS = OP::RL * 8;               // of a lane
     static constexpr bool MIXED = sizeof(V) == 4;
-    // row of the lane's q-th row in its wave's rows, column of its q-th column in its wave's 64 columns
-    static __device__ __forceinline__ uint32_t row_at(uint32_t li, uint32_t q) { return (q >> 2) * 32 + li * 4 + (q & 3); }
-    static __device__ __forceinline__ uint32_t col_at(uint32_t lj, uint32_t q) { return (q >> 2) * 32 + lj * 4 + (q & 3); }
-};
-
-// four consecutive values of LDS (one 16-byte read, or two)
-template <class V> __device__ __forceinline__ void read4(V (&x)[4], const V* p) {
-    typedef __attribute__((ext_vector_type(16 / sizeof(V)))) V vec;
-    constexpr int N = 16 / sizeof(V);
+    static constexpr uint32_t G = 16 / sizeof(V);               // values of one 16-byte LDS read
+    // the lane's q-th row in its wave's rows (l = li), or column in its wave's 64 columns (l = lj)
+    static __device__ __forceinline__ uint32_t at(uint32_t l, uint32_t q) { return q / G * (8 * G) + l * G + q % G; }
+    // a lane's N values at(l, 0 .. N - 1) of a staged panel
+    template <int N> static __device__ __forceinline__ void read(V (&x)[N], const V* panel, uint32_t l) {
+        typedef __attribute__((ext_vector_type(G))) V vec;
 #pragma unroll
-    for (int h = 0; h < 4 / N; ++h) {
-        const vec v = reinterpret_cast<const vec*>(p)[h];
+        for (int h = 0; h < N / (int)G; ++h) {
+            const vec v = *reinterpret_cast<const vec*>(panel + at(l, h * G));
 #pragma unroll
-        for (int z = 0; z < N; ++z) x[h * N + z] = v[z];
+            for (int z = 0; z < (int)G; ++z) x[h * G + z] = v[z];
+        }
     }
-}
+};
 
 // the distance of pair i < j, written to both triangles
 template <class OP>
@@ -85,7 +109,7 @@ __device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j
     typedef typename OP::V V;
     V* out = (V*)g.out;
     const double share = g.add_partial ? (double)out[i * g.n + j] : 0.0;   // the rare nodes', from the posting walk
-    const double d = OP::distance(x, share, g.normalized ? g.S[i] + g.S[j] : 0.0, g.normalized);
+    const double d = OP::distance(x, share, g.S[i] + g.S[j], g.normalized);
     out[i * g.n + j] = (V)d;
     out[j * g.n + i] = (V)d;
 }
@@ -160,17 +184,15 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         if (k0 + EB < kb) index(k0 + EB);
     };
     auto node = [&](int buf, uint32_t e) __attribute__((always_inline)) {
-        V a[RL / 4][4], b[2][4];
-#pragma unroll
-        for (int h = 0; h < RL / 4; ++h) read4(a[h], &sv[buf][e][wr + 32 * h + li * 4]);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) read4(b[h], &sv[buf][e][SH::ROWS + wc + 32 * h + lj * 4]);
+        V a[RL], b[8];
+        SH::read(a, &sv[buf][e][wr], li);
+        SH::read(b, &sv[buf][e][SH::ROWS + wc], lj);
         const V l = OP::LEN ? sl[buf][e] : V(0);
         V none = V(0);
 #pragma unroll
         for (int r = 0; r < RL; ++r)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) OP::term(a[r >> 2][r & 3], b[c >> 2][c & 3], l, num[r][c], none);
+            for (int c = 0; c < 8; ++c) OP::term(a[r], b[c], l, num[r][c], none);
     };
     auto merge = [&]() __attribute__((always_inline)) {
         if constexpr (SH::MIXED) {
@@ -219,7 +241,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
     for (int r = 0; r < RL; ++r)
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            const size_t i = i0 + wr + SH::row_at(li, r), j = j0 + wc + SH::col_at(lj, c);
+            const size_t i = i0 + wr + SH::at(li, r), j = j0 + wc + SH::at(lj, c);
             double x;
             if constexpr (SH::MIXED) x = num64[r][c];
             else x = num[r][c];
@@ -248,7 +270,7 @@ __global__ void __launch_bounds__(256) k_tiles_finish(TileArgs g) {
         for (int c = 0; c < 8; ++c) x[c] += w[(size_t)p * (SH::PAIRS * 256) + (r * 8 + c) * 256];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const size_t i = bi * SH::ROWS + wr + SH::row_at(li, r), j = bj * TILE_COLS + wc + SH::col_at(lj, c);
+        const size_t i = bi * SH::ROWS + wr + SH::at(li, r), j = bj * TILE_COLS + wc + SH::at(lj, c);
         if (i < j && j < g.n) write_pair<OP>(g, i, j, x[c]);
         else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
     }
@@ -363,7 +385,7 @@ hipError_t launch_dense_list(uint32_t* dlist, const uint32_t* dmask, uint32_t K,
 template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_t st) {
     constexpr uint32_t rows = Shape<OP>::ROWS;
     if (!a.n || !a.n_units) return hipSuccess;   // (a selection without a tile here)
-    if (!a.U || !a.dlist || !a.out || !a.units || (a.normalized && !a.S) || a.ldn % TILE_COLS || a.ldn < a.n ||
+    if (!a.U || !a.dlist || !a.out || !a.units || !a.S || a.ldn % TILE_COLS || a.ldn < a.n ||
         a.ldn % rows || (a.n + rows - 1) / rows > 65535 || (a.n_split && (!a.split || !a.ws)) || (OP::LEN && !a.len))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_tiles<OP>, dim3(a.per_xcd * N_XCDS), dim3(256), 0, st, a);
@@ -371,6 +393,9 @@ template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_tiles_w32(const TileArgs& a, hipStream_t st) { return launch_tiles<OpW32>(a, st); }
+hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st) {
+    if (fp64 && !a.rows) return hipErrorInvalidValue;
+    return fp64 ? launch_tiles<OpW64>(a, st) : launch_tiles<OpW32>(a, st);
+}
 
 }  // namespace ssu

@@ -61,9 +61,11 @@ constexpr uint32_t TILE_ROWS_W = 128;      // rows per tile of the weighted kern
 constexpr size_t TILE_SLOT_W = size_t(TILE_ROWS_W) * TILE_COLS * sizeof(double);   // bytes of one workspace slot
 constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD (32 CUs) holds at 2 waves per SIMD
 
-// FP32 weighted: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
-// share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (U's rows are scaled)
-hipError_t launch_tiles_w32(const TileArgs& a, hipStream_t st);
+// Weighted.  FP32: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
+// share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (U's rows are scaled).
+// FP64: x = S_i + S_j - 2 M in its place, M = sum of l min(u_i, u_j) + the rare
+// share, U the embedding (row rows[r] for processed node r).
+hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st);
 
 // dlist from the dense mask ([ceil(K / 32)] words): dlist[0] = their number,
 // then the set bits in increasing order

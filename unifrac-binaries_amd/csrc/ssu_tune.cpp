@@ -11,7 +11,7 @@ namespace {
 // three thresholds each on the 16,384-sample (100k tips) and 8,192-sample
 // (50k tips) workloads (total = fixed + terms * term + postings * posting); the
 // modelled optimum lands within the measured one for every kind (weighted
-// 0.193 vs 0.2, FP64 weighted 0.229 vs 0.25, generalized 0.738 vs 0.8,
+// 0.193 vs 0.2, FP64 weighted 0.24 vs 0.23 - 0.3, generalized 0.738 vs 0.8,
 // Gram 0.075 vs 0.06 - 0.1).  The per-term cost includes the list building
 // and row lists, whose work follows the postings.
 struct Rates {
@@ -25,7 +25,9 @@ Rates rates_of(SplitKind k) {
     // 16,384 samples, theta 0.14 .. 0.26: tiles 70.1 .. 42.6 ms, posting phase 29.1 .. 56.5 ms,
     // device total 115.1, 111.6 (0.17), 111.2 (0.2), 112.5 (0.23), 115.0 ms
     case SplitKind::weighted32: return {3.3e-14, 8.9e-13};
-    case SplitKind::weighted64: return {7.1e-14, 1.36e-12};
+    // 3,001 samples (20k tips), theta 0.1 / 0.23 / 0.4: tiles 2.91 / 1.62 / 1.01 ms, posting
+    // phase 0.54 / 1.09 / 1.96 ms, device total 4.20 / 3.46 / 3.73 ms (0.3: 3.50)
+    case SplitKind::weighted64: return {8.2e-14, 1.42e-12};
     case SplitKind::generalized32: return {6.0e-13, 1.1e-12};
     case SplitKind::gram: return {3.4e-15, 6.1e-13};
     // FP64 generalized (an FP64 power and division per tile term, two powers per
@@ -45,10 +47,11 @@ Rates rates_of(SplitKind k) {
 // expected tiled-kernel terms of a node held by c of n samples, placed at
 // random: the pair blocks visit a node either of their sample panels holds
 // (the kernels' counts agree within 1% on the workloads above); a Gram
-// column, a VAW node and a node of the FP32 weighted tiles cost every pair
+// column, a VAW node and a node of the weighted tiles cost every pair
 double tile_terms(SplitKind k, uint32_t n, uint32_t c) {
     const double pairs = 0.5 * (double)n * n;
-    if (k == SplitKind::gram || k == SplitKind::vaw32 || k == SplitKind::vaw64 || k == SplitKind::weighted32)
+    if (k == SplitKind::gram || k == SplitKind::vaw32 || k == SplitKind::vaw64 || k == SplitKind::weighted32 ||
+        k == SplitKind::weighted64)
         return pairs;
     const double q = 1.0 - (double)c / n;   // a given sample lacks the node
     const double q2 = q * q, q4 = q2 * q2, q8 = q4 * q4, q16 = q8 * q8, q32 = q16 * q16;

@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 TOL = {"fp32": 1e-6, "fp64": 1e-11}
 OPS = [("weighted_normalized", {}), ("weighted_unnormalized", {}), ("weighted_normalized_fp64", {}),
-       ("weighted_unnormalized_fp64", {})]
+       ("weighted_unnormalized_fp64", {}), ("generalized", {"alpha": 0.5}), ("generalized", {"alpha": 1.0}),
+       ("generalized", {"alpha": 0.3}), ("generalized", {"alpha": 0.0}), ("generalized_fp64", {"alpha": 0.5}),
+       ("generalized_fp64", {"alpha": 1.0}), ("generalized_fp64", {"alpha": 0.3})]
 
 
 @pytest.fixture(scope="module", autouse=True)

@@ -477,9 +477,10 @@ struct PlanImpl {
     bool bits = false;
     uint32_t ldb = 0;
     std::vector<uint32_t> block_order;  // pair blocks / Gram tiles in launch order
-    // pair tiles over the dense nodes (weighted): the work list of the full
+    // pair tiles over the dense nodes (weighted, generalized): the work list of the full
     // matrix, a stripe selection's, and the output bands'
     bool tiled = false;
+    uint32_t tile_rows() const { return gen ? TILE_ROWS_2 : TILE_ROWS_W; }
     uint32_t n_dense_max = 0;        // the most dense nodes an execution can have
     TileSet tset, tset_run;
     struct TileBand { uint32_t unit0, n_units, per_xcd, split0, n_split; };
@@ -548,9 +549,9 @@ struct PlanImpl {
                 d_heavy.as<int32_t>(), d_child_ptr.as<int32_t>(), d_child_idx.as<int32_t>()};
     }
     void build_paths(const PostorderNodes& nodes);
-    DevMem d_knodes, d_klen, d_klen_sum, d_len_all, d_E, d_C, d_U, d_Cu, d_S, d_Spart, d_masks, d_visits, d_order, d_Pt, d_digits, d_chunks, d_G, d_col, d_out,
+    DevMem d_knodes, d_klen, d_klen_sum, d_len_all, d_E, d_C, d_U, d_Cu, d_S, d_Spart, d_order, d_Pt, d_digits, d_chunks, d_G, d_col, d_out,
         d_faith, d_stripes, d_smask, d_dmask, d_pc, d_pidx, d_pval, d_walked, d_rows, d_rcount, d_roff, d_rbsum,
-        d_sp_node, d_sp_len, d_umasks, d_B, d_poff, d_pcnt, d_obsum, d_Ssp, d_out2, d_pspmax, d_urare, d_close,
+        d_sp_node, d_sp_len, d_B, d_poff, d_pcnt, d_obsum, d_Ssp, d_out2, d_pspmax, d_urare, d_close,
         d_ridx, d_dlist, d_units, d_split, d_units_run, d_split_run, d_units_band, d_split_band, d_tws, d_udense,
         d_order_run, d_order_band, d_vdense, d_vrows, d_vlen, d_tau, d_kidx, d_H, d_pcv, d_nbound;
 
@@ -785,7 +786,7 @@ bool PlanImpl::split_weighted(std::string* err) {
     // tiles, which moves the balance)
     const SplitKind kind = gen ? (spec.fp64 ? SplitKind::generalized64 : SplitKind::generalized32)
                                : spec.fp64 ? SplitKind::weighted64 : SplitKind::weighted32;
-    uint32_t thr = env_theta ? (uint32_t)std::max(1.0, std::ceil(theta * n)) : choose_split(kind, n, cnt, 1ull << 30).thr;
+    uint32_t thr = env_theta ? (uint32_t)std::max(1.0, std::ceil(theta * n)) : choose_split(kind, n, cnt, 1ull << 30, 0, spec.alpha).thr;
     if (thr == 0) return true;
     auto bound = [&](uint32_t t) {
         uint64_t b = 0;
@@ -1243,11 +1244,7 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
         ok = upload(P.d_klen_sum, ls, P.st, err);
     }
     // 6 x 6 super-tiles of 128-sample Gram tiles: about the number of tiles resident on one XCD
-    P.tiled = P.sparse && !P.gen;
-    if (ok && P.sparse && !P.tiled) {
-        P.block_order = rect_block_order(P.n);
-        ok = upload(P.d_order, P.block_order, P.st, err);
-    }
+    P.tiled = P.sparse;
     if (ok && P.gram) {
         P.block_order = upper_block_order((uint32_t)(P.n_pad / GRAM_BM), 6);
         ok = upload(P.d_order, P.block_order, P.st, err);
@@ -1264,7 +1261,7 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
             for (uint32_t q = 0; q < K; ++q) all[q + 1] = q;
             ok = upload(P.d_dlist, all, P.st, err) && hipStreamSynchronize(P.st) == hipSuccess;
         }
-        P.tset = tile_set(P.n, TILE_ROWS_W, P.n_dense_max, TILE_RESIDENT);
+        P.tset = tile_set(P.n, P.tile_rows(), P.n_dense_max, TILE_RESIDENT);
         ok = ok && P.upload_tiles(P.tset, P.d_units, P.d_split, err);
     }
     if (ok && P.vsplit) ok = P.split_vaw(err);
@@ -1320,7 +1317,6 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         if (!P.d_Spart.ensure(parts * sizeof(double), err)) return false;
     }
     const bool shared = P.sparse || P.vsplit;   // sample masks and (with a split) posting lists
-    if (shared && !P.d_masks.ensure(std::max<size_t>((P.ldn / 32) * Kw, 1) * sizeof(uint32_t), err)) return false;
     const bool split = shared && P.split_thr > 0 && K > 0;
     const bool vsplit = P.vsplit && split;
     // VAW one-sided sums: at the plan's distinct totals, or at every sample's when the
@@ -1355,9 +1351,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
     const uint32_t Ks = (uint32_t)P.sp_node.size();
     const bool gsplit = P.gram && P.gsplit_slots > 0 && Ks > 0;
     if (gsplit) {
-        const size_t ks = Ks, kws = (ks + 31) / 32, panels = P.ldn / 32;
-        if (!P.d_umasks.ensure(panels * kws * sizeof(uint32_t), err) ||
-            !P.d_smask.ensure(panels * ks * sizeof(uint32_t), err) ||
+        const size_t ks = Ks, panels = P.ldn / 32;
+        if (!P.d_smask.ensure(panels * ks * sizeof(uint32_t), err) ||
             !P.d_pc.ensure((size_t)(npan + 1) * ks * sizeof(uint32_t), err) ||
             !P.d_pidx.ensure((size_t)P.gsplit_slots * sizeof(uint32_t), err) ||
             !P.d_walked.ensure((size_t)sparse_rows_blocks(P.n) * sizeof(uint32_t), err) ||
@@ -1386,7 +1381,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                       P.d_sp_node.as<int32_t>(), Ks, npan, P.st));
     }
     if (P.tiled && ((split && !P.d_dlist.ensure(((size_t)K + 1) * sizeof(uint32_t), err)) ||
-                    !P.d_tws.ensure(std::max<size_t>(P.tset.slots * TILE_SLOT_W, 1), err)))
+                    !P.d_tws.ensure(std::max<size_t>(P.tset.slots * TILE_SLOT, 1), err)))
         return false;
     // one embedding block (E holds every sample): the postings of the FP32 split take their
     // values from E, and the gather skips the operand rows of nodes that are never dense
@@ -1401,18 +1396,17 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                 SSU_HIP(launch_presence_T(P.d_Pt.as<int8_t>(), P.Kp, P.d_E.as<double>(), w, (uint32_t)c0,
                                           P.d_col.as<int32_t>(), (uint32_t)P.Kp, P.n, P.st));
             if (gsplit)
-                SSU_HIP(launch_gather_sums(nullptr, 0, nullptr, nullptr, P.d_umasks.as<uint32_t>(),
+                SSU_HIP(launch_gather_sums(nullptr, 0, nullptr, nullptr,
                                            P.d_smask.as<uint32_t>(), P.d_E.as<double>(), w, (uint32_t)c0,
                                            P.d_sp_node.as<int32_t>(), nullptr, Ks, P.n, P.st));
-        } else if (gather || sums || shared) {
+        } else if (gather || sums || split) {
             SSU_HIP(launch_gather_sums(gather ? P.d_U.as<float>() : nullptr, P.ldn, sums ? P.S_ptr() : nullptr,
-                                       P.d_Spart.as<double>(), shared ? P.d_masks.as<uint32_t>() : nullptr,
-                                       split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
+                                       P.d_Spart.as<double>(), split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
                                        split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled && gather));
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled && gather && !P.gen));
             if (gather && s.vaw)
-                SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
+                SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
                                            (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st));
         }
     }
@@ -1455,7 +1449,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.band = P.band;
         if (P.tiled) {
             b.dlist = P.d_dlist.as<uint32_t>();
-            if (gather && !skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
+            if (gather && !P.gen && !skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
         }
         if (vsplit) {
             const bool unw = s.method == Method::unweighted || s.method == Method::unweighted_unnormalized;
@@ -1560,6 +1554,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         a.normalized = s.method == Method::weighted_normalized;
         a.out = P.out_ptr();
         a.add_partial = split;
+        a.out2 = P.d_out2.p;
+        a.alpha = s.alpha;
         a.ws = P.d_tws.as<double>();
         const uint32_t nbands = P.banded_run ? (uint32_t)P.band_ev.size() : 1;
         if (P.banded_run && nbands > 1) {
@@ -1584,46 +1580,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                 a.split = (P.band_all ? P.d_split : P.d_split_run).as<TileUnit>();
                 a.n_split = (uint32_t)t.split.size();
             }
-            SSU_HIP(launch_tiles_weighted(s.fp64, a, bs));
-            if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
-        }
-        if (P.banded_run && nbands > 1)   // the later work on st reads every band
-            SSU_HIP(hipStreamWaitEvent(P.st, P.band_ev[(nbands - 2) | 1], 0));   // the last band on band_st2
-        SSU_HIP(P.mark(3));
-        SSU_HIP(P.mark(4));
-    } else if (P.sparse) {
-        SparseArgs a{};
-        a.U = s.fp64 ? P.d_E.p : P.d_U.p;
-        a.rows = s.fp64 ? P.d_knodes.as<int32_t>() : nullptr;
-        a.ldn = P.ldn;
-        a.len = P.d_klen_sum.as<double>();
-        a.masks = P.d_masks.as<uint32_t>();
-        a.Kw = Kw;
-        a.n = P.n;
-        a.S = P.S_ptr();
-        a.normalized = s.method == Method::weighted_normalized;
-        a.out = P.out_ptr();
-        a.out_fp64 = s.fp64;
-        const size_t nb = (P.n + 63) / 64;
-        if (!P.d_visits.ensure(std::max<size_t>(2 * nb * nb, 1) * sizeof(uint32_t), err)) return false;
-        a.visits = P.d_visits.as<uint32_t>();
-        a.order = P.band_all ? P.d_order.as<uint32_t>() : P.d_order_run.as<uint32_t>();
-        a.n_blocks = (uint32_t)P.order_used().size();
-        if (split) a.dmask = P.d_dmask.as<uint32_t>();   // dense nodes only; adds the posting-list share
-        const uint32_t nbands = P.banded_run ? (uint32_t)P.band_ev.size() : 1;
-        if (P.banded_run && nbands > 1) {
-            SSU_HIP(hipEventRecord(P.band_go, P.st));
-            SSU_HIP(hipStreamWaitEvent(P.band_st2, P.band_go, 0));
-        }
-        for (uint32_t k = 0; k < nbands; ++k) {
-            hipStream_t bs = P.st;
-            if (P.banded_run) {
-                a.order = P.d_order_band.as<uint32_t>() + P.band_off[k];
-                a.n_blocks = P.band_off[k + 1] - P.band_off[k];
-                if (k & 1) bs = P.band_st2;
-            }
-            if (s.fp64) SSU_HIP(launch_pairs_gen64(a, s.alpha, split ? P.d_out2.p : nullptr, bs));
-            else SSU_HIP(launch_pairs_gen32(a, (float)s.alpha, split ? P.d_out2.p : nullptr, bs));
+            SSU_HIP(P.gen ? launch_tiles_generalized(s.fp64, a, bs) : launch_tiles_weighted(s.fp64, a, bs));
             if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
         }
         if (P.banded_run && nbands > 1)   // the later work on st reads every band
@@ -1735,7 +1692,7 @@ bool Plan::refines() const { return p_->refine_on; }
 // samples; Gram: 128-sample tile rows, band 0 holding every diagonal tile).
 bool PlanImpl::prepare_bands(std::string* err) {
     if (!band_ev.empty()) return true;
-    const uint32_t ei = gram ? GRAM_BM : tiled ? TILE_ROWS_W : 32;   // (generalized: 32 x 64 pair blocks)
+    const uint32_t ei = gram ? GRAM_BM : tile_rows();
     const uint32_t nbi = (n + ei - 1) / ei;
     // the Gram path's bands are cheaper to compute than to copy: more, smaller ones
     // (16 bands measured 27.0 ms against 28.1 ms for 10 at 16,384 samples; the
@@ -1866,14 +1823,14 @@ bool Plan::set_stripes(uint32_t start, uint32_t stop, std::string* err) {
     P.run_order.clear();
     if (P.tiled) {
         P.tset_run = tile_subset(P.tset, [&](uint32_t bi, uint32_t bj) {
-            return P.band.meets_tile(bi * TILE_ROWS_W, std::min(P.n, (bi + 1) * TILE_ROWS_W), bj * TILE_COLS,
+            const uint32_t tr = P.tile_rows();
+            return P.band.meets_tile(bi * tr, std::min(P.n, (bi + 1) * tr), bj * TILE_COLS,
                                      std::min(P.n, (bj + 1) * TILE_COLS));
         });
         return P.upload_tiles(P.tset_run, P.d_units_run, P.d_split_run, err);
     }
     uint32_t ei = 0, ej = 0;   // block edges (rows, columns)
     if (P.gram) ei = ej = GRAM_BM;
-    else if (P.sparse) { ei = 32; ej = 64; }
     for (uint32_t bij : P.block_order) {
         const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
         const bool diag_tile = P.gram && bi == bj;   // diag(G) feeds every pair of the combine
@@ -2031,18 +1988,7 @@ uint64_t Plan::kernel_terms() const {
     if (P.tiled) {
         uint32_t nd = 0;
         if (!P.d_dlist.p || hipMemcpy(&nd, P.d_dlist.p, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess) return 0;
-        return (P.band_all ? P.tset : P.tset_run).tiles * TILE_ROWS_W * TILE_COLS * nd;
-    }
-    if (P.sparse) {
-        // visited nodes per block, times the pairs a block evaluates
-        const size_t nbi = (P.n + 31) / 32, nbj = (P.n + 63) / 64;
-        if (!nbj || !P.d_visits.p) return 0;
-        std::vector<uint32_t> v(nbi * nbj);
-        if (hipMemcpy(v.data(), P.d_visits.p, v.size() * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
-            return 0;
-        uint64_t sum = 0;
-        for (uint32_t bij : P.order_used()) sum += v[(size_t)(bij >> 16) * nbj + (bij & 0xffffu)];
-        return sum * (32 * 64);
+        return (P.band_all ? P.tset : P.tset_run).tiles * P.tile_rows() * TILE_COLS * nd;
     }
     // dense tiles: 128 x 128 for weighted / plain unweighted, 64 x 64 for generalized and VAW
     const bool small = P.spec.vaw || P.spec.method == Method::generalized;

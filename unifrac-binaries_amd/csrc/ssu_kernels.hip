@@ -7,6 +7,7 @@
 //   pair tiles    register-tiled VALU kernels for weighted / generalized / VAW
 //                 (src/unifrac_task_impl.hpp formulas), FP32 with FP64 merges or FP64
 //   Faith PD      src/unifrac.cpp:362-387, same FP64 summation order
+#include "ssu_devmath.hpp"
 #include "ssu_kernels.hpp"
 #include "ssu_tiles.hpp"
 
@@ -192,14 +193,12 @@ __global__ void __launch_bounds__(256) k_bits_paths(uint32_t* __restrict__ B, ui
 //           with scale_u the other rows hold (float)(klen[r] * e)
 //   SUMS:   Spart[seg][s] = sum_{r in seg} klen[r] * e', increasing r, where e'
 //           is e as the pair kernels see it ((float)e when GATHER, else e)
-//   MASKS:  bit (r % 32) of masks[panel][r / 32] = any e > 0 over the 32
-//           samples of the panel (one wavefront = two panels)
-// E holds the sample columns [col0, col0 + lde); U (row stride ldu) and the
-// masks are indexed by absolute sample, Spart by column within the block.
-template <bool GATHER, bool SUMS, bool MASKS>
+//   BITS:   smask[panel][r] = the 32-sample panel's bits e > 0 (one wavefront = two panels)
+// E holds the sample columns [col0, col0 + lde); U (row stride ldu) and smask
+// are indexed by absolute sample, Spart by column within the block.
+template <bool GATHER, bool SUMS, bool BITS>
 __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums(float* __restrict__ U, size_t ldu, uint32_t col0,
                                                              double* __restrict__ Spart,
-                                                             uint32_t* __restrict__ masks, uint32_t Kw,
                                                              uint32_t* __restrict__ smask,
                                                              const double* __restrict__ E, size_t lde,
                                                              const int32_t* __restrict__ knodes,
@@ -209,12 +208,11 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums(float* __restrict__
                                                              int scale_u) {
     const size_t s = (size_t)blockIdx.x * EMB_THREADS + threadIdx.x;
     if (s >= lde) return;
-    const bool real = s < n_valid;   // columns past the last sample never enter a mask
+    const bool real = s < n_valid;   // columns past the last sample never set a bit
     const uint32_t k0 = blockIdx.y * rows_per_seg;
     const uint32_t k1 = min(K, k0 + rows_per_seg);
     const size_t panel = (col0 + s) / 64 * 2;   // the wave's lower 32-sample panel
     double acc = 0.0;
-    uint32_t lo = 0, hi = 0;
 #pragma unroll 8
     for (uint32_t r = k0; r < k1; ++r) {
         double e = E[(size_t)knodes[r] * lde + s];
@@ -225,20 +223,11 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums(float* __restrict__
             e = (double)f;
         }
         if constexpr (SUMS) acc += klen[r] * e;
-        if constexpr (MASKS) {
+        if constexpr (BITS) {
             const uint64_t b = __ballot(real && e > 0.0);
-            lo |= ((uint32_t)b != 0u ? 1u : 0u) << (r & 31);
-            hi |= ((uint32_t)(b >> 32) != 0u ? 1u : 0u) << (r & 31);
-            if (smask && (threadIdx.x & 63) == 0) {   // the samples themselves, [panel][K]
+            if ((threadIdx.x & 63) == 0) {
                 smask[panel * K + r] = (uint32_t)b;
                 smask[(panel + 1) * K + r] = (uint32_t)(b >> 32);
-            }
-            if ((r & 31) == 31 || r + 1 == k1) {
-                if ((threadIdx.x & 63) == 0) {
-                    masks[panel * Kw + (r >> 5)] = lo;
-                    masks[(panel + 1) * Kw + (r >> 5)] = hi;
-                }
-                lo = hi = 0;
             }
         }
     }
@@ -261,13 +250,12 @@ __device__ __forceinline__ uint32_t spread16(uint32_t x) {
 // the word of the group's row j for panel 0 (2), lane 32 + j that for panel 1
 // (3), and stored as one coalesced store per panel pair, not a one-lane store
 // per row and panel.
-// Needs lde, col0 and ldu even; with masks, lde and col0 multiples of 64, so a
+// Needs lde, col0 and ldu even; with BITS, lde and col0 multiples of 64, so a
 // wave that runs past lde does so by exactly its upper two panels: all its
 // lanes stay (for the stores), those past lde neither load nor store samples.
-template <bool GATHER, bool SUMS, bool MASKS>
+template <bool GATHER, bool SUMS, bool BITS>
 __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums2(float* __restrict__ U, size_t ldu, uint32_t col0,
                                                               double* __restrict__ Spart,
-                                                              uint32_t* __restrict__ masks, uint32_t Kw,
                                                               uint32_t* __restrict__ smask,
                                                               const double* __restrict__ E, size_t lde,
                                                               const int32_t* __restrict__ knodes,
@@ -286,7 +274,6 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums2(float* __restrict_
     const size_t panel = (col0 + wave0) / 32;         // the wave's first 32-sample panel
     const uint32_t npan = lde - wave0 >= 128 ? 4u : 2u;   // panels of the wave inside [0, lde)
     double acc0 = 0.0, acc1 = 0.0;
-    uint32_t pb[4] = {0u, 0u, 0u, 0u};
     uint32_t w01 = 0u, w23 = 0u;
 #pragma unroll 8
     for (uint32_t r = k0; r < k1; ++r) {
@@ -311,30 +298,22 @@ __global__ void __launch_bounds__(EMB_THREADS) k_gather_sums2(float* __restrict_
             acc0 += klen[r] * e0;
             acc1 += klen[r] * e1;
         }
-        if constexpr (MASKS) {
+        if constexpr (BITS) {
             // lane l holds samples wave0 + 2l (b0) and wave0 + 2l + 1 (b1): panel q is lanes 16q .. 16q + 15
             const uint64_t b0 = __ballot(real0 && e0 > 0.0);
             const uint64_t b1 = __ballot(real1 && e1 > 0.0);
-            const uint64_t bo = b0 | b1;
-#pragma unroll
-            for (uint32_t q = 0; q < 4; ++q)
-                pb[q] |= (((bo >> (16 * q)) & 0xffffu) != 0u ? 1u : 0u) << (r & 31);
-            if (smask && (lane & 31) == (r & 31)) {   // row r's words go to lanes r % 32 and 32 + r % 32
+            if ((lane & 31) == (r & 31)) {   // row r's words go to lanes r % 32 and 32 + r % 32
                 const uint32_t sh = 16 * (lane >> 5);
                 w01 = spread16((uint32_t)(b0 >> sh)) | (spread16((uint32_t)(b1 >> sh)) << 1);
                 w23 = spread16((uint32_t)(b0 >> (32 + sh))) | (spread16((uint32_t)(b1 >> (32 + sh))) << 1);
             }
             if ((r & 31) == 31 || r + 1 == k1) {
                 const uint32_t rc = r & ~31u, rows = (r & 31) + 1;   // this group's first row, its rows
-                if (smask && (lane & 31) < rows) {
+                if ((lane & 31) < rows) {
                     const uint32_t q = lane >> 5;
                     smask[(panel + q) * K + rc + (lane & 31)] = w01;
                     if (npan == 4) smask[(panel + 2 + q) * K + rc + (lane & 31)] = w23;
                 }
-                if (lane == 0)
-                    for (uint32_t q = 0; q < npan; ++q) masks[(panel + q) * Kw + (r >> 5)] = pb[q];
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) pb[q] = 0u;
             }
         }
     }
@@ -723,80 +702,13 @@ template <> __device__ __forceinline__ double dsqrt<double>(double x) { return s
 template <class T> __device__ __forceinline__ T dpow(T x, T a);
 template <> __device__ __forceinline__ float dpow<float>(float x, float a) { return powf(x, a); }
 
-// FP64 log2 of a positive normal x: x = m 2^e with m in [sqrt(1/2), sqrt(2)),
-// log2 m = (2 / ln 2) atanh t with t = (m - 1) / (m + 1), |t| <= 0.1716, summed
-// as t (1 + t^2/3 + t^4/5 + ... + t^24/25) (the next term is below 2e-20 of the
-// sum): a few ulps, against the many branches of the general pow.
-__device__ __forceinline__ double log2_normal(double x) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    int e = (int)((b >> 52) & 0x7ff) - 1022;
-    double m = __longlong_as_double((long long)((b & 0x000fffffffffffffull) | 0x3fe0000000000000ull));  // [0.5, 1)
-    if (m < 0.70710678118654752440) { m *= 2.0; --e; }
-    const double t = (m - 1.0) / (m + 1.0), t2 = t * t;
-    double p = 1.0 / 25.0;
-    p = fma(p, t2, 1.0 / 23.0);
-    p = fma(p, t2, 1.0 / 21.0);
-    p = fma(p, t2, 1.0 / 19.0);
-    p = fma(p, t2, 1.0 / 17.0);
-    p = fma(p, t2, 1.0 / 15.0);
-    p = fma(p, t2, 1.0 / 13.0);
-    p = fma(p, t2, 1.0 / 11.0);
-    p = fma(p, t2, 1.0 / 9.0);
-    p = fma(p, t2, 1.0 / 7.0);
-    p = fma(p, t2, 1.0 / 5.0);
-    p = fma(p, t2, 1.0 / 3.0);
-    p = fma(p, t2, 1.0);
-    return (double)e + (t * p) * 2.88539008177792681472;   // 2 / ln 2
-}
-
-// FP64 2^y for |y| < 1000: y = k + f with k = rint(y), |f| <= 1/2, and
-// 2^f = e^z, z = f ln 2, from the Taylor series to z^16/16! (|z| <= 0.347:
-// the next term is below 1e-21), scaled by 2^k in the exponent bits.
-__device__ __forceinline__ double exp2_finite(double y) {
-    const double k = rint(y);
-    const double z = (y - k) * 0.69314718055994530942;   // ln 2
-    double p = 1.0 / 20922789888000.0;                    // 1/16!
-    p = fma(p, z, 1.0 / 1307674368000.0);
-    p = fma(p, z, 1.0 / 87178291200.0);
-    p = fma(p, z, 1.0 / 6227020800.0);
-    p = fma(p, z, 1.0 / 479001600.0);
-    p = fma(p, z, 1.0 / 39916800.0);
-    p = fma(p, z, 1.0 / 3628800.0);
-    p = fma(p, z, 1.0 / 362880.0);
-    p = fma(p, z, 1.0 / 40320.0);
-    p = fma(p, z, 1.0 / 5040.0);
-    p = fma(p, z, 1.0 / 720.0);
-    p = fma(p, z, 1.0 / 120.0);
-    p = fma(p, z, 1.0 / 24.0);
-    p = fma(p, z, 1.0 / 6.0);
-    p = fma(p, z, 0.5);
-    p = fma(p, z, 1.0);
-    p = fma(p, z, 1.0);
-    return ldexp(p, (int)k);
-}
-
-// x^a for x > 0 in FP64: 2^(a log2 x) for the normal range, the general pow otherwise
+// any a (dense pair tiles): the general pow outside the range of the straight-line form
 template <> __device__ __forceinline__ double dpow<double>(double x, double a) {
     if (x >= 2.2250738585072014e-308 && x < 1.0e300) {
-        const double y = a * log2_normal(x);
+        const double y = a * log2_pos(x);
         if (y > -1000.0 && y < 1000.0) return exp2_finite(y);
     }
     return pow(x, a);
-}
-
-// 1 / sqrt(x) for normal x > 0 in FP64: the hardware FP64 reciprocal square
-// root approximation (5.2e-8 relative at most, measured over 1e-30..1e30)
-// refined by STEPS Newton steps r += r (1 - x r^2) / 2, each of which squares
-// the relative error (one step: 4.1e-15; two: FP64 rounding).  Straight-line
-// code, no branch.
-template <int STEPS> __device__ __forceinline__ double rsqrt_nr(double x) {
-    double r = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        const double e = fma(-x * r, r, 1.0);
-        r = fma(0.5 * r, e, r);
-    }
-    return r;
 }
 
 // Newton steps after the hardware start: FP64 values two (FP64 rounding);
@@ -1153,261 +1065,6 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
         }
 }
 
-// ------------------------------------------------------ generalized pair blocks
-//
-// 32 x 64 blocks of pairs that only visit the nodes present in one of their
-// sample panels: the OR of the panels' node masks.
-
-// Compacts the set bits of the wave's 64 mask words (lane l holds word l) into
-// list[], in increasing order of l * 32 + bit; returns their number (uniform).
-__device__ __forceinline__ uint32_t build_list(uint16_t* list, uint32_t word, uint32_t lane) {
-    const uint32_t cnt = __popc(word);
-    uint32_t incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(incl, d, 64);
-        if ((int)lane >= d) incl += y;
-    }
-    const uint32_t total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
-    uint32_t o = incl - cnt;
-    while (word) {
-        const uint32_t b = __ffs(word) - 1;
-        list[o++] = (uint16_t)(lane * 32 + b);
-        word &= word - 1;
-    }
-    __syncthreads();
-    return total;
-}
-
-constexpr uint32_t SP_WORDS = 64;    // mask words (32 nodes each) per list chunk
-
-// Blocks are numbered so that each XCD (workgroups go to the XCDs round robin)
-// walks a contiguous run of `order` (rect_block_order): the blocks resident
-// on one XCD then share their sample panels in that XCD's L2.
-
-// FP32 operands: 32 x 64 blocks of pairs (rows: a 32-sample panel, columns:
-// a 64-sample panel), one wavefront each, a 4 x 8 tile per lane.  The kernel
-// sums l * |u - v| directly over the nodes either panel holds (the dense
-// nodes, with the occupancy split): v_sub_f32 + v_fma_f32 with an |x| source
-// modifier, summed in FP32 over S3_MERGE listed nodes and then merged into
-// FP64, so the distance never comes from a difference of large sums and stays
-// accurate for near-identical samples.  S only normalises.  Only pairs i < j
-// are written (both (i, j) and (j, i)), so every pair has one writer even
-// where blocks straddle the diagonal.
-constexpr uint32_t S3_BI = 32, S3_BJ = 64;
-constexpr uint32_t S3_EB = 8;          // nodes per step; two steps in flight
-constexpr uint32_t S3_MERGE = 64;      // FP32 accumulation span, in listed nodes
-constexpr uint32_t S3_GSJ = 12;        // column groups of 8 floats sit 48 bytes apart (bank-conflict free)
-constexpr uint32_t S3_JOFF = 32;       // the 32 row values come first, contiguous
-constexpr uint32_t S3_NODE = S3_JOFF + 8 * S3_GSJ;
-
-
-// generalized (GEN) terms, FP32 as in the dense kernel: w = s^a l, q = s^(a-1) l
-// from the hardware log2 / exp2 (s = u + v > 0), or, HALF (a = 1/2), from the
-// hardware square root and reciprocal square root; num += q |u - v|, den += w
-template <bool HALF = false>
-__device__ __forceinline__ void gen_term(float u, float v, float l, float alpha, float& num, float& den) {
-    const float s = u + v;
-    const bool nz = s != 0.0f;
-    float w, q;
-    if constexpr (HALF) {
-        const float ss = nz ? s : 1.0f;
-        w = nz ? __builtin_amdgcn_sqrtf(ss) * l : 0.0f;
-        q = nz ? __builtin_amdgcn_rsqf(ss) * l : 0.0f;
-    } else {
-        const float lg = __builtin_amdgcn_logf(nz ? s : 1.0f);
-        w = nz ? __builtin_amdgcn_exp2f(alpha * lg) * l : 0.0f;
-        q = nz ? __builtin_amdgcn_exp2f((alpha - 1.0f) * lg) * l : 0.0f;
-    }
-    num = __builtin_fmaf(q, __builtin_fabsf(u - v), num);
-    den += w;
-}
-// FP64 as in the dense FP64 kernel: w = s^a l, num += w |u - v| / s, den += w
-template <bool HALF = false>   // (FP64: dpow for every alpha)
-__device__ __forceinline__ void gen_term(double u, double v, double l, double alpha, double& num, double& den) {
-    const double s = u + v;
-    const bool nz = s != 0.0;
-    const double ss = nz ? s : 1.0;
-    const double w = nz ? dpow<double>(ss, alpha) * l : 0.0;
-    num = fma(w, __builtin_fabs(u - v) / ss, num);
-    den += w;
-}
-
-// V: the operand type.  FP32 operands are the gathered rows U[r] of the
-// processed nodes, summed in FP32 over S3_MERGE listed nodes and then merged
-// into FP64; FP64 operands (generalized only) are the embedding rows
-// U[rows[r]], summed in FP64.
-template <class TOut, bool GEN, class V = float, bool HALF = false>
-__device__ __forceinline__ void pairs_sparse32_body(const V* __restrict__ U, const int32_t* __restrict__ rows,
-                                                       size_t ldn, const double* __restrict__ len,
-                                                       const uint32_t* __restrict__ masks, uint32_t Kw, uint32_t n,
-                                                       const double* __restrict__ S, int normalized,
-                                                       TOut* __restrict__ out, uint32_t* __restrict__ visits,
-                                                       const uint32_t* __restrict__ order, uint32_t n_blocks,
-                                                       uint32_t per_xcd, const uint32_t* __restrict__ dmask,
-                                                       int add_partial, V alpha, TOut* __restrict__ out2) {
-    constexpr bool F64 = sizeof(V) == 8;
-    static_assert(!F64 || GEN, "FP64 operands take the generalized terms only");
-    constexpr uint32_t EB = S3_EB;
-    const uint32_t seq = (blockIdx.x % N_XCDS) * per_xcd + blockIdx.x / N_XCDS;
-    if (seq >= n_blocks) return;
-    const uint32_t pi = order[seq] >> 16, pj = order[seq] & 0xffffu;   // 32-panel, 64-panel
-    uint32_t visited = 0;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t li = lane >> 3, lj = lane & 7;
-
-    __shared__ uint16_t list[SP_WORDS * 32];
-    __shared__ __attribute__((aligned(16))) V sv[EB][S3_NODE];
-    __shared__ V sl[EB];
-
-    V acc[4][8];
-    double acc64[4][8];
-    V accd[GEN ? 4 : 1][GEN ? 8 : 1];        // GEN: the denominator
-    double accd64[GEN ? 4 : 1][GEN ? 8 : 1];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            acc[r][c] = V(0);
-            acc64[r][c] = 0.0;
-            if constexpr (GEN) { accd[r][c] = V(0); accd64[r][c] = 0.0; }
-        }
-    uint32_t pending = 0;
-
-    const uint32_t* mI = masks + (size_t)pi * Kw;
-    const uint32_t* mJ = masks + (size_t)(2 * pj) * Kw;
-    const size_t offI = (size_t)pi * S3_BI + (lane & 31), offJ = (size_t)pj * S3_BJ + lane;
-    const uint32_t slotJ = S3_JOFF + (lane >> 3) * S3_GSJ + (lane & 7);
-
-    for (uint32_t w0 = 0; w0 < Kw; w0 += SP_WORDS) {
-        const uint32_t w = w0 + lane;
-        uint32_t word = w < Kw ? (mI[w] | mJ[w] | mJ[Kw + w]) : 0u;
-        if (dmask && w < Kw) word &= dmask[w];   // the other nodes come from the posting-list kernel
-        const uint32_t total = build_list(list, word, lane);
-        visited += total;
-        const uint32_t base = w0 * 32;
-        V pA[EB], qA[EB], pB[EB], qB[EB];
-        V lA = V(0), lB = V(0);
-        uint64_t vA = 0, vB = 0;
-        auto fetch = [&](V (&p)[EB], V (&q)[EB], V& l, uint64_t& valid, uint32_t t0)
-                         __attribute__((always_inline)) {
-            const uint32_t idx = t0 + lane;
-            const bool real = lane < EB && idx < total;
-            int32_t row = 0;
-            l = V(0);
-            if (real) {
-                const uint32_t r = base + list[idx];
-                row = F64 ? rows[r] : (int32_t)r;
-                l = (V)len[r];
-            }
-            valid = __ballot(real);
-#pragma unroll
-            for (uint32_t e = 0; e < EB; ++e) {
-                const size_t off = (size_t)__builtin_amdgcn_readlane(row, e) * ldn;
-                p[e] = U[off + offI];      // lanes 32..63 repeat lanes 0..31
-                q[e] = U[off + offJ];
-            }
-        };
-        auto step = [&](V (&p)[EB], V (&q)[EB], V& l, uint64_t& valid, uint32_t t_next)
-                        __attribute__((always_inline)) {
-#pragma unroll
-            for (uint32_t e = 0; e < EB; ++e) {
-                const bool on = (valid >> e) & 1;
-                if (lane < S3_BI) sv[e][lane] = on ? p[e] : V(0);
-                sv[e][slotJ] = on ? q[e] : V(0);
-            }
-            if (lane < EB) sl[lane] = l;
-            __syncthreads();
-            if (t_next < total) fetch(p, q, l, valid, t_next);
-#pragma unroll 2
-            for (uint32_t e = 0; e < EB; ++e) {
-                V a[4], b[8];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = sv[e][li * 4 + r];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) b[c] = sv[e][S3_JOFF + lj * S3_GSJ + c];
-                const V ln = sl[e];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        if constexpr (GEN)
-                            gen_term<HALF>(a[r], b[c], ln, alpha, acc[r][c], accd[r][c]);
-                        else
-                            acc[r][c] = __builtin_fmaf(__builtin_fabsf(a[r] - b[c]), ln, acc[r][c]);
-                    }
-            }
-            if constexpr (!F64) {
-                pending += EB;
-                if (pending >= S3_MERGE) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int c = 0; c < 8; ++c) {
-                            acc64[r][c] += (double)acc[r][c];
-                            acc[r][c] = 0.0f;
-                            if constexpr (GEN) { accd64[r][c] += (double)accd[r][c]; accd[r][c] = 0.0f; }
-                        }
-                    pending = 0;
-                }
-            }
-            __syncthreads();
-        };
-        if (total) fetch(pA, qA, lA, vA, 0);
-        if (total > EB) fetch(pB, qB, lB, vB, EB);
-        for (uint32_t t0 = 0; t0 < total; t0 += 2 * EB) {
-            step(pA, qA, lA, vA, t0 + 2 * EB);
-            if (t0 + EB >= total) break;
-            step(pB, qB, lB, vB, t0 + 3 * EB);
-        }
-    }
-
-    if (visits && lane == 0) visits[(size_t)pi * ((n + S3_BJ - 1) / S3_BJ) + pj] = visited;
-    const size_t i0 = (size_t)pi * S3_BI + li * 4, j0 = (size_t)pj * S3_BJ + lj * 8;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const size_t i = i0 + r, j = j0 + c;
-            if (j >= n || i > j) continue;
-            if (i == j) { out[i * n + i] = (TOut)0; continue; }
-            double x = acc64[r][c] + (double)acc[r][c];
-            if (add_partial) x += (double)out[i * n + j];   // the sparse nodes' share, from k_pairs_rows
-            x = x < 0.0 ? 0.0 : x;   // the share's rounding can undershoot 0; NaN (empty samples) passes
-            double d;
-            if constexpr (GEN) {
-                double y = accd64[r][c] + (double)accd[r][c];
-                if (add_partial) y += (double)out2[i * n + j];
-                d = x / y;   // 0 / 0 (no node held by either sample) gives NaN, as the dense kernel
-            } else {
-                d = normalized ? x / (S[i] + S[j]) : x;
-            }
-            out[i * n + j] = (TOut)d;
-            out[j * n + i] = (TOut)d;
-        }
-}
-
-// generalized: numerator and denominator summed directly (two accumulator sets, 2 waves per SIMD)
-template <class TOut, bool HALF = false>
-__global__ void __launch_bounds__(64) k_pairs_gen32(
-        const float* __restrict__ U, size_t ldn, const double* __restrict__ len, const uint32_t* __restrict__ masks,
-        uint32_t Kw, uint32_t n, TOut* __restrict__ out, TOut* __restrict__ out2, uint32_t* __restrict__ visits,
-        const uint32_t* __restrict__ order, uint32_t n_blocks, uint32_t per_xcd, const uint32_t* __restrict__ dmask,
-        int add_partial, float alpha) {
-    pairs_sparse32_body<TOut, true, float, HALF>(U, nullptr, ldn, len, masks, Kw, n, nullptr, 1, out, visits, order, n_blocks,
-                                    per_xcd, dmask, add_partial, alpha, out2);
-}
-
-// generalized on FP64 operands: the FP64 embedding rows, FP64 terms and sums (one wave per SIMD)
-__global__ void __launch_bounds__(64) k_pairs_gen64(
-        const double* __restrict__ U, const int32_t* __restrict__ rows, size_t ldn, const double* __restrict__ len,
-        const uint32_t* __restrict__ masks, uint32_t Kw, uint32_t n, double* __restrict__ out,
-        double* __restrict__ out2, uint32_t* __restrict__ visits, const uint32_t* __restrict__ order,
-        uint32_t n_blocks, uint32_t per_xcd, const uint32_t* __restrict__ dmask, int add_partial, double alpha) {
-    pairs_sparse32_body<double, true, double>(U, rows, ldn, len, masks, Kw, n, nullptr, 1, out, visits, order,
-                                              n_blocks, per_xcd, dmask, add_partial, alpha, out2);
-}
-
 // --------------------------------------------- sparse nodes: posting lists
 
 // Node occupancy split: a node held by at least `thr` samples is dense (its
@@ -1671,7 +1328,9 @@ template <class TV> struct alignas(16) RowEntry<TV, true> {   // generalized
 __device__ __forceinline__ float gen_pow(float x, double alpha) {
     return alpha == 0.5 ? __builtin_amdgcn_sqrtf(x) : pow_alpha(x, (float)alpha);
 }
-__device__ __forceinline__ double gen_pow(double x, double alpha) { return dpow<double>(x, alpha); }
+__device__ __forceinline__ double gen_pow(double x, double alpha) {   // (0 <= alpha <= 1)
+    return alpha == 0.5 ? sqrt(x) : dpow64(x, alpha);
+}
 
 // round(x * ls) as a signed integer (two's complement in the 64-bit
 // accumulators) for |x * ls| < 2^51: the FMA adds 1.5 * 2^52, so the sum lies
@@ -1702,8 +1361,8 @@ __device__ __forceinline__ void row_term(unsigned long long* accb, const RowEntr
         // FP64 values: the same corrections in FP64, truncated to integers in units
         // of 2^-61 of the row's bound (|x * ls| < 2^61)
         const double uu = en.lu, vv = v, sm = uu + vv;
-        const double p1 = dpow<double>(sm, alpha - 1.0);
-        const double one = en.uap + dpow<double>(vv, alpha);
+        const double p1 = alpha == 0.5 ? rsqrt_nr<2>(sm) : dpow64(sm, alpha - 1.0);
+        const double one = en.uap + gen_pow(vv, alpha);
         const double ls = __longlong_as_double((long long)en.q8);
         const double cn = p1 * __builtin_fabs(uu - vv) - one;
         const double cd = p1 * sm - one;
@@ -2586,27 +2245,26 @@ uint32_t gather_segments(uint32_t K, size_t ldn) {
 
 template <bool G, bool S, bool M>
 static void gather_sums_t(dim3 grid, hipStream_t st, float* U, size_t ldu, uint32_t col0, double* Spart,
-                          uint32_t* masks, uint32_t Kw, uint32_t* smask, const double* E, size_t lde,
+                          uint32_t* smask, const double* E, size_t lde,
                           const int32_t* knodes, const double* klen, uint32_t K, uint32_t rps, uint32_t n_valid,
                           const uint32_t* rare_u, bool write_rare, bool scale_u) {
     // two samples per thread where the layout allows 16-byte loads (SSU_GATHER2=0: one)
     static const bool two_ok = !(getenv("SSU_GATHER2") && atoi(getenv("SSU_GATHER2")) == 0);
     if (two_ok && lde % 2 == 0 && col0 % 2 == 0 && ldu % 2 == 0) {
         const dim3 g2(grid1(lde / 2, EMB_THREADS), grid.y);
-        hipLaunchKernelGGL((k_gather_sums2<G, S, M>), g2, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart, masks, Kw,
+        hipLaunchKernelGGL((k_gather_sums2<G, S, M>), g2, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart,
                            smask, E, lde, knodes, klen, K, rps, n_valid, rare_u, (int)write_rare, (int)scale_u);
         return;
     }
-    hipLaunchKernelGGL((k_gather_sums<G, S, M>), grid, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart, masks, Kw,
+    hipLaunchKernelGGL((k_gather_sums<G, S, M>), grid, dim3(EMB_THREADS), 0, st, U, ldu, col0, Spart,
                        smask, E, lde, knodes, klen, K, rps, n_valid, rare_u, (int)write_rare, (int)scale_u);
 }
 
-hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* masks, uint32_t* smask,
+hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* smask,
                               const double* E, size_t lde, uint32_t col0, const int32_t* knodes, const double* klen,
                               uint32_t K, uint32_t n, hipStream_t st, const uint32_t* rare_u, uint32_t rps_fixed, bool write_rare, bool scale_u) {
-    if (masks && (lde % 64 || col0 % 64)) return hipErrorInvalidValue;
+    if (smask && (lde % 64 || col0 % 64)) return hipErrorInvalidValue;
     if (rps_fixed % 32) return hipErrorInvalidValue;
-    if (smask && !masks) return hipErrorInvalidValue;
     if (scale_u && !klen) return hipErrorInvalidValue;
     if (col0 >= n) return hipSuccess;
     const uint32_t cnt = (uint32_t)std::min<size_t>(lde, n - col0);   // real samples in this block
@@ -2619,19 +2277,18 @@ hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, ui
     const uint32_t cb = grid1(ldn, EMB_THREADS);
     const uint32_t segs0 = gather_segments(K, ldn);
     const uint32_t rps = rps_fixed ? rps_fixed
-                                   : (((K + segs0 - 1) / segs0) + 31) / 32 * 32;   // mask words never straddle segments
+                                   : (((K + segs0 - 1) / segs0) + 31) / 32 * 32;   // 32-row groups never straddle segments
     const uint32_t segs = (K + rps - 1) / rps;
-    const uint32_t Kw = (K + 31) / 32;
     const dim3 grid(cb, segs);
-    const int key = (U ? 4 : 0) | (S ? 2 : 0) | (masks ? 1 : 0);
+    const int key = (U ? 4 : 0) | (S ? 2 : 0) | (smask ? 1 : 0);
     switch (key) {
-    case 7: gather_sums_t<true, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 6: gather_sums_t<true, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 5: gather_sums_t<true, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 4: gather_sums_t<true, false, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 3: gather_sums_t<false, true, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 2: gather_sums_t<false, true, false>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
-    case 1: gather_sums_t<false, false, true>(grid, st, U, ldu, col0, Spart, masks, Kw, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 7: gather_sums_t<true, true, true>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 6: gather_sums_t<true, true, false>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 5: gather_sums_t<true, false, true>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 4: gather_sums_t<true, false, false>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 3: gather_sums_t<false, true, true>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 2: gather_sums_t<false, true, false>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
+    case 1: gather_sums_t<false, false, true>(grid, st, U, ldu, col0, Spart, smask, E, lde, knodes, klen, K, rps, cnt, rare_u, write_rare, scale_u); break;
     case 0: return hipSuccess;
     default: return hipErrorInvalidValue;
     }
@@ -2708,18 +2365,6 @@ std::vector<uint32_t> upper_block_order(uint32_t nb, uint32_t super) {
         for (uint32_t sj = si; sj < nb; sj += super)
             for (uint32_t bi = si; bi < std::min(nb, si + super); ++bi)
                 for (uint32_t bj = std::max(bi, sj); bj < std::min(nb, sj + super); ++bj) order.push_back(bi << 16 | bj);
-    return order;
-}
-
-std::vector<uint32_t> rect_block_order(uint32_t n) {
-    constexpr uint32_t SI = 32, SJ = 16;   // 32 x 16 blocks of 32 x 64 pairs: ~ the waves resident on one XCD
-    const uint32_t nbi = (n + S3_BI - 1) / S3_BI, nbj = (n + S3_BJ - 1) / S3_BJ;
-    std::vector<uint32_t> order;
-    for (uint32_t si = 0; si < nbi; si += SI)
-        for (uint32_t sj = si / 2; sj < nbj; sj += SJ)
-            for (uint32_t bi = si; bi < std::min(nbi, si + SI); ++bi)
-                for (uint32_t bj = sj; bj < std::min(nbj, sj + SJ); ++bj)
-                    if (bi <= 2 * bj + 1) order.push_back(bi << 16 | bj);
     return order;
 }
 
@@ -2919,39 +2564,6 @@ uint32_t row_list_chunks(uint32_t n, uint32_t K) {
 size_t offset_scan_blocks(uint32_t K) { return ((size_t)K + SCAN_BLOCK - 1) / SCAN_BLOCK; }
 size_t row_list_scan_blocks(uint32_t n, uint32_t K) {
     return ((size_t)n * row_list_chunks(n, K) + SCAN_BLOCK - 1) / SCAN_BLOCK;
-}
-
-hipError_t launch_pairs_gen32(const SparseArgs& a, float alpha, void* out2, hipStream_t st) {
-    if (a.ldn % S3_BJ || a.out_fp64) return hipErrorInvalidValue;
-    const uint32_t nbj = (a.n + S3_BJ - 1) / S3_BJ;
-    if (!nbj) return hipSuccess;
-    if (a.dmask && !out2) return hipErrorInvalidValue;
-    if (!a.order) return hipErrorInvalidValue;
-    if (!a.n_blocks) return hipSuccess;   // a stripe selection without a block here
-    const uint32_t per_xcd = (a.n_blocks + N_XCDS - 1) / N_XCDS;
-    if (alpha == 0.5f)   // square roots in place of log2 / exp2 (gen_term's HALF)
-        hipLaunchKernelGGL((k_pairs_gen32<float, true>), dim3(per_xcd * N_XCDS), dim3(64), 0, st, (const float*)a.U,
-                           a.ldn, a.len, a.masks, a.Kw, a.n, (float*)a.out, (float*)out2, a.visits, a.order,
-                           a.n_blocks, per_xcd, a.dmask, (int)(a.dmask != nullptr), alpha);
-    else
-        hipLaunchKernelGGL((k_pairs_gen32<float>), dim3(per_xcd * N_XCDS), dim3(64), 0, st, (const float*)a.U, a.ldn,
-                           a.len, a.masks, a.Kw, a.n, (float*)a.out, (float*)out2, a.visits, a.order, a.n_blocks,
-                           per_xcd, a.dmask, (int)(a.dmask != nullptr), alpha);
-    return hipGetLastError();
-}
-
-hipError_t launch_pairs_gen64(const SparseArgs& a, double alpha, void* out2, hipStream_t st) {
-    if (a.ldn % S3_BJ || !a.out_fp64 || !a.rows) return hipErrorInvalidValue;
-    const uint32_t nbj = (a.n + S3_BJ - 1) / S3_BJ;
-    if (!nbj) return hipSuccess;
-    if (a.dmask && !out2) return hipErrorInvalidValue;
-    if (!a.order) return hipErrorInvalidValue;
-    if (!a.n_blocks) return hipSuccess;   // a stripe selection without a block here
-    const uint32_t per_xcd = (a.n_blocks + N_XCDS - 1) / N_XCDS;
-    hipLaunchKernelGGL(k_pairs_gen64, dim3(per_xcd * N_XCDS), dim3(64), 0, st, (const double*)a.U, a.rows, a.ldn,
-                       a.len, a.masks, a.Kw, a.n, (double*)a.out, (double*)out2, a.visits, a.order, a.n_blocks,
-                       per_xcd, a.dmask, (int)(a.dmask != nullptr), alpha);
-    return hipGetLastError();
 }
 
 template <class TIn>

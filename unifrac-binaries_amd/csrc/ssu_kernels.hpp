@@ -119,16 +119,14 @@ hipError_t launch_bits_smask(uint32_t* smask, const uint32_t* B, uint32_t ldb, c
 //   S (if non-null): S[s] = sum_r klen[r] * u_rs in FP64 (u as the pair kernels
 //     see it: FP32-rounded when U is written), summed per segment then over
 //     segments in order, into S[col0 ..]; Spart holds gather_segments(K, lde) * lde doubles;
-//   masks (if non-null; lde, col0 multiples of 64): [ldn/32][ceil(K/32)] words, bit r%32 of
-//     word r/32 of panel p set iff some sample of p*32..p*32+31 has u_rs > 0;
-//   smask (if non-null, with masks): [ldn/32][K] words, bit s%32 of smask[s/32][r] = u_rs > 0;
+//   smask (if non-null; lde, col0 multiples of 64): [ldn/32][K] words, bit s%32 of smask[s/32][r] = u_rs > 0;
 //   rare_u (optional, [ceil(K/32)] words): rows r with bit r set are not written to U (S and
-//     the masks still see their FP32-rounded values), unless write_rare;
+//     the bits still see their FP32-rounded values), unless write_rare;
 //   scale_u: U[r] = (float)(klen[r] * E[knodes[r]]) instead (one rounding), the rare rows excepted.
 uint32_t gather_segments(uint32_t K, size_t ldn);
 //   rps_fixed (optional, a multiple of 32): rows per segment, in place of the
 //     default that depends on lde (S then depends on a sample's column alone).
-hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* masks, uint32_t* smask,
+hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, uint32_t* smask,
                               const double* E,
                               size_t lde, uint32_t col0, const int32_t* knodes, const double* klen, uint32_t K,
                               uint32_t n, hipStream_t st, const uint32_t* rare_u = nullptr, uint32_t rps_fixed = 0,
@@ -201,31 +199,12 @@ struct PairArgs {
 };
 hipError_t launch_pairs(PairOp op, bool fp64, const PairArgs& a, hipStream_t st);
 
-// Generalized pair blocks (launch_pairs_gen32 / gen64).
-struct SparseArgs {
-    const void* U;          // node rows, float (row r) or double (row rows[r])
-    const int32_t* rows;    // nullptr: identity
-    size_t ldn;             // multiple of 64
-    const double* len;      // [K] lengths as the accumulation uses them
-    const uint32_t* masks;  // from launch_gather_sums
-    uint32_t Kw;            // ceil(K / 32)
-    uint32_t n;
-    const double* S;        // per-sample sums from launch_gather_sums
-    bool normalized;
-    void* out;              // n x n
-    bool out_fp64;
-    uint32_t* visits;       // optional [nb][nb], nb = ceil(n/64): nodes visited per block (bi <= bj)
-    const uint32_t* order;  // device copy of upper_block_order(ceil(n/64), 16)
-    uint32_t n_blocks;      // its length, nb (nb + 1) / 2
-    const uint32_t* dmask = nullptr;   // visit only these nodes and add the posting-list shares in `out`
-};
-
 // Occupancy split.  Weighted (shared-node path, FP32 or FP64 values): nodes
 // held by at least `thr` samples are dense (bit set in dmask, [ceil(K/32)]
 // words, set here by launch_sparse_lists); for the others the posting lists
 // are built from the value rows and the sample masks at offsets scanned from
 // their counts, and each row's share over them is written, in the value type,
-// to out[a * n + b] (b > a) for the tiled kernel to add (SparseArgs::dmask):
+// to out[a * n + b] (b > a) for the tiles to add (TileArgs::add_partial):
 // with FP32 values the share of sum l |u_a - u_b| (ssp[a] + ssp[b] - 2 M,
 // formed in FP64), with FP64 values the share of M.  Unweighted (gram != nullptr): the K nodes are the
 // plan's sparse nodes with offsets fixed when the plan is built (dmask all
@@ -310,17 +289,6 @@ size_t row_list_scan_blocks(uint32_t n, uint32_t K);
 // The upper-triangle blocks (bi <= bj < nb) as bi << 16 | bj, super x super
 // super-tile by super-tile; kernels walk it in XCD-contiguous runs.
 std::vector<uint32_t> upper_block_order(uint32_t nb, uint32_t super);
-// 32 x 64 blocks (32-sample row panel pi <= 2 pj + 1, 64-sample column panel pj):
-// `order` = rect_block_order(n) and visits is [ceil(n/32)][ceil(n/64)].
-std::vector<uint32_t> rect_block_order(uint32_t n);
-// generalized (FP32, 0 <= alpha <= 1) on the same blocks: numerator and denominator summed
-// directly over the nodes either panel holds; with dmask, adds the posting-list shares in
-// out (numerator) and out2 (denominator)
-hipError_t launch_pairs_gen32(const SparseArgs& a, float alpha, void* out2, hipStream_t st);
-// the same on FP64 operands (U: the FP64 embedding, row rows[r] for processed node r),
-// FP64 terms, sums and output
-hipError_t launch_pairs_gen64(const SparseArgs& a, double alpha, void* out2, hipStream_t st);
-
 // --------------------------------------------------------- output layouts
 // stripes[s - start][k] = M[k][(k+s+1) % n]   (double output)
 template <class TIn>

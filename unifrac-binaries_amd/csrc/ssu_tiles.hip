@@ -8,6 +8,7 @@
 // apart from the next lane's, so that its operands are ds_read_b128 of 8
 // distinct contiguous pieces (no bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
 // to LDS by global_load_lds, 16 bytes per lane, a stage of nodes ahead.
+#include "ssu_devmath.hpp"
 #include "ssu_tiles.hpp"
 
 #include <algorithm>
@@ -34,10 +35,20 @@ __device__ __forceinline__ void part_range(uint32_t nd, uint32_t eb, uint32_t p,
 // An operation says what a lane holds and how a node's values enter a pair:
 //   V        operand type; FP32 sums are merged into FP64 every MERGE nodes
 //   RL       rows a lane holds (8, or 4 with two sums per pair), so a tile has 16 RL rows
-//   EB       nodes per LDS stage (two stages are resident)
+//   EB       nodes per LDS stage (two stages are resident), UNROLL of them in one loop body
 //   TWO      a denominator is summed beside the numerator
 //   LEN      the node's length is staged too (otherwise U's rows are scaled by it)
+//   COUNTS   the samples' counts are staged beside their values, and the pair's totals used (VAW)
+//   prep     what a lane does to a value it reads
 constexpr uint32_t MERGE = 64;
+
+// the distance from numerator and denominator and the rare nodes' shares of them
+// (0 / 0, no node held by either sample: NaN)
+__device__ __forceinline__ double ratio(double nm, double dn, double share, double share2, bool normalized) {
+    nm += share;
+    nm = nm < 0.0 ? 0.0 : nm;   // the shares' rounding can undershoot 0
+    return normalized ? nm / (dn + share2) : nm;
+}
 
 // FP32 weighted: |l u - l v|, two instructions at the full FP32 rate (register
 // operands only: an SGPR operand halves it, as do min, max and v_sad_u32).
@@ -47,13 +58,13 @@ constexpr uint32_t MERGE = 64;
 // took 70.4 ms.
 struct OpW32 {
     typedef float V;
-    static constexpr int RL = 8, EB = 16;
-    static constexpr bool TWO = false, LEN = false;
-    static __device__ __forceinline__ void term(float u, float v, float, float& num, float&) {
-        num += __builtin_fabsf(u - v);
-    }
-    // d from the tile's sum x and the rare nodes' share of it
-    static __device__ __forceinline__ double distance(double x, double share, double tot, bool normalized) {
+    static constexpr int RL = 8, EB = 16, UNROLL = 16, BATCH = 1;
+    static constexpr bool TWO = false, LEN = false, COUNTS = false, FLAGS = false;
+    static __device__ __forceinline__ float prep(float u) { return u; }
+    static __device__ __forceinline__ void term(float u, float v, float, float& num) { num += __builtin_fabsf(u - v); }
+    // d from the tile's sums x, y and the rare nodes' shares of them
+    static __device__ __forceinline__ double distance(double x, double, double share, double, double tot,
+                                                      bool normalized) {
         x += share;
         x = x < 0.0 ? 0.0 : x;   // the share's rounding can undershoot 0; NaN (empty samples) passes
         return normalized ? x / tot : x;
@@ -67,17 +78,69 @@ struct OpW32 {
 // wave; 131 samples 0.37 -> 0.04 ms, the parts filling the device.
 struct OpW64 {
     typedef double V;
-    static constexpr int RL = 8, EB = 8;
-    static constexpr bool TWO = false, LEN = true;
-    static __device__ __forceinline__ void term(double u, double v, double l, double& num, double&) {
+    static constexpr int RL = 8, EB = 8, UNROLL = 8, BATCH = 1;
+    static constexpr bool TWO = false, LEN = true, COUNTS = false, FLAGS = false;
+    static __device__ __forceinline__ double prep(double u) { return u; }
+    static __device__ __forceinline__ void term(double u, double v, double l, double& num) {
         double m;
         asm("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(u), "v"(v));
         num = __builtin_fma(m, l, num);
     }
-    static __device__ __forceinline__ double distance(double m, double share, double tot, bool normalized) {
+    static __device__ __forceinline__ double distance(double m, double, double share, double, double tot,
+                                                      bool normalized) {
         double x = tot - 2.0 * (m + share);
         x = x < 0.0 ? 0.0 : x;
         return normalized ? x / tot : x;
+    }
+};
+
+// s^(a-1) for s >= 0, finite at s = 0 (the terms it weighs are 0 there).  AL
+// picks the power: 0 any a (FP32: hardware log2 / exp2), 1 a = 1/2 (reciprocal
+// square root), 2 a = 1.
+template <int AL> __device__ __forceinline__ float pow_less_one(float s, float a) {
+    const float ss = fmaxf(s, 1.17549435e-38f);
+    if constexpr (AL == 2) return 1.0f;
+    else if constexpr (AL == 1) return __builtin_amdgcn_rsqf(ss);
+    else return __builtin_amdgcn_exp2f((a - 1.0f) * __builtin_amdgcn_logf(ss));
+}
+template <int AL> __device__ __forceinline__ double pow_less_one(double s, double a) {
+    const double ss = s > 0.0 ? s : 1.0;
+    if constexpr (AL == 2) return 1.0;
+    else if constexpr (AL == 1) return rsqrt_nr<2>(ss);
+    else return dpow64(ss, a - 1.0);
+}
+
+// Generalized (src/unifrac_task_impl.hpp:1016-1024): num += l s^a |u - v| / s,
+// den += l s^a with s = u + v, both from the one power s^(a-1) (its error is
+// then the same in both and largely leaves the ratio).  Bound by VALU issue, the
+// transcendental a quarter of the add's rate: 4,000 samples x 1,930 dense nodes,
+// a = 1/2 in 3.7 ms (4.05 ms without the batches of 8, which hide the latency of
+// rsq), a = 1 in 1.4 ms, other a in 4.5 ms (batches do not help: 5.0).  32 x 64
+// pairs per wave with two powers per term: 1,777 samples 1.15 -> 0.64 ms at the
+// same split.
+template <class T, int AL> struct OpGen {
+    typedef T V;
+    static constexpr int RL = 4, EB = sizeof(T) == 4 ? 16 : 8, UNROLL = sizeof(T) == 4 ? 2 : 1, BATCH = sizeof(T) == 4 && AL == 1 ? 8 : 1;
+    static constexpr bool TWO = true, LEN = true, COUNTS = false, FLAGS = false;
+    static __device__ __forceinline__ T prep(T u) { return u; }
+    // BATCH pairs in step, so that one pair's power is computed while another's is under way
+    static __device__ __forceinline__ void terms(T u, const T* v, T l, T alpha, T* num, T* den) {
+        T s[BATCH], q[BATCH];
+#pragma unroll
+        for (int c = 0; c < BATCH; ++c) s[c] = u + v[c];
+        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < BATCH; ++c) q[c] = pow_less_one<AL>(s[c], alpha);
+        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < BATCH; ++c) {
+            num[c] = __builtin_elementwise_fma(__builtin_elementwise_abs(u - v[c]) * q[c], l, num[c]);
+            den[c] = __builtin_elementwise_fma(s[c] * q[c], l, den[c]);
+        }
+        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    static __device__ __forceinline__ double distance(double x, double y, double share, double share2, double, bool) {
+        return ratio(x, y, share, share2, true);
     }
 };
 
@@ -85,10 +148,12 @@ template <class OP> struct Shape {
     typedef typename OP::V V;
     static constexpr uint32_t ROWS = 16 * OP::RL;               // of a tile: two waves of 8 RL
     static constexpr uint32_t WAVE_ROWS = 8 * OP::RL;
-    static constexpr uint32_t NODE = ROWS + TILE_COLS;          // staged values of a node
+    static constexpr uint32_t NODE = ROWS + TILE_COLS;          // staged values of a node (and as many counts)
     static constexpr uint32_t PAIRS = OP::RL * 8;               // of a lane
+    static constexpr uint32_t SLOT = PAIRS * (OP::TWO ? 2 : 1) * 256;   // doubles of a workspace slot
     static constexpr bool MIXED = sizeof(V) == 4;
     static constexpr uint32_t G = 16 / sizeof(V);               // values of one 16-byte LDS read
+    static_assert(SLOT * sizeof(double) == TILE_SLOT, "every operation's slots have one size");
     // the lane's q-th row in its wave's rows (l = li), or column in its wave's 64 columns (l = lj)
     static __device__ __forceinline__ uint32_t at(uint32_t l, uint32_t q) { return q / G * (8 * G) + l * G + q % G; }
     // a lane's N values at(l, 0 .. N - 1) of a staged panel
@@ -105,11 +170,25 @@ template <class OP> struct Shape {
 
 // the distance of pair i < j, written to both triangles
 template <class OP>
-__device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j, double x) {
+__device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j, double x, double y) {
     typedef typename OP::V V;
     V* out = (V*)g.out;
-    const double share = g.add_partial ? (double)out[i * g.n + j] : 0.0;   // the rare nodes', from the posting walk
-    const double d = OP::distance(x, share, g.S[i] + g.S[j], g.normalized);
+    double share = 0.0, share2 = 0.0;   // the rare nodes', from the posting walk
+    if (g.add_partial) {
+        share = (double)out[i * g.n + j];
+        if constexpr (OP::TWO) share2 = (double)((const V*)g.out2)[i * g.n + j];
+    }
+    const double tot = OP::TWO ? 0.0 : g.S[i] + g.S[j];
+    const double d = OP::distance(x, y, share, share2, tot, g.normalized);
+    if constexpr (OP::FLAGS) {
+        // unnormalised: near-duplicates (distance below flag_tau of the pair's VAW
+        // denominator) marked for the FP64 recomputation
+        if (g.flags && d < (double)g.flag_tau * (y + share2)) {
+            g.flags[1 + i] = 1u;
+            g.flags[1 + j] = 1u;
+            atomicAdd(g.flags, 1u);
+        }
+    }
     out[i * g.n + j] = (V)d;
     out[j * g.n + i] = (V)d;
 }
@@ -119,7 +198,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
     typedef Shape<OP> SH;
     typedef typename OP::V V;
     constexpr int RL = OP::RL;
-    constexpr uint32_t EB = OP::EB;
+    constexpr uint32_t EB = OP::EB, PANELS = OP::COUNTS ? 2 : 1;
     const uint32_t seq = (blockIdx.x % N_XCDS) * g.per_xcd + blockIdx.x / N_XCDS;
     if (seq >= g.n_units) return;
     const uint32_t bij = g.units[seq].bij, part = g.units[seq].part;
@@ -127,7 +206,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
     const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
-    __shared__ __attribute__((aligned(16))) V sv[2][EB][SH::NODE];   // a node: its rows, then its columns
+    __shared__ __attribute__((aligned(16))) V sv[2][EB][PANELS][SH::NODE];   // a node: its rows, then its columns
     __shared__ V sl[2][EB];
 
     const uint32_t nd = g.dlist[0];
@@ -135,21 +214,35 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
     uint32_t ka, kb;
     part_range(nd, EB, (part >> 6) & 63u, np, ka, kb);
 
-    V num[RL][8];
-    double num64[SH::MIXED ? RL : 1][SH::MIXED ? 8 : 1];
+    V num[RL][8], den[OP::TWO ? RL : 1][OP::TWO ? 8 : 1];
+    double num64[SH::MIXED ? RL : 1][SH::MIXED ? 8 : 1], den64[SH::MIXED && OP::TWO ? RL : 1][SH::MIXED && OP::TWO ? 8 : 1];
 #pragma unroll
     for (int r = 0; r < RL; ++r)
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             num[r][c] = V(0);
+            if constexpr (OP::TWO) den[r][c] = V(0);
             if constexpr (SH::MIXED) num64[r][c] = 0.0;
+            if constexpr (SH::MIXED && OP::TWO) den64[r][c] = 0.0;
         }
 
     // wave w stages nodes w, w + 4, ..: 16 bytes per lane, rows then columns
     constexpr uint32_t VEC = 16 / sizeof(V), RLANES = SH::ROWS / VEC, CLANES = TILE_COLS / VEC;
-    const V* U = (const V*)g.U;
     const uint32_t* dl = g.dlist + 1;
     const uint32_t i0 = bi * SH::ROWS, j0 = bj * TILE_COLS;
+    V ti[OP::COUNTS ? RL : 1], tj[OP::COUNTS ? 8 : 1];   // the samples' totals
+    if constexpr (OP::COUNTS) {
+#pragma unroll
+        for (int r = 0; r < RL; ++r) {
+            const uint32_t i = i0 + wr + SH::at(li, r);
+            ti[r] = i < g.n ? (V)g.totals[i] : V(0);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t j = j0 + wc + SH::at(lj, c);
+            tj[c] = j < g.n ? (V)g.totals[j] : V(0);
+        }
+    }
     // the rows of the wave's nodes of the stage after the next one to be loaded, read ahead of their use
     uint32_t row_next[EB / 4];
     V len_next = V(0);
@@ -162,44 +255,62 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         }
         if constexpr (OP::LEN) len_next = threadIdx.x < EB ? (V)g.len[dl[min(k0 + threadIdx.x, kb - 1)]] : V(0);
     };
-    // stages nodes k0 .. (those past the end are zeros, which add nothing) and reads the indices of the next ones
+    // stages nodes k0 .. and reads the indices of the next ones
     auto stage = [&](int buf, uint32_t k0) __attribute__((always_inline)) {
 #pragma unroll
         for (uint32_t e = 0; e < EB / 4; ++e) {
             const uint32_t ee = wave + 4 * e;
-            const V* u = U + (size_t)row_next[e] * g.ldn;
-            V* to = &sv[buf][ee][0];
-            if constexpr (RLANES + CLANES <= 64) {
-                const V* src = u + (lane < RLANES ? i0 + lane * VEC : j0 + (lane - RLANES) * VEC);
-                if (RLANES + CLANES == 64 || lane < RLANES + CLANES)
-                    __builtin_amdgcn_global_load_lds(SSU_GLOBAL(src), SSU_LDS(to), 16, 0, 0);
-            } else {
-                static_assert(CLANES == 64 && RLANES <= 64, "a node is staged by one or two instructions");
-                if (RLANES == 64 || lane < RLANES)
-                    __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + i0 + lane * VEC), SSU_LDS(to), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + j0 + lane * VEC), SSU_LDS(to + SH::ROWS), 16, 0, 0);
+#pragma unroll
+            for (uint32_t p = 0; p < PANELS; ++p) {
+                const V* u = (const V*)(p ? g.C : g.U) + (size_t)row_next[e] * g.ldn;
+                V* to = &sv[buf][ee][p][0];
+                if constexpr (RLANES + CLANES <= 64) {
+                    const V* src = u + (lane < RLANES ? i0 + lane * VEC : j0 + (lane - RLANES) * VEC);
+                    if (RLANES + CLANES == 64 || lane < RLANES + CLANES)
+                        __builtin_amdgcn_global_load_lds(SSU_GLOBAL(src), SSU_LDS(to), 16, 0, 0);
+                } else {
+                    static_assert(CLANES == 64 && RLANES <= 64, "a node is staged by one or two instructions");
+                    if (RLANES == 64 || lane < RLANES)
+                        __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + i0 + lane * VEC), SSU_LDS(to), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds(SSU_GLOBAL(u + j0 + lane * VEC), SSU_LDS(to + SH::ROWS), 16, 0, 0);
+                }
             }
         }
         if constexpr (OP::LEN) if (threadIdx.x < EB) sl[buf][threadIdx.x] = len_next;
         if (k0 + EB < kb) index(k0 + EB);
     };
     auto node = [&](int buf, uint32_t e) __attribute__((always_inline)) {
-        V a[RL], b[8];
-        SH::read(a, &sv[buf][e][wr], li);
-        SH::read(b, &sv[buf][e][SH::ROWS + wc], lj);
+        V a[RL], b[8], ca[OP::COUNTS ? RL : 1], cb[OP::COUNTS ? 8 : 1];
+        SH::read(a, &sv[buf][e][0][wr], li);
+        SH::read(b, &sv[buf][e][0][SH::ROWS + wc], lj);
+        if constexpr (OP::COUNTS) {
+            SH::read(ca, &sv[buf][e][PANELS - 1][wr], li);
+            SH::read(cb, &sv[buf][e][PANELS - 1][SH::ROWS + wc], lj);
+        }
+#pragma unroll
+        for (int r = 0; r < RL; ++r) a[r] = OP::prep(a[r]);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) b[c] = OP::prep(b[c]);
         const V l = OP::LEN ? sl[buf][e] : V(0);
-        V none = V(0);
+        const V alpha = (V)g.alpha;
 #pragma unroll
         for (int r = 0; r < RL; ++r)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) OP::term(a[r], b[c], l, num[r][c], none);
+            for (int c = 0; c < 8; c += OP::BATCH) {
+                if constexpr (OP::TWO) OP::terms(a[r], b + c, l, alpha, num[r] + c, den[r] + c);
+                else OP::term(a[r], b[c], l, num[r][c]);
+            }
     };
     auto merge = [&]() __attribute__((always_inline)) {
         if constexpr (SH::MIXED) {
 #pragma unroll
             for (int r = 0; r < RL; ++r)
 #pragma unroll
-                for (int c = 0; c < 8; ++c) { num64[r][c] += (double)num[r][c]; num[r][c] = V(0); }
+                for (int c = 0; c < 8; ++c) {
+                    num64[r][c] += (double)num[r][c];
+                    num[r][c] = V(0);
+                    if constexpr (OP::TWO) { den64[r][c] += (double)den[r][c]; den[r][c] = V(0); }
+                }
         }
     };
 
@@ -211,12 +322,12 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         uint32_t span = 0;
         for (uint32_t k0 = ka; k0 < kb; k0 += EB) {
             if (k0 + EB < kb) stage(buf ^ 1, k0 + EB);
-            else if (k0 + EB > kb) {   // (uniform) the last, partial stage: its missing nodes zero
-                for (uint32_t q = (kb - k0) * SH::NODE + threadIdx.x; q < EB * SH::NODE; q += 256)
-                    (&sv[buf][0][0])[q] = V(0);
+            else if (k0 + EB > kb) {   // (uniform) the last, partial stage: its missing nodes zero, which add nothing
+                for (uint32_t q = (kb - k0) * PANELS * SH::NODE + threadIdx.x; q < EB * PANELS * SH::NODE; q += 256)
+                    (&sv[buf][0][0][0])[q] = V(0);
                 __syncthreads();
             }
-#pragma unroll
+#pragma unroll OP::UNROLL
             for (uint32_t e = 0; e < EB; ++e) node(buf, e);
             span += EB;
             if (span == MERGE) { merge(); span = 0; }
@@ -226,14 +337,20 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         merge();
     }
 
+    auto sum = [&](int r, int c) { if constexpr (SH::MIXED) return num64[r][c]; else return num[r][c]; };
+    auto sum2 = [&](int r, int c) {
+        if constexpr (!OP::TWO) return 0.0;
+        else if constexpr (SH::MIXED) return den64[r][c];
+        else return den[r][c];
+    };
     if (np > 1) {   // this part's sums to its slot, [pair of the lane][thread], for k_tiles_finish
-        double* w = g.ws + (size_t)(part >> 12) * (SH::PAIRS * 256) + threadIdx.x;
+        double* w = g.ws + (size_t)(part >> 12) * SH::SLOT + threadIdx.x;
 #pragma unroll
         for (int r = 0; r < RL; ++r)
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                if constexpr (SH::MIXED) w[(r * 8 + c) * 256] = num64[r][c];
-                else w[(r * 8 + c) * 256] = num[r][c];
+                w[(r * 8 + c) * 256] = sum(r, c);
+                if constexpr (OP::TWO) w[(SH::PAIRS + r * 8 + c) * 256] = sum2(r, c);
             }
         return;
     }
@@ -242,10 +359,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const size_t i = i0 + wr + SH::at(li, r), j = j0 + wc + SH::at(lj, c);
-            double x;
-            if constexpr (SH::MIXED) x = num64[r][c];
-            else x = num[r][c];
-            if (i < j && j < g.n) write_pair<OP>(g, i, j, x);
+            if (i < j && j < g.n) write_pair<OP>(g, i, j, sum(r, c), sum2(r, c));
             else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
         }
 }
@@ -260,18 +374,21 @@ __global__ void __launch_bounds__(256) k_tiles_finish(TileArgs g) {
     const uint32_t bi = bij >> 16, bj = bij & 0xffffu, np = (part & 63u) + 1, r = blockIdx.y;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
-    const double* w = g.ws + (size_t)(part >> 12) * (SH::PAIRS * 256) + threadIdx.x;
-    double x[8];
+    const double* w = g.ws + (size_t)(part >> 12) * SH::SLOT + threadIdx.x;
+    double x[8], y[8];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) x[c] = 0.0;
+    for (int c = 0; c < 8; ++c) x[c] = y[c] = 0.0;
 #pragma unroll 2
     for (uint32_t p = 0; p < np; ++p)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) x[c] += w[(size_t)p * (SH::PAIRS * 256) + (r * 8 + c) * 256];
+        for (int c = 0; c < 8; ++c) {
+            x[c] += w[(size_t)p * SH::SLOT + (r * 8 + c) * 256];
+            if constexpr (OP::TWO) y[c] += w[(size_t)p * SH::SLOT + (SH::PAIRS + r * 8 + c) * 256];
+        }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         const size_t i = bi * SH::ROWS + wr + SH::at(li, r), j = bj * TILE_COLS + wc + SH::at(lj, c);
-        if (i < j && j < g.n) write_pair<OP>(g, i, j, x[c]);
+        if (i < j && j < g.n) write_pair<OP>(g, i, j, x[c], y[c]);
         else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
     }
 }
@@ -385,7 +502,8 @@ hipError_t launch_dense_list(uint32_t* dlist, const uint32_t* dmask, uint32_t K,
 template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_t st) {
     constexpr uint32_t rows = Shape<OP>::ROWS;
     if (!a.n || !a.n_units) return hipSuccess;   // (a selection without a tile here)
-    if (!a.U || !a.dlist || !a.out || !a.units || !a.S || a.ldn % TILE_COLS || a.ldn < a.n ||
+    if (!a.U || !a.dlist || !a.out || !a.units || (OP::TWO ? a.add_partial && !a.out2 : !a.S) ||
+        (OP::COUNTS && (!a.C || !a.totals)) || (sizeof(typename OP::V) == 8 && !a.rows) || a.ldn % TILE_COLS || a.ldn < a.n ||
         a.ldn % rows || (a.n + rows - 1) / rows > 65535 || (a.n_split && (!a.split || !a.ws)) || (OP::LEN && !a.len))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_tiles<OP>, dim3(a.per_xcd * N_XCDS), dim3(256), 0, st, a);
@@ -394,8 +512,16 @@ template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_
 }
 
 hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st) {
-    if (fp64 && !a.rows) return hipErrorInvalidValue;
     return fp64 ? launch_tiles<OpW64>(a, st) : launch_tiles<OpW32>(a, st);
+}
+
+template <class T> static hipError_t launch_gen(const TileArgs& a, hipStream_t st) {
+    if (a.alpha == 0.5) return launch_tiles<OpGen<T, 1>>(a, st);
+    if (a.alpha == 1.0) return launch_tiles<OpGen<T, 2>>(a, st);
+    return launch_tiles<OpGen<T, 0>>(a, st);
+}
+hipError_t launch_tiles_generalized(bool fp64, const TileArgs& a, hipStream_t st) {
+    return fp64 ? launch_gen<double>(a, st) : launch_gen<float>(a, st);
 }
 
 }  // namespace ssu

@@ -50,15 +50,22 @@ struct TileArgs {
     const double* S;          // per-sample sums
     bool normalized;
     void* out;                // n x n, the operand's type
-    bool add_partial;         // out[i * n + j], i < j, holds the rare nodes' share
-    double* ws;               // workspace slots of rows * TILE_COLS doubles
+    bool add_partial;         // out[i * n + j] (and out2), i < j, hold the rare nodes' shares
+    const void* out2;         // two sums: the denominator's share
+    double alpha;             // generalized
+    const void* C;            // VAW: count rows, as U
+    const double* totals;     // VAW: the samples' totals
+    uint32_t* flags;          // unnormalised VAW weighted: marks of near-duplicates (below
+    float flag_tau;           //   flag_tau of the pair's VAW denominator), as launch_flag_close's
+    double* ws;               // workspace slots of TILE_SLOT bytes
     const TileUnit* units;
     uint32_t n_units, per_xcd;
     const TileUnit* split;
     uint32_t n_split;
 };
-constexpr uint32_t TILE_ROWS_W = 128;      // rows per tile of the weighted kernels
-constexpr size_t TILE_SLOT_W = size_t(TILE_ROWS_W) * TILE_COLS * sizeof(double);   // bytes of one workspace slot
+constexpr uint32_t TILE_ROWS_W = 128;      // rows per tile: one sum per pair (weighted)
+constexpr uint32_t TILE_ROWS_2 = 64;       // two sums per pair (generalized)
+constexpr size_t TILE_SLOT = size_t(128) * 128 * sizeof(double);   // bytes of one workspace slot
 constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD (32 CUs) holds at 2 waves per SIMD
 
 // Weighted.  FP32: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
@@ -66,6 +73,8 @@ constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD 
 // FP64: x = S_i + S_j - 2 M in its place, M = sum of l min(u_i, u_j) + the rare
 // share, U the embedding (row rows[r] for processed node r).
 hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st);
+// Generalized, 0 <= alpha <= 1: numerator over denominator, each with its share
+hipError_t launch_tiles_generalized(bool fp64, const TileArgs& a, hipStream_t st);
 
 // dlist from the dense mask ([ceil(K / 32)] words): dlist[0] = their number,
 // then the set bits in increasing order

@@ -11,7 +11,7 @@ namespace {
 // three thresholds each on the 16,384-sample (100k tips) and 8,192-sample
 // (50k tips) workloads (total = fixed + terms * term + postings * posting); the
 // modelled optimum lands within the measured one for every kind (weighted
-// 0.193 vs 0.2, FP64 weighted 0.24 vs 0.23 - 0.3, generalized 0.738 vs 0.8,
+// 0.193 vs 0.2, FP64 weighted 0.24 vs 0.23 - 0.3, generalized 0.38 vs 0.4,
 // Gram 0.075 vs 0.06 - 0.1).  The per-term cost includes the list building
 // and row lists, whose work follows the postings.
 struct Rates {
@@ -20,7 +20,7 @@ struct Rates {
     double onesided = 0.0;   // VAW: one (posting slot, total) one-sided term
 };
 
-Rates rates_of(SplitKind k) {
+Rates rates_of(SplitKind k, double alpha) {
     switch (k) {
     // 16,384 samples, theta 0.14 .. 0.26: tiles 70.1 .. 42.6 ms, posting phase 29.1 .. 56.5 ms,
     // device total 115.1, 111.6 (0.17), 111.2 (0.2), 112.5 (0.23), 115.0 ms
@@ -28,12 +28,18 @@ Rates rates_of(SplitKind k) {
     // 3,001 samples (20k tips), theta 0.1 / 0.23 / 0.4: tiles 2.91 / 1.62 / 1.01 ms, posting
     // phase 0.54 / 1.09 / 1.96 ms, device total 4.20 / 3.46 / 3.73 ms (0.3: 3.50)
     case SplitKind::weighted64: return {8.2e-14, 1.42e-12};
-    case SplitKind::generalized32: return {6.0e-13, 1.1e-12};
+    // 4,000 samples (20k tips), theta 0.2 .. 0.6: tiles 8.29 .. 3.03 ms (alpha 1/2: reciprocal
+    // square roots), 9.94 .. 3.74 (0.3: log2 and exp2), 3.14 .. 1.14 (1: no power), posting
+    // phase 1.73 .. 6.20 ms; best totals at 0.4 (9.39 ms), 0.5 (10.5) and 0.2 - 0.3 (5.9)
+    case SplitKind::generalized32: return {alpha == 1.0 ? 8.5e-14 : alpha == 0.5 ? 2.25e-13 : 2.65e-13, 1.57e-12};
     case SplitKind::gram: return {3.4e-15, 6.1e-13};
-    // FP64 generalized (an FP64 power and division per tile term, two powers per
-    // posting): fitted to the 8,192-sample workload at theta 0.5 / 0.707 / 0.9
-    // (within 2% of each phase's measured time)
-    case SplitKind::generalized64: return {7.7e-12, 7.5e-12};
+    // FP64 generalized, 1,200 samples, theta 0.2 .. 0.6: alpha 1/2 tiles 2.54 .. 0.90 ms, posting
+    // phase 0.58 .. 1.55 (totals 3.51, 2.83 at 0.4 - 0.6); other alpha (an FP64 power per tile
+    // term, two per posting) 8.07 .. 2.84 and 1.01 .. 3.28 (totals 9.47, 6.5 at 0.6); alpha 1
+    // takes no power on the tiles
+    case SplitKind::generalized64:
+        if (alpha == 0.5) return {6.7e-13, 3.8e-12};
+        return {alpha == 1.0 ? 2.0e-13 : 2.15e-12, 8.8e-12};
     // VAW: the dense kernel's term over the dense nodes' rows; a posting (three
     // FP64 reciprocal square roots); a one-sided term at one total.  Fitted to the
     // 8,192-sample workload at theta 0.25 / 0.5 / 1 (weighted and presence terms
@@ -44,36 +50,22 @@ Rates rates_of(SplitKind k) {
     return {1.0, 1.0};
 }
 
-// expected tiled-kernel terms of a node held by c of n samples, placed at
-// random: the pair blocks visit a node either of their sample panels holds
-// (the kernels' counts agree within 1% on the workloads above); a Gram
-// column, a VAW node and a node of the weighted tiles cost every pair
-double tile_terms(SplitKind k, uint32_t n, uint32_t c) {
-    const double pairs = 0.5 * (double)n * n;
-    if (k == SplitKind::gram || k == SplitKind::vaw32 || k == SplitKind::vaw64 || k == SplitKind::weighted32 ||
-        k == SplitKind::weighted64)
-        return pairs;
-    const double q = 1.0 - (double)c / n;   // a given sample lacks the node
-    const double q2 = q * q, q4 = q2 * q2, q8 = q4 * q4, q16 = q8 * q8, q32 = q16 * q16;
-    return pairs * (1.0 - q32 * q32 * q32);   // 1 - q^96
-}
-
 }  // namespace
 
 SplitChoice choose_split(SplitKind kind, uint32_t n, const std::vector<uint32_t>& occupancy, uint64_t max_slots,
-                         uint32_t cols) {
+                         uint32_t cols, double alpha) {
     SplitChoice best;
     if (n < 2 || occupancy.empty()) return best;
-    const Rates r = rates_of(kind);
+    const Rates r = rates_of(kind, alpha);
     // nodes by occupancy (0: held by no sample, no cost either way); an
     // occupancy above n (never, for counts of n samples) counts as n
     std::vector<uint64_t> hist((size_t)n + 1, 0);
     for (uint32_t x : occupancy) ++hist[std::min(x, n)];
     // cost with every node on the tiles; then move nodes to the posting lists in
     // increasing occupancy (thr = c + 1 moves every node held by at most c samples)
+    const double pairs = 0.5 * (double)n * n;   // a node on the tiles costs every pair
     double tiles = 0.0;
-    for (uint32_t c = 1; c <= n; ++c)
-        if (hist[c]) tiles += (double)hist[c] * tile_terms(kind, n, c) * r.term;
+    for (uint32_t c = 1; c <= n; ++c) tiles += (double)hist[c] * pairs * r.term;
     best.model_ms_none = best.model_ms = tiles * 1e3;
     double cost = tiles, posts = 0.0;
     uint64_t slots = 0;
@@ -81,7 +73,7 @@ SplitChoice choose_split(SplitKind kind, uint32_t n, const std::vector<uint32_t>
         if (!hist[c]) continue;
         if (c > 0) {
             const double m = (double)hist[c], x = c;
-            cost -= m * tile_terms(kind, n, c) * r.term;
+            cost -= m * pairs * r.term;
             posts += m * (0.5 * x * (x - 1.0) * r.posting + x * (double)cols * r.onesided);
             slots += hist[c] * c;
         }

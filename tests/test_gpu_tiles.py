@@ -15,6 +15,10 @@ OPS = [("weighted_normalized", {}), ("weighted_unnormalized", {}), ("weighted_no
        ("weighted_unnormalized_fp64", {}), ("generalized", {"alpha": 0.5}), ("generalized", {"alpha": 1.0}),
        ("generalized", {"alpha": 0.3}), ("generalized", {"alpha": 0.0}), ("generalized_fp64", {"alpha": 0.5}),
        ("generalized_fp64", {"alpha": 1.0}), ("generalized_fp64", {"alpha": 0.3})]
+VAW = {"variance_adjust": True}
+OPS += [(m + p, dict(VAW, **k)) for p in ("", "_fp64")
+        for m, k in (("weighted_normalized", {}), ("weighted_unnormalized", {}), ("unweighted", {}),
+                     ("generalized", {"alpha": 0.5}), ("generalized", {"alpha": 1.0}), ("generalized", {"alpha": 0.3}))]
 
 
 @pytest.fixture(scope="module", autouse=True)

@@ -450,15 +450,12 @@ struct PlanImpl {
     bool sparse = false;             // weighted (or generalized) through the shared-node kernels
     bool gen = false;                // generalized on the shared-node path
     // VAW on the shared-node path: nodes held by at least split_thr samples of the
-    // plan's table (vdense_mask) stay with the dense pair kernel (its rows vrows,
-    // lengths vlen_*), the others go to the posting lists; the one-sided sums are
+    // plan's table (vdense_mask) stay with the pair tiles (vdense: their number, then
+    // their indices), the others go to the posting lists; the one-sided sums are
     // taken at the table's distinct totals tau_h (sample s at kidx_h[s])
     bool vsplit = false;
-    uint32_t n_vdense = 0;
-    std::vector<uint32_t> vdense_mask, kidx_h;
-    std::vector<int32_t> vrows;
-    std::vector<float> vlen_f;
-    std::vector<double> vlen_d, tau_h;
+    std::vector<uint32_t> vdense_mask, vdense, kidx_h;
+    std::vector<double> tau_h;
     uint32_t split_thr = 0;          // FP32 shared-node path: nodes held by fewer samples use posting lists (0: off)
     double split_theta = 0.0;        // the occupancy split chosen (threshold / n; 0: none)
     uint32_t split_slots = 0;        // bound on their postings in any execution
@@ -477,10 +474,10 @@ struct PlanImpl {
     bool bits = false;
     uint32_t ldb = 0;
     std::vector<uint32_t> block_order;  // pair blocks / Gram tiles in launch order
-    // pair tiles over the dense nodes (weighted, generalized): the work list of the full
+    // pair tiles over the dense nodes (weighted, generalized, VAW): the work list of the full
     // matrix, a stripe selection's, and the output bands'
     bool tiled = false;
-    uint32_t tile_rows() const { return gen ? TILE_ROWS_2 : TILE_ROWS_W; }
+    uint32_t tile_rows() const { return gen || vsplit ? TILE_ROWS_2 : TILE_ROWS_1; }
     uint32_t n_dense_max = 0;        // the most dense nodes an execution can have
     TileSet tset, tset_run;
     struct TileBand { uint32_t unit0, n_units, per_xcd, split0, n_split; };
@@ -553,7 +550,7 @@ struct PlanImpl {
         d_faith, d_stripes, d_smask, d_dmask, d_pc, d_pidx, d_pval, d_walked, d_rows, d_rcount, d_roff, d_rbsum,
         d_sp_node, d_sp_len, d_B, d_poff, d_pcnt, d_obsum, d_Ssp, d_out2, d_pspmax, d_urare, d_close,
         d_ridx, d_dlist, d_units, d_split, d_units_run, d_split_run, d_units_band, d_split_band, d_tws, d_udense,
-        d_order_run, d_order_band, d_vdense, d_vrows, d_vlen, d_tau, d_kidx, d_H, d_pcv, d_nbound;
+        d_order_run, d_order_band, d_vdense, d_tau, d_kidx, d_H, d_pcv, d_nbound;
 
     hipStream_t own_st = nullptr;    // created with the plan; st may point at a caller's stream
     // per-execution inputs and output (nullptr: the plan's own table data / totals / result)
@@ -820,7 +817,7 @@ bool PlanImpl::upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std:
 
 // VAW on the shared-node path: nodes held by fewer than theta * n samples of the
 // plan's table (structural occupancy: no execution holds more) are summed from
-// posting lists, the others by the dense pair kernel, decided once here.  The
+// posting lists, the others on the pair tiles, decided once here.  The
 // one-sided sums are taken at the table's distinct totals (an execution with
 // totals of its own takes them at every sample's).  The [n][D] sums must fit
 // VAW_H_BUDGET; SSU_VAW_SPLIT sets theta (0: off).
@@ -855,26 +852,16 @@ bool PlanImpl::split_vaw(std::string* err) {
     split_thr = thr;
     split_slots = (uint32_t)std::max<uint64_t>(slots, 1);
     vdense_mask.assign((K + 31) / 32, 0u);
-    vrows.clear();
-    vlen_f.clear();
-    vlen_d.clear();
+    vdense.assign(1, 0u);
     for (uint32_t q = 0; q < K; ++q) {
         if (cnt[q] < thr) continue;
         vdense_mask[q >> 5] |= 1u << (q & 31);
-        vrows.push_back(spec.fp64 ? knodes[q] : (int32_t)q);   // FP64: embedding rows; FP32: operand rows
-        if (spec.fp64) vlen_d.push_back(klen_d[q]);
-        else vlen_f.push_back(klen_f[q]);
+        vdense.push_back(q);
     }
-    n_vdense = (uint32_t)vrows.size();
-    if (vrows.empty()) {   // (uploads of one padding row; the kernel takes n_vdense = 0 rows)
-        vrows.push_back(0);
-        if (spec.fp64) vlen_d.push_back(0.0);
-        else vlen_f.push_back(0.0f);
-    }
+    vdense[0] = n_dense_max = (uint32_t)vdense.size() - 1;
     vsplit = true;
     // (members: the host copies outlive the uploads)
-    return upload(d_vdense, vdense_mask, st, err) && upload(d_vrows, vrows, st, err) &&
-           (spec.fp64 ? upload(d_vlen, vlen_d, st, err) : upload(d_vlen, vlen_f, st, err)) &&
+    return upload(d_vdense, vdense_mask, st, err) && upload(d_dlist, vdense, st, err) &&
            upload(d_tau, tau_h, st, err) && upload(d_kidx, kidx_h, st, err);
 }
 
@@ -1244,7 +1231,6 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
         ok = upload(P.d_klen_sum, ls, P.st, err);
     }
     // 6 x 6 super-tiles of 128-sample Gram tiles: about the number of tiles resident on one XCD
-    P.tiled = P.sparse;
     if (ok && P.gram) {
         P.block_order = upper_block_order((uint32_t)(P.n_pad / GRAM_BM), 6);
         ok = upload(P.d_order, P.block_order, P.st, err);
@@ -1253,6 +1239,8 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
     if (ok && P.gram) ok = P.split_gram(err);   // builds the Gram columns (narrowed when it splits)
     if (ok && P.gram && P.col_node.empty() && !P.build_gram_columns()) ok = false;
     if (ok && P.sparse) ok = P.split_weighted(err);
+    if (ok && P.vsplit) ok = P.split_vaw(err);
+    P.tiled = P.sparse || P.vsplit;
     if (ok && P.tiled) {
         const uint32_t K = (uint32_t)P.knodes.size();
         if (!P.split_thr) {   // no split: every node is dense
@@ -1261,10 +1249,9 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
             for (uint32_t q = 0; q < K; ++q) all[q + 1] = q;
             ok = upload(P.d_dlist, all, P.st, err) && hipStreamSynchronize(P.st) == hipSuccess;
         }
-        P.tset = tile_set(P.n, P.tile_rows(), P.n_dense_max, TILE_RESIDENT);
+        P.tset = tile_set(P.n, P.tile_rows(), P.n_dense_max);
         ok = ok && P.upload_tiles(P.tset, P.d_units, P.d_split, err);
     }
-    if (ok && P.vsplit) ok = P.split_vaw(err);
     step("occupancy split");
     if (ok && P.gram && P.Kp)
         ok = upload(P.d_col, P.col_node, P.st, err) && upload(P.d_digits, P.digits, P.st, err) &&
@@ -1381,7 +1368,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                       P.d_sp_node.as<int32_t>(), Ks, npan, P.st));
     }
     if (P.tiled && ((split && !P.d_dlist.ensure(((size_t)K + 1) * sizeof(uint32_t), err)) ||
-                    !P.d_tws.ensure(std::max<size_t>(P.tset.slots * TILE_SLOT, 1), err)))
+                    !P.d_tws.ensure(std::max<size_t>(P.tset.slots * tile_slot_bytes(P.tile_rows()), 1), err)))
         return false;
     // one embedding block (E holds every sample): the postings of the FP32 split take their
     // values from E, and the gather skips the operand rows of nodes that are never dense
@@ -1404,7 +1391,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                        P.d_Spart.as<double>(), split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
                                        split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.tiled && gather && !P.gen));
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.sparse && gather && !P.gen));
             if (gather && s.vaw)
                 SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
                                            (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st));
@@ -1447,7 +1434,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.out2 = P.gen || vsplit ? P.d_out2.p : nullptr;
         b.pspmax = P.gen ? P.d_pspmax.as<double>() : nullptr;
         b.band = P.band;
-        if (P.tiled) {
+        if (P.sparse) {
             b.dlist = P.d_dlist.as<uint32_t>();
             if (gather && !P.gen && !skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
         }
@@ -1491,6 +1478,20 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
     }
     SSU_HIP(P.mark(2));
 
+    // unnormalised VAW weighted: the pair kernel marks the near-duplicates itself
+    auto mark_vaw = [&](auto& a) -> bool {
+        if (!P.refine_vaw) return true;
+        uint32_t* vf = d_flags;
+        if (!vf && !quiet) {
+            if (!P.d_close.ensure(((size_t)P.n + 1) * sizeof(uint32_t), err)) return false;
+            vf = P.d_close.as<uint32_t>();
+        }
+        if (!vf) return true;
+        SSU_HIP(launch_fill_u32(vf, (size_t)P.n + 1, 0u, P.st));
+        a.flags = vf;
+        a.flag_tau = P.refine_tau;
+        return true;
+    };
     const bool norm = s.method == Method::unweighted;
     auto combine = [&](uint32_t r0, uint32_t r1) {
         return s.fp64 ? launch_unweighted_combine<double>((double*)P.out_ptr(), P.d_G.as<double>(), P.n_pad, P.n,
@@ -1556,6 +1557,14 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         a.add_partial = split;
         a.out2 = P.d_out2.p;
         a.alpha = s.alpha;
+        int vaw = 0;   // the kind of VAW terms
+        if (vsplit) {
+            vaw = s.method == Method::generalized ? 3 : op == PairOp::vaw_unweighted ? 2 : 1;
+            a.normalized = normalized;
+            a.C = s.fp64 ? P.d_C.p : P.d_Cu.p;
+            a.totals = P.totals_ptr();
+        }
+        if (!mark_vaw(a)) return false;
         a.ws = P.d_tws.as<double>();
         const uint32_t nbands = P.banded_run ? (uint32_t)P.band_ev.size() : 1;
         if (P.banded_run && nbands > 1) {
@@ -1580,7 +1589,9 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                 a.split = (P.band_all ? P.d_split : P.d_split_run).as<TileUnit>();
                 a.n_split = (uint32_t)t.split.size();
             }
-            SSU_HIP(P.gen ? launch_tiles_generalized(s.fp64, a, bs) : launch_tiles_weighted(s.fp64, a, bs));
+            SSU_HIP(vaw     ? launch_tiles_vaw(vaw, s.fp64, a, bs)
+                    : P.gen ? launch_tiles_generalized(s.fp64, a, bs)
+                            : launch_tiles_weighted(s.fp64, a, bs));
             if (P.banded_run) SSU_HIP(hipEventRecord(P.band_ev[k], bs));
         }
         if (P.banded_run && nbands > 1)   // the later work on st reads every band
@@ -1609,25 +1620,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             a.Cn = s.vaw ? P.d_Cu.p : nullptr;
             a.rows = nullptr;
         }
-        if (vsplit) {   // the dense nodes only, plus the posting-list shares
-            a.rows = P.d_vrows.as<int32_t>();
-            a.len = P.d_vlen.p;
-            a.K = P.n_vdense;
-            a.out2 = P.d_out2.p;
-            a.len_nonneg = true;   // (the split needs every length finite and >= 0)
-        }
-        if (P.refine_vaw) {   // the kernel marks the near-duplicates itself
-            uint32_t* vf = d_flags;
-            if (!vf && !quiet) {
-                if (!P.d_close.ensure(((size_t)P.n + 1) * sizeof(uint32_t), err)) return false;
-                vf = P.d_close.as<uint32_t>();
-            }
-            if (vf) {
-                SSU_HIP(launch_fill_u32(vf, (size_t)P.n + 1, 0u, P.st));
-                a.flags = vf;
-                a.flag_tau = P.refine_tau;
-            }
-        }
+        if (!mark_vaw(a)) return false;
         SSU_HIP(launch_pairs(op, s.fp64, a, P.st));
         SSU_HIP(P.mark(3));
         SSU_HIP(P.mark(4));
@@ -1748,7 +1741,7 @@ bool Plan::execute_to_host(void* host, std::string* err) {
     // paths write their output in one final pass)
     static const bool off = getenv("SSU_OUT_BANDS") && atoi(getenv("SSU_OUT_BANDS")) == 0;
     const bool gram_bands = P.gram && P.Kp;   // (no Gram columns: one fill, nothing to band)
-    if (off || !(P.sparse || gram_bands) || !P.band_all || P.n < 4096 ||
+    if (off || !(P.tiled || gram_bands) || !P.band_all || P.n < 4096 ||
         (P.tiled ? P.tset.units.empty() : P.block_order.empty()))
         return execute(err) && copy_matrix(host, err);
     if (!P.prepare_bands(err)) return false;
@@ -1759,7 +1752,7 @@ bool Plan::execute_to_host(void* host, std::string* err) {
         const size_t n = P.n, pitch = n * es;
         for (size_t k = 0; k < P.band_ev.size(); ++k) {
             const size_t r0 = P.band_row0[k], r1 = P.band_row0[k + 1];
-            if (P.sparse || P.gram) {
+            if (P.tiled || P.gram) {
                 // band k writes every pair (i, j), i < j, of its rows i and the mirror
                 // (j, i) (the tiled kernel's blocks; the Gram path's banded combine):
                 // once it is done, its rows from column r0 on and the columns [r0, r1)
@@ -1824,8 +1817,8 @@ bool Plan::set_stripes(uint32_t start, uint32_t stop, std::string* err) {
     if (P.tiled) {
         P.tset_run = tile_subset(P.tset, [&](uint32_t bi, uint32_t bj) {
             const uint32_t tr = P.tile_rows();
-            return P.band.meets_tile(bi * tr, std::min(P.n, (bi + 1) * tr), bj * TILE_COLS,
-                                     std::min(P.n, (bj + 1) * TILE_COLS));
+            return P.band.meets_tile(bi * tr, std::min(P.n, (bi + 1) * tr), bj * tr,
+                                     std::min(P.n, (bj + 1) * tr));
         });
         return P.upload_tiles(P.tset_run, P.d_units_run, P.d_split_run, err);
     }
@@ -1988,13 +1981,13 @@ uint64_t Plan::kernel_terms() const {
     if (P.tiled) {
         uint32_t nd = 0;
         if (!P.d_dlist.p || hipMemcpy(&nd, P.d_dlist.p, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess) return 0;
-        return (P.band_all ? P.tset : P.tset_run).tiles * P.tile_rows() * TILE_COLS * nd;
+        return (P.band_all ? P.tset : P.tset_run).tiles * P.tile_rows() * P.tile_rows() * nd;
     }
     // dense tiles: 128 x 128 for weighted / plain unweighted, 64 x 64 for generalized and VAW
     const bool small = P.spec.vaw || P.spec.method == Method::generalized;
     const uint64_t edge = small ? 64 : PAIR_TILE;
     const uint64_t t = (P.n + edge - 1) / edge;
-    return t * (t + 1) / 2 * edge * edge * (P.vsplit ? (uint64_t)P.n_vdense : K);
+    return t * (t + 1) / 2 * edge * edge * K;
 }
 uint64_t Plan::sparse_terms() const {
     const PlanImpl& P = *p_;

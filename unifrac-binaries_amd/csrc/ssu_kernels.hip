@@ -764,14 +764,11 @@ template <PairOp OP> struct PairTraits {
 };
 
 // Per-node term for one pair.  u, v: embedded values; cu, cv: embedded counts
-// (VAW); m: c_k + c_l sample totals (VAW); l: branch length.  LPRE (VAW
-// presence terms, and FP64 weighted terms; lengths >= 0): u and v arrive
-// multiplied by l, so l |u - v| = |lu - lv| and l (u + v) = lu + lv
-// (presence: l max(u, v) = max(lu, lv), exact for 0/1 values).
+// (VAW); m: c_k + c_l sample totals (VAW); l: branch length.
 // PW (FP32 generalized powers): 0 the hardware exp2(a log2 s), 1 the exponent of s kept
 // exact (pow_alpha2_split, alpha outside [0, 1]), 2 alpha = 1/2 by the hardware square
 // root and reciprocal square root (1 ulp each, and one instruction fewer than 0)
-template <PairOp OP, class T, bool LPRE = false, int PW = 0>
+template <PairOp OP, class T, int PW = 0>
 __device__ __forceinline__ void pair_term(T u, T v, T cu, T cv, T m, T l, T alpha, T& num, T& den) {
     if constexpr (OP == PairOp::weighted) {
         // src/unifrac_task_impl.hpp:117-127
@@ -816,10 +813,7 @@ __device__ __forceinline__ void pair_term(T u, T v, T cu, T cv, T m, T l, T alph
         T rv;
         if constexpr (sizeof(T) == 4) rv = ok ? __builtin_amdgcn_rsqf(vv) : 0.0f;
         else rv = ok ? T(1) / dsqrt<T>(vv) : T(0);
-        if constexpr (OP == PairOp::vaw_weighted && LPRE) {
-            num = fma(dabs(u - v), rv, num);
-            den = fma(u + v, rv, den);
-        } else if constexpr (OP == PairOp::vaw_weighted) {
+        if constexpr (OP == PairOp::vaw_weighted) {
             num = fma(dabs(u - v) * l, rv, num);
             den = fma((u + v) * l, rv, den);
         } else if constexpr (OP == PairOp::vaw_generalized) {
@@ -847,9 +841,6 @@ __device__ __forceinline__ void pair_term(T u, T v, T cu, T cv, T m, T l, T alph
                 num = fma(w, d1 / ss, num);
                 den += w;
             }
-        } else if constexpr (LPRE) {   // vaw_unweighted: u, v are l or 0
-            num = fma(dabs(u - v), rv, num);
-            den = fma(u > v ? u : v, rv, den);
         } else {  // vaw_unweighted: u, v are 0/1 presence values
             const T lv = l * rv;
             num = fma(dabs(u - v), lv, num);
@@ -867,15 +858,12 @@ template <class T> struct PairStage { static constexpr int EB = sizeof(T) == 4 ?
 // of both 128-sample panels (and of the count panels for VAW) are staged in
 // LDS per step; the next step's rows are prefetched into registers while the
 // current one is consumed, and LDS is double-buffered (one barrier per step).
-// add_partial (two-accumulator ops): out[i * n + j] and out2[i * n + j], i < j,
-// hold the posting-list shares of the numerator and the denominator, added
-// before the division; each pair is then written by its i < j thread alone.
-template <PairOp OP, class T, int RI, int RJ, int TT, bool LPRE = false, int PW = 0>
+template <PairOp OP, class T, int RI, int RJ, int TT, int PW = 0>
 __global__ void __launch_bounds__((TT / RI) * (TT / RJ))
 k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __restrict__ rows, size_t ldn,
         const T* __restrict__ len, uint32_t K,
         uint32_t n, const double* __restrict__ S, const double* __restrict__ totals, double alpha_d, int normalized,
-        void* __restrict__ out_v, int out_fp64, GapBand band, int add_partial, const void* __restrict__ out2_v,
+        void* __restrict__ out_v, int out_fp64, GapBand band,
         uint32_t* __restrict__ flags, float flag_tau) {
     constexpr int NTI = TT / RI, NTJ = TT / RJ, NT = NTI * NTJ;
     constexpr bool TWO = PairTraits<OP>::two;
@@ -923,7 +911,6 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
 
     vecT pre[LPT];
     T pre_l = T(0);
-    T pre_lq[LPRE ? LPT : 1];   // LPRE: each load's node length
     // load step k0 into registers: load q -> panel, node e, 16-byte column group x
     auto fetch = [&](uint32_t k0) __attribute__((always_inline)) {
 #pragma unroll
@@ -940,7 +927,6 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
                 v = *reinterpret_cast<const vecT*>(src);
             }
             pre[q] = v;
-            if constexpr (LPRE) pre_lq[q] = k < K ? len[k] : T(0);
         }
         if (t < EB) pre_l = (k0 + t < K) ? len[k0 + t] : T(0);
     };
@@ -956,12 +942,6 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
                 if (panel < 2) {
 #pragma unroll
                     for (int z = 0; z < VEC; ++z) v[z] = v[z] > T(0) ? T(1) : T(0);
-                }
-            }
-            if constexpr (LPRE) {
-                if (panel < 2) {
-#pragma unroll
-                    for (int z = 0; z < VEC; ++z) v[z] *= pre_lq[q];
                 }
             }
             *reinterpret_cast<vecT*>(&sp[buf][panel][e][x]) = v;
@@ -995,7 +975,7 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
 #pragma unroll
                 for (int c = 0; c < RJ; ++c) {
                     if constexpr (TWO)
-                        pair_term<OP, T, LPRE, PW>(u[r], v[c], cu[r], cv[c], CNT ? mrow[r][c] : T(0), l, alpha,
+                        pair_term<OP, T, PW>(u[r], v[c], cu[r], cv[c], CNT ? mrow[r][c] : T(0), l, alpha,
                                                     num[r][c], den[r][c]);
                     else
                         pair_term<OP, T>(u[r], v[c], cu[r], cv[c], T(0), l, alpha, num[r][c], dummy);
@@ -1026,21 +1006,6 @@ k_pairs(const T* __restrict__ U, const T* __restrict__ Cn, const int32_t* __rest
             double nm, dn = 0.0;
             if constexpr (MIXED) { nm = num64[r][c]; if constexpr (TWO) dn = den64[r][c]; }
             else { nm = (double)num[r][c]; if constexpr (TWO) dn = (double)den[r][c]; }
-            if constexpr (TWO) {
-                if (add_partial) {
-                    if (i > j) continue;   // (the pair's i < j thread writes both entries)
-                    if (i < j) {
-                        if (out_fp64) {
-                            nm += ((const double*)out_v)[i * n + j];
-                            dn += ((const double*)out2_v)[i * n + j];
-                        } else {
-                            nm += (double)((const float*)out_v)[i * n + j];
-                            dn += (double)((const float*)out2_v)[i * n + j];
-                        }
-                        nm = nm < 0.0 ? 0.0 : nm;   // the shares' rounding can undershoot 0
-                    }
-                }
-            }
             double d;
             if (i == j) d = 0.0;
             else if (!normalized) d = nm;
@@ -1979,15 +1944,15 @@ __global__ void __launch_bounds__(256) k_matrix_to_stripes(double* __restrict__ 
     st[(size_t)blockIdx.y * n + k] = (double)M[(size_t)k * n + l];
 }
 
-template <PairOp OP, class T, int RI, int RJ, int TT = PAIR_TILE, bool LPRE = false, int PW = 0>
+template <PairOp OP, class T, int RI, int RJ, int TT = PAIR_TILE, int PW = 0>
 hipError_t launch_pairs_t(const PairArgs& a, hipStream_t st) {
     static_assert(PAIR_TILE % TT == 0, "the row stride is padded to PAIR_TILE");
     const uint32_t tiles = (a.n + TT - 1) / TT;
     dim3 grid(tiles, tiles);
     constexpr int NT = (TT / RI) * (TT / RJ);
-    hipLaunchKernelGGL((k_pairs<OP, T, RI, RJ, TT, LPRE, PW>), grid, dim3(NT), 0, st, (const T*)a.U, (const T*)a.Cn, a.rows, a.ldn,
+    hipLaunchKernelGGL((k_pairs<OP, T, RI, RJ, TT, PW>), grid, dim3(NT), 0, st, (const T*)a.U, (const T*)a.Cn, a.rows, a.ldn,
                        (const T*)a.len, a.K, a.n, a.S, a.totals, a.alpha, (int)a.normalized, a.out, (int)a.out_fp64,
-                       a.band, a.out2 ? 1 : 0, a.out2, a.flags, a.flag_tau);
+                       a.band, a.flags, a.flag_tau);
     return hipGetLastError();
 }
 
@@ -2001,24 +1966,20 @@ hipError_t launch_pairs_prec(PairOp op, const PairArgs& a, hipStream_t st) {
     // FP32 generalized powers (pair_term's PW): alpha = 1/2 by square roots, outside [0, 1]
     // with the exponent kept exact, otherwise the hardware exp2(a log2 s)
     case PairOp::generalized:
-        if (sizeof(T) == 4 && a.alpha == 0.5) return launch_pairs_t<PairOp::generalized, T, 4, 4, 64, false, 2>(a, st);
+        if (sizeof(T) == 4 && a.alpha == 0.5) return launch_pairs_t<PairOp::generalized, T, 4, 4, 64, 2>(a, st);
         return sizeof(T) == 4 && !(a.alpha >= 0.0 && a.alpha <= 1.0)
-                   ? launch_pairs_t<PairOp::generalized, T, 4, 4, 64, false, 1>(a, st)
+                   ? launch_pairs_t<PairOp::generalized, T, 4, 4, 64, 1>(a, st)
                    : launch_pairs_t<PairOp::generalized, T, 4, 4, 64>(a, st);
     case PairOp::vaw_weighted:
-        // FP64 only: in FP32, rounding l u and l v separately doubles the worst-case error of
-        // l |u - v| (2^-23 (u + v) l), past what the near-duplicate bound allows
-        return a.len_nonneg && sizeof(T) == 8 ? launch_pairs_t<PairOp::vaw_weighted, T, 4, 4, 64, true>(a, st)
-                                              : launch_pairs_t<PairOp::vaw_weighted, T, 4, 4, 64>(a, st);
+        return launch_pairs_t<PairOp::vaw_weighted, T, 4, 4, 64>(a, st);
     case PairOp::vaw_generalized:
         if (sizeof(T) == 4 && a.alpha == 0.5)
-            return launch_pairs_t<PairOp::vaw_generalized, T, 4, 4, 64, false, 2>(a, st);
+            return launch_pairs_t<PairOp::vaw_generalized, T, 4, 4, 64, 2>(a, st);
         return sizeof(T) == 4 && !(a.alpha >= 0.0 && a.alpha <= 1.0)
-                   ? launch_pairs_t<PairOp::vaw_generalized, T, 4, 4, 64, false, 1>(a, st)
+                   ? launch_pairs_t<PairOp::vaw_generalized, T, 4, 4, 64, 1>(a, st)
                    : launch_pairs_t<PairOp::vaw_generalized, T, 4, 4, 64>(a, st);
     case PairOp::vaw_unweighted:
-        return a.len_nonneg ? launch_pairs_t<PairOp::vaw_unweighted, T, 4, 4, 64, true>(a, st)
-                            : launch_pairs_t<PairOp::vaw_unweighted, T, 4, 4, 64>(a, st);
+        return launch_pairs_t<PairOp::vaw_unweighted, T, 4, 4, 64>(a, st);
     }
     return hipErrorInvalidValue;
 }
@@ -2354,7 +2315,6 @@ template hipError_t launch_unweighted_combine<double>(double*, const double*, ui
                                                       uint32_t, uint32_t);
 
 hipError_t launch_pairs(PairOp op, bool fp64, const PairArgs& a, hipStream_t st) {
-    if (a.out2 && op == PairOp::weighted) return hipErrorInvalidValue;   // (one accumulator: no denominator)
     return fp64 ? launch_pairs_prec<double>(op, a, st) : launch_pairs_prec<float>(op, a, st);
 }
 

@@ -187,11 +187,6 @@ struct PairArgs {
     void* out;              // n x n output
     bool out_fp64;
     GapBand band;           // tiles without a selected pair are skipped
-    // two-accumulator ops (VAW): with out2, out[i * n + j] and out2[i * n + j] (i < j) hold
-    // the posting-list shares of the numerator and denominator, added before the division
-    const void* out2 = nullptr;
-    // every length >= 0 (VAW weighted / presence terms stage l u instead of u)
-    bool len_nonneg = false;
     // unnormalised VAW weighted: with flags, a pair (i < j) whose distance is below
     // flag_tau of its VAW denominator sets flags[1 + i], flags[1 + j] and adds 1 to flags[0]
     uint32_t* flags = nullptr;

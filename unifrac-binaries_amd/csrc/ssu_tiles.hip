@@ -3,8 +3,7 @@
 // Every dense node is held by a sizeable share of the samples, so every pair
 // block visits it: the kernels are dense contractions with |x_i - x_j| in
 // place of the product, which no matrix instruction forms.  They are laid out
-// like a vector-ALU GEMM: 128 columns per tile, four waves of (rows / 2) x 64
-// pairs, a lane holding its rows and columns in groups of 16 bytes, a group
+// like a vector-ALU GEMM: a tile is a workgroup of 2 x 2 waves, a lane holding its rows and columns in groups of 16 bytes, a group
 // apart from the next lane's, so that its operands are ds_read_b128 of 8
 // distinct contiguous pieces (no bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
 // to LDS by global_load_lds, 16 bytes per lane, a stage of nodes ahead.
@@ -34,11 +33,13 @@ __device__ __forceinline__ void part_range(uint32_t nd, uint32_t eb, uint32_t p,
 //
 // An operation says what a lane holds and how a node's values enter a pair:
 //   V        operand type; FP32 sums are merged into FP64 every MERGE nodes
-//   RL       rows a lane holds (8, or 4 with two sums per pair), so a tile has 16 RL rows
+//   RL, CL   rows and columns a lane holds, so a tile has 16 RL x 16 CL pairs, WAVES of them per SIMD
+//            (8 x 8 at two waves; with two sums per pair 4 x 4 at three or four, which hide the
+//            transcendentals' latency: 8 rows by 4 at two took 15 to 20% longer for the VAW terms)
 //   EB       nodes per LDS stage (two stages are resident), UNROLL of them in one loop body
 //   TWO      a denominator is summed beside the numerator
 //   LEN      the node's length is staged too (otherwise U's rows are scaled by it)
-//   COUNTS   the samples' counts are staged beside their values, and the pair's totals used (VAW)
+//   COUNTS   the samples' counts are staged in the last of PANELS panels, and the pair's totals used (VAW)
 //   prep     what a lane does to a value it reads
 constexpr uint32_t MERGE = 64;
 
@@ -58,8 +59,9 @@ __device__ __forceinline__ double ratio(double nm, double dn, double share, doub
 // took 70.4 ms.
 struct OpW32 {
     typedef float V;
-    static constexpr int RL = 8, EB = 16, UNROLL = 16, BATCH = 1;
+    static constexpr int RL = 8, CL = 8, WAVES = 2, EB = 16, UNROLL = 16;
     static constexpr bool TWO = false, LEN = false, COUNTS = false, FLAGS = false;
+    static constexpr uint32_t PANELS = 1;
     static __device__ __forceinline__ float prep(float u) { return u; }
     static __device__ __forceinline__ void term(float u, float v, float, float& num) { num += __builtin_fabsf(u - v); }
     // d from the tile's sums x, y and the rare nodes' shares of them
@@ -78,8 +80,9 @@ struct OpW32 {
 // wave; 131 samples 0.37 -> 0.04 ms, the parts filling the device.
 struct OpW64 {
     typedef double V;
-    static constexpr int RL = 8, EB = 8, UNROLL = 8, BATCH = 1;
+    static constexpr int RL = 8, CL = 8, WAVES = 2, EB = 8, UNROLL = 8;
     static constexpr bool TWO = false, LEN = true, COUNTS = false, FLAGS = false;
+    static constexpr uint32_t PANELS = 1;
     static __device__ __forceinline__ double prep(double u) { return u; }
     static __device__ __forceinline__ void term(double u, double v, double l, double& num) {
         double m;
@@ -113,48 +116,87 @@ template <int AL> __device__ __forceinline__ double pow_less_one(double s, doubl
 // Generalized (src/unifrac_task_impl.hpp:1016-1024): num += l s^a |u - v| / s,
 // den += l s^a with s = u + v, both from the one power s^(a-1) (its error is
 // then the same in both and largely leaves the ratio).  Bound by VALU issue, the
-// transcendental a quarter of the add's rate: 4,000 samples x 1,930 dense nodes,
-// a = 1/2 in 3.7 ms (4.05 ms without the batches of 8, which hide the latency of
-// rsq), a = 1 in 1.4 ms, other a in 4.5 ms (batches do not help: 5.0).  32 x 64
-// pairs per wave with two powers per term: 1,777 samples 1.15 -> 0.64 ms at the
-// same split.
+// transcendental at a quarter of the add's rate: 4,000 samples x 1,930 dense
+// nodes, a = 1/2 in 3.76 ms, a = 1 in 1.25 ms, other a in 4.3 ms (several pairs'
+// powers in step measured the same).  32 x 64 pairs per wave with two powers per
+// term took 1.8 times as long.
 template <class T, int AL> struct OpGen {
     typedef T V;
-    static constexpr int RL = 4, EB = sizeof(T) == 4 ? 16 : 8, UNROLL = sizeof(T) == 4 ? 2 : 1, BATCH = sizeof(T) == 4 && AL == 1 ? 8 : 1;
+    static constexpr int RL = 4, CL = 4, WAVES = 4, EB = sizeof(T) == 4 ? 16 : 8, UNROLL = 1;
     static constexpr bool TWO = true, LEN = true, COUNTS = false, FLAGS = false;
+    static constexpr uint32_t PANELS = 1;
     static __device__ __forceinline__ T prep(T u) { return u; }
-    // BATCH pairs in step, so that one pair's power is computed while another's is under way
-    static __device__ __forceinline__ void terms(T u, const T* v, T l, T alpha, T* num, T* den) {
-        T s[BATCH], q[BATCH];
-#pragma unroll
-        for (int c = 0; c < BATCH; ++c) s[c] = u + v[c];
-        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < BATCH; ++c) q[c] = pow_less_one<AL>(s[c], alpha);
-        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < BATCH; ++c) {
-            num[c] = __builtin_elementwise_fma(__builtin_elementwise_abs(u - v[c]) * q[c], l, num[c]);
-            den[c] = __builtin_elementwise_fma(s[c] * q[c], l, den[c]);
-        }
-        if constexpr (BATCH > 1) __builtin_amdgcn_sched_barrier(0);
+    static __device__ __forceinline__ void term(T u, T v, T l, T alpha, T& num, T& den) {
+        const T s = u + v;
+        const T q = pow_less_one<AL>(s, alpha);
+        num = __builtin_elementwise_fma(__builtin_elementwise_abs(u - v) * q, l, num);
+        den = __builtin_elementwise_fma(s * q, l, den);
     }
     static __device__ __forceinline__ double distance(double x, double y, double share, double share2, double, bool) {
         return ratio(x, y, share, share2, true);
     }
 };
 
+// VAW (src/unifrac_task_impl.hpp:881-893, 1098-1109, 1817-1829): each node's
+// terms over vaw = sqrt(mi (m - mi)), mi = c_i + c_j, m = T_i + T_j, and 0 where
+// that is 0.  KIND 1: weighted, 2: presence (the counts are the one panel: a
+// sample holds the node where its count is positive), 3: generalized (0 <= alpha
+// <= 1: the weighted terms' quotients in the generalized terms).  Bound by VALU
+// issue: 4,000 samples x 3,550 dense nodes in 7.8 ms (FP32), 1,500 samples 1.36 ms
+// against 2.2 ms in whole 64 x 64 tiles (300 workgroups, node counts and totals in
+// registers).
+template <class T, int KIND, int AL = 0> struct OpVaw {
+    typedef T V;
+    static constexpr int RL = 4, CL = 4, WAVES = 3, EB = sizeof(T) == 4 ? 16 : 8, UNROLL = 1;
+    static constexpr bool TWO = true, LEN = true, COUNTS = true, FLAGS = KIND == 1;
+    static constexpr uint32_t PANELS = KIND == 2 ? 1 : 2;
+    static __device__ __forceinline__ T prep(T u) { return KIND == 2 ? (u > T(0) ? T(1) : T(0)) : u; }
+    static __device__ __forceinline__ float rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
+    static __device__ __forceinline__ double rsqrt(double x) { return rsqrt_nr<2>(x); }
+    // m - mi.  FP32 (whole counts, any two totals below 2^24: exact either way): from what
+    // each sample's total leaves of its count, once per sample and node; FP64: m - mi itself
+    // (the totals opaque here, or their 32 sums would be kept in registers across the nodes)
+    static __device__ __forceinline__ float other(float t, float c) { return t - c; }
+    static __device__ __forceinline__ double other(double t, double) {
+        asm volatile("" : "+v"(t));
+        return t;
+    }
+    static __device__ __forceinline__ float rest(float eu, float ev, float) { return eu + ev; }
+    static __device__ __forceinline__ double rest(double tu, double tv, double mi) { return (tu + tv) - mi; }
+    static __device__ __forceinline__ void term(T u, T v, T cu, T cv, T tu, T tv, T l, T alpha, T& num, T& den) {
+        const T mi = cu + cv;
+        const T x = mi * rest(tu, tv, mi);
+        const T rv = rsqrt(x);   // (x = 0: not finite, and not taken)
+        const T r = x > T(0) ? rv : T(0);
+        if constexpr (KIND == 3) {
+            const T s1 = (u + v) * r, d1 = __builtin_elementwise_abs(u - v) * r;
+            const T q = pow_less_one<AL>(s1, alpha);
+            num = __builtin_elementwise_fma(d1 * q, l, num);
+            den = __builtin_elementwise_fma(s1 * q, l, den);
+        } else {
+            const T t = l * r;
+            num = __builtin_elementwise_fma(__builtin_elementwise_abs(u - v), t, num);
+            const T o = KIND == 2 ? (u > v ? u : v) : u + v;
+            den = __builtin_elementwise_fma(o, t, den);
+        }
+    }
+    static __device__ __forceinline__ double distance(double x, double y, double share, double share2, double,
+                                                      bool normalized) {
+        return ratio(x, y, share, share2, normalized);
+    }
+};
+
 template <class OP> struct Shape {
     typedef typename OP::V V;
-    static constexpr uint32_t ROWS = 16 * OP::RL;               // of a tile: two waves of 8 RL
-    static constexpr uint32_t WAVE_ROWS = 8 * OP::RL;
-    static constexpr uint32_t NODE = ROWS + TILE_COLS;          // staged values of a node (and as many counts)
-    static constexpr uint32_t PAIRS = OP::RL * 8;               // of a lane
+    static constexpr uint32_t ROWS = 16 * OP::RL, COLS = 16 * OP::CL;   // of a tile: 2 x 2 waves
+    static constexpr uint32_t WAVE_ROWS = 8 * OP::RL, WAVE_COLS = 8 * OP::CL;
+    static constexpr uint32_t NODE = ROWS + COLS;               // staged values of a node (and as many counts)
+    static constexpr uint32_t PAIRS = OP::RL * OP::CL;          // of a lane
     static constexpr uint32_t SLOT = PAIRS * (OP::TWO ? 2 : 1) * 256;   // doubles of a workspace slot
     static constexpr bool MIXED = sizeof(V) == 4;
     static constexpr uint32_t G = 16 / sizeof(V);               // values of one 16-byte LDS read
-    static_assert(SLOT * sizeof(double) == TILE_SLOT, "every operation's slots have one size");
-    // the lane's q-th row in its wave's rows (l = li), or column in its wave's 64 columns (l = lj)
+    static_assert(SLOT * sizeof(double) == tile_slot_bytes(ROWS), "the workspace is sized by the tile's rows");
+    // the lane's q-th row in its wave's rows (l = li), or column in its wave's columns (l = lj)
     static __device__ __forceinline__ uint32_t at(uint32_t l, uint32_t q) { return q / G * (8 * G) + l * G + q % G; }
     // a lane's N values at(l, 0 .. N - 1) of a staged panel
     template <int N> static __device__ __forceinline__ void read(V (&x)[N], const V* panel, uint32_t l) {
@@ -194,32 +236,33 @@ __device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j
 }
 
 template <class OP>
-__global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
+__global__ void __launch_bounds__(256, OP::WAVES) k_tiles(TileArgs g) {
     typedef Shape<OP> SH;
     typedef typename OP::V V;
-    constexpr int RL = OP::RL;
-    constexpr uint32_t EB = OP::EB, PANELS = OP::COUNTS ? 2 : 1;
+    constexpr int RL = OP::RL, CL = OP::CL;
+    constexpr uint32_t EB = OP::EB, PANELS = OP::PANELS;
     const uint32_t seq = (blockIdx.x % N_XCDS) * g.per_xcd + blockIdx.x / N_XCDS;
     if (seq >= g.n_units) return;
     const uint32_t bij = g.units[seq].bij, part = g.units[seq].part;
     if (bij == TILE_NONE) return;
     const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
+    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * SH::WAVE_COLS;
     __shared__ __attribute__((aligned(16))) V sv[2][EB][PANELS][SH::NODE];   // a node: its rows, then its columns
     __shared__ V sl[2][EB];
+    __shared__ __attribute__((aligned(16))) V st[OP::COUNTS ? SH::NODE : 1];
 
     const uint32_t nd = g.dlist[0];
     const uint32_t np = (part & 63u) + 1;
     uint32_t ka, kb;
     part_range(nd, EB, (part >> 6) & 63u, np, ka, kb);
 
-    V num[RL][8], den[OP::TWO ? RL : 1][OP::TWO ? 8 : 1];
-    double num64[SH::MIXED ? RL : 1][SH::MIXED ? 8 : 1], den64[SH::MIXED && OP::TWO ? RL : 1][SH::MIXED && OP::TWO ? 8 : 1];
+    V num[RL][CL], den[OP::TWO ? RL : 1][OP::TWO ? CL : 1];
+    double num64[SH::MIXED ? RL : 1][SH::MIXED ? CL : 1], den64[SH::MIXED && OP::TWO ? RL : 1][SH::MIXED && OP::TWO ? CL : 1];
 #pragma unroll
     for (int r = 0; r < RL; ++r)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
+        for (int c = 0; c < CL; ++c) {
             num[r][c] = V(0);
             if constexpr (OP::TWO) den[r][c] = V(0);
             if constexpr (SH::MIXED) num64[r][c] = 0.0;
@@ -227,20 +270,13 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         }
 
     // wave w stages nodes w, w + 4, ..: 16 bytes per lane, rows then columns
-    constexpr uint32_t VEC = 16 / sizeof(V), RLANES = SH::ROWS / VEC, CLANES = TILE_COLS / VEC;
+    constexpr uint32_t VEC = 16 / sizeof(V), RLANES = SH::ROWS / VEC, CLANES = SH::COLS / VEC;
     const uint32_t* dl = g.dlist + 1;
-    const uint32_t i0 = bi * SH::ROWS, j0 = bj * TILE_COLS;
-    V ti[OP::COUNTS ? RL : 1], tj[OP::COUNTS ? 8 : 1];   // the samples' totals
-    if constexpr (OP::COUNTS) {
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-            const uint32_t i = i0 + wr + SH::at(li, r);
-            ti[r] = i < g.n ? (V)g.totals[i] : V(0);
-        }
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint32_t j = j0 + wc + SH::at(lj, c);
-            tj[c] = j < g.n ? (V)g.totals[j] : V(0);
+    const uint32_t i0 = bi * SH::ROWS, j0 = bj * SH::COLS;
+    if constexpr (OP::COUNTS) {   // the samples' totals (read again at each node: registers are short)
+        for (uint32_t q = threadIdx.x; q < SH::NODE; q += 256) {
+            const uint32_t smp = q < SH::ROWS ? i0 + q : j0 + q - SH::ROWS;
+            st[q] = smp < g.n ? (V)g.totals[smp] : V(0);
         }
     }
     // the rows of the wave's nodes of the stage after the next one to be loaded, read ahead of their use
@@ -262,7 +298,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
             const uint32_t ee = wave + 4 * e;
 #pragma unroll
             for (uint32_t p = 0; p < PANELS; ++p) {
-                const V* u = (const V*)(p ? g.C : g.U) + (size_t)row_next[e] * g.ldn;
+                const V* u = (const V*)(p == PANELS - 1 && OP::COUNTS ? g.C : g.U) + (size_t)row_next[e] * g.ldn;
                 V* to = &sv[buf][ee][p][0];
                 if constexpr (RLANES + CLANES <= 64) {
                     const V* src = u + (lane < RLANES ? i0 + lane * VEC : j0 + (lane - RLANES) * VEC);
@@ -280,24 +316,32 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
         if (k0 + EB < kb) index(k0 + EB);
     };
     auto node = [&](int buf, uint32_t e) __attribute__((always_inline)) {
-        V a[RL], b[8], ca[OP::COUNTS ? RL : 1], cb[OP::COUNTS ? 8 : 1];
+        V a[RL], b[CL], ca[OP::COUNTS ? RL : 1], cb[OP::COUNTS ? CL : 1], ea[OP::COUNTS ? RL : 1], eb[OP::COUNTS ? CL : 1];
         SH::read(a, &sv[buf][e][0][wr], li);
         SH::read(b, &sv[buf][e][0][SH::ROWS + wc], lj);
-        if constexpr (OP::COUNTS) {
+        if constexpr (OP::COUNTS) {   // (the last panel: the only one for presence terms)
             SH::read(ca, &sv[buf][e][PANELS - 1][wr], li);
             SH::read(cb, &sv[buf][e][PANELS - 1][SH::ROWS + wc], lj);
+            SH::read(ea, &st[wr], li);
+            SH::read(eb, &st[SH::ROWS + wc], lj);
+#pragma unroll
+            for (int r = 0; r < RL; ++r) ea[r] = OP::other(ea[r], ca[r]);
+#pragma unroll
+            for (int c = 0; c < CL; ++c) eb[c] = OP::other(eb[c], cb[c]);
         }
 #pragma unroll
         for (int r = 0; r < RL; ++r) a[r] = OP::prep(a[r]);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) b[c] = OP::prep(b[c]);
+        for (int c = 0; c < CL; ++c) b[c] = OP::prep(b[c]);
         const V l = OP::LEN ? sl[buf][e] : V(0);
         const V alpha = (V)g.alpha;
 #pragma unroll
         for (int r = 0; r < RL; ++r)
 #pragma unroll
-            for (int c = 0; c < 8; c += OP::BATCH) {
-                if constexpr (OP::TWO) OP::terms(a[r], b + c, l, alpha, num[r] + c, den[r] + c);
+            for (int c = 0; c < CL; ++c) {
+                if constexpr (OP::COUNTS)
+                    OP::term(a[r], b[c], ca[r], cb[c], ea[r], eb[c], l, alpha, num[r][c], den[r][c]);
+                else if constexpr (OP::TWO) OP::term(a[r], b[c], l, alpha, num[r][c], den[r][c]);
                 else OP::term(a[r], b[c], l, num[r][c]);
             }
     };
@@ -306,7 +350,7 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
 #pragma unroll
             for (int r = 0; r < RL; ++r)
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
+                for (int c = 0; c < CL; ++c) {
                     num64[r][c] += (double)num[r][c];
                     num[r][c] = V(0);
                     if constexpr (OP::TWO) { den64[r][c] += (double)den[r][c]; den[r][c] = V(0); }
@@ -348,16 +392,16 @@ __global__ void __launch_bounds__(256, 2) k_tiles(TileArgs g) {
 #pragma unroll
         for (int r = 0; r < RL; ++r)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                w[(r * 8 + c) * 256] = sum(r, c);
-                if constexpr (OP::TWO) w[(SH::PAIRS + r * 8 + c) * 256] = sum2(r, c);
+            for (int c = 0; c < CL; ++c) {
+                w[(r * CL + c) * 256] = sum(r, c);
+                if constexpr (OP::TWO) w[(SH::PAIRS + r * CL + c) * 256] = sum2(r, c);
             }
         return;
     }
 #pragma unroll
     for (int r = 0; r < RL; ++r)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
+        for (int c = 0; c < CL; ++c) {
             const size_t i = i0 + wr + SH::at(li, r), j = j0 + wc + SH::at(lj, c);
             if (i < j && j < g.n) write_pair<OP>(g, i, j, sum(r, c), sum2(r, c));
             else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
@@ -370,24 +414,25 @@ template <class OP>
 __global__ void __launch_bounds__(256) k_tiles_finish(TileArgs g) {
     typedef Shape<OP> SH;
     typedef typename OP::V V;
+    constexpr int CL = OP::CL;
     const uint32_t bij = g.split[blockIdx.x].bij, part = g.split[blockIdx.x].part;
     const uint32_t bi = bij >> 16, bj = bij & 0xffffu, np = (part & 63u) + 1, r = blockIdx.y;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * 64;
+    const uint32_t li = lane >> 3, lj = lane & 7, wr = (wave >> 1) * SH::WAVE_ROWS, wc = (wave & 1) * SH::WAVE_COLS;
     const double* w = g.ws + (size_t)(part >> 12) * SH::SLOT + threadIdx.x;
-    double x[8], y[8];
+    double x[CL], y[CL];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) x[c] = y[c] = 0.0;
+    for (int c = 0; c < CL; ++c) x[c] = y[c] = 0.0;
 #pragma unroll 2
     for (uint32_t p = 0; p < np; ++p)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            x[c] += w[(size_t)p * SH::SLOT + (r * 8 + c) * 256];
-            if constexpr (OP::TWO) y[c] += w[(size_t)p * SH::SLOT + (SH::PAIRS + r * 8 + c) * 256];
+        for (int c = 0; c < CL; ++c) {
+            x[c] += w[(size_t)p * SH::SLOT + (r * CL + c) * 256];
+            if constexpr (OP::TWO) y[c] += w[(size_t)p * SH::SLOT + (SH::PAIRS + r * CL + c) * 256];
         }
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const size_t i = bi * SH::ROWS + wr + SH::at(li, r), j = bj * TILE_COLS + wc + SH::at(lj, c);
+    for (int c = 0; c < CL; ++c) {
+        const size_t i = bi * SH::ROWS + wr + SH::at(li, r), j = bj * SH::COLS + wc + SH::at(lj, c);
         if (i < j && j < g.n) write_pair<OP>(g, i, j, x[c], y[c]);
         else if (i == j && i < g.n) ((V*)g.out)[i * g.n + i] = V(0);
     }
@@ -433,17 +478,18 @@ __global__ void __launch_bounds__(DL_T) k_dense_list(uint32_t* __restrict__ dlis
 // more round, are cut into np parts over the nodes, np the cheapest of
 // ceil(left * np / resident) rounds of 1 / np of a tile each plus the cost of
 // writing and reading the parts' sums.
-TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes, uint32_t resident) {
+TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes) {
+    const uint32_t resident = tile_resident(rows), cols = rows;
     TileSet t;
-    const uint32_t nbi = (n + rows - 1) / rows, nbj = (n + TILE_COLS - 1) / TILE_COLS;
+    const uint32_t nbi = (n + rows - 1) / rows, nbj = (n + cols - 1) / cols;
     // 1024 x 1024 samples per super-tile: about the tiles resident on one XCD
-    const uint32_t SI = std::max<uint32_t>(1, 1024 / rows), SJ = 1024 / TILE_COLS;
+    const uint32_t SI = std::max<uint32_t>(1, 1024 / rows), SJ = std::max<uint32_t>(1, 1024 / cols);
     std::vector<uint32_t> order;
     for (uint32_t si = 0; si < nbi; si += SI)
         for (uint32_t sj = 0; sj < nbj; sj += SJ)
             for (uint32_t bi = si; bi < std::min(nbi, si + SI); ++bi)
                 for (uint32_t bj = sj; bj < std::min(nbj, sj + SJ); ++bj)
-                    if ((bj + 1) * TILE_COLS > bi * rows) order.push_back(bi << 16 | bj);   // (with the diagonal)
+                    if (bj >= bi) order.push_back(bi << 16 | bj);   // (with the diagonal)
     t.tiles = order.size();
     // a part is at least 64 nodes; writing and reading one costs about as much as 24 nodes' terms
     const uint32_t most = std::max<uint32_t>(1, std::min<uint32_t>(TILE_MAX_PARTS, max_nodes / 64));
@@ -502,8 +548,8 @@ hipError_t launch_dense_list(uint32_t* dlist, const uint32_t* dmask, uint32_t K,
 template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_t st) {
     constexpr uint32_t rows = Shape<OP>::ROWS;
     if (!a.n || !a.n_units) return hipSuccess;   // (a selection without a tile here)
-    if (!a.U || !a.dlist || !a.out || !a.units || (OP::TWO ? a.add_partial && !a.out2 : !a.S) ||
-        (OP::COUNTS && (!a.C || !a.totals)) || (sizeof(typename OP::V) == 8 && !a.rows) || a.ldn % TILE_COLS || a.ldn < a.n ||
+    if ((!a.U && (!OP::COUNTS || OP::PANELS == 2)) || !a.dlist || !a.out || !a.units || (OP::TWO ? a.add_partial && !a.out2 : !a.S) ||
+        (OP::COUNTS && (!a.C || !a.totals)) || (sizeof(typename OP::V) == 8 && !a.rows) || a.ldn < a.n ||
         a.ldn % rows || (a.n + rows - 1) / rows > 65535 || (a.n_split && (!a.split || !a.ws)) || (OP::LEN && !a.len))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_tiles<OP>, dim3(a.per_xcd * N_XCDS), dim3(256), 0, st, a);
@@ -522,6 +568,21 @@ template <class T> static hipError_t launch_gen(const TileArgs& a, hipStream_t s
 }
 hipError_t launch_tiles_generalized(bool fp64, const TileArgs& a, hipStream_t st) {
     return fp64 ? launch_gen<double>(a, st) : launch_gen<float>(a, st);
+}
+
+template <class T> static hipError_t launch_vaw(int kind, const TileArgs& a, hipStream_t st) {
+    switch (kind) {
+    case 1: return launch_tiles<OpVaw<T, 1>>(a, st);
+    case 2: return launch_tiles<OpVaw<T, 2>>(a, st);
+    case 3:
+        if (a.alpha == 0.5) return launch_tiles<OpVaw<T, 3, 1>>(a, st);
+        if (a.alpha == 1.0) return launch_tiles<OpVaw<T, 3, 2>>(a, st);
+        return launch_tiles<OpVaw<T, 3, 0>>(a, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+hipError_t launch_tiles_vaw(int kind, bool fp64, const TileArgs& a, hipStream_t st) {
+    return fp64 ? launch_vaw<double>(kind, a, st) : launch_vaw<float>(kind, a, st);
 }
 
 }  // namespace ssu

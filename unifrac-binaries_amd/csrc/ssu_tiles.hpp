@@ -12,11 +12,19 @@
 
 namespace ssu {
 
-constexpr uint32_t TILE_COLS = 128;     // columns of every tile; its rows depend on the kernel
+// Tiles are square: 128 x 128 pairs with one sum per pair (weighted), 64 x 64 with
+// two (generalized, VAW).
+constexpr uint32_t TILE_ROWS_1 = 128, TILE_ROWS_2 = 64;
+// workgroups of 256 threads one XCD (32 CUs) holds: two (128) or three (64) waves per SIMD
+constexpr uint32_t tile_resident(uint32_t rows) { return rows == TILE_ROWS_1 ? 64 : 96; }
+// bytes of one workspace slot: a tile's sums in FP64
+constexpr size_t tile_slot_bytes(uint32_t rows) {
+    return size_t(rows) * rows * sizeof(double) * (rows == TILE_ROWS_1 ? 1 : 2);
+}
 constexpr uint32_t TILE_MAX_PARTS = 64;
 
 // One workgroup's work: part p of np of the tile of rows bi * rows .., columns
-// bj * TILE_COLS ..  Parts of one tile hold consecutive workspace slots.
+// bj * rows ..  Parts of one tile hold consecutive workspace slots.
 struct TileUnit {
     uint32_t bij;    // bi << 16 | bj; TILE_NONE: nothing
     uint32_t part;   // slot << 12 | p << 6 | (np - 1)
@@ -33,9 +41,8 @@ struct TileSet {
     uint32_t slots = 0;            // workspace slots used (parts of cut tiles)
     uint64_t tiles = 0;
 };
-// rows: tile rows (a divisor or multiple of TILE_COLS); max_nodes: an upper
-// bound on the dense nodes; resident: workgroups one XCD holds at a time.
-TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes, uint32_t resident);
+// rows: the tile's edge; max_nodes: an upper bound on the dense nodes.
+TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes);
 // those of `full` that keep(bi, bj) selects, cut as in `full` (so that a tile's
 // sums do not depend on the selection)
 TileSet tile_subset(const TileSet& full, const std::function<bool(uint32_t, uint32_t)>& keep);
@@ -43,7 +50,7 @@ TileSet tile_subset(const TileSet& full, const std::function<bool(uint32_t, uint
 struct TileArgs {
     const void* U;            // operand rows
     const int32_t* rows;      // FP64: operand row of processed node r (nullptr: r itself)
-    size_t ldn;               // their stride, a multiple of TILE_COLS
+    size_t ldn;               // their stride, a multiple of the tile's edge
     const double* len;        // [K] lengths (FP64 operands)
     const uint32_t* dlist;    // dlist[0] = dense nodes, then their processed-node indices
     uint32_t n;
@@ -57,17 +64,12 @@ struct TileArgs {
     const double* totals;     // VAW: the samples' totals
     uint32_t* flags;          // unnormalised VAW weighted: marks of near-duplicates (below
     float flag_tau;           //   flag_tau of the pair's VAW denominator), as launch_flag_close's
-    double* ws;               // workspace slots of TILE_SLOT bytes
+    double* ws;               // workspace slots of tile_slot_bytes
     const TileUnit* units;
     uint32_t n_units, per_xcd;
     const TileUnit* split;
     uint32_t n_split;
 };
-constexpr uint32_t TILE_ROWS_W = 128;      // rows per tile: one sum per pair (weighted)
-constexpr uint32_t TILE_ROWS_2 = 64;       // two sums per pair (generalized)
-constexpr size_t TILE_SLOT = size_t(128) * 128 * sizeof(double);   // bytes of one workspace slot
-constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD (32 CUs) holds at 2 waves per SIMD
-
 // Weighted.  FP32: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
 // share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (U's rows are scaled).
 // FP64: x = S_i + S_j - 2 M in its place, M = sum of l min(u_i, u_j) + the rare
@@ -75,6 +77,9 @@ constexpr uint32_t TILE_RESIDENT = 64;     // workgroups of 256 threads one XCD 
 hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st);
 // Generalized, 0 <= alpha <= 1: numerator over denominator, each with its share
 hipError_t launch_tiles_generalized(bool fp64, const TileArgs& a, hipStream_t st);
+// VAW (kind 1: weighted, 2: presence, 3: generalized, 0 <= alpha <= 1): numerator
+// over denominator, each with its share (or the numerator, not normalized)
+hipError_t launch_tiles_vaw(int kind, bool fp64, const TileArgs& a, hipStream_t st);
 
 // dlist from the dense mask ([ceil(K / 32)] words): dlist[0] = their number,
 // then the set bits in increasing order

@@ -61,3 +61,42 @@ def test_tiles_blocked_embedding(ssu, synth, O, monkeypatch, name, kw):
     # (the postings then take their values from the operand rows, which must not be scaled)
     monkeypatch.setenv("SSU_EMBED_BLOCK_SAMPLES", "128")
     check(ssu, O, *case(ssu, synth, O, 400, 300, 0.06, 5), name, kw)
+
+
+@pytest.mark.parametrize("name", ["weighted_normalized", "unweighted", "weighted_normalized_fp64", "unweighted_fp64",
+                                  "generalized_fp64"])
+@pytest.mark.parametrize("totals", ["few", "narrow", "wide", "beyond", "with_zero"])
+def test_vaw_one_sided_points(ssu, synth, O, monkeypatch, name, totals):
+    """One-sided VAW sums at the distinct totals themselves (at most 64), from a
+    series over totals within a factor of 2 and of 10,000, summed at every total
+    beyond that, and with an empty sample's zero total: against the oracle, and
+    against the sums at every total."""
+    monkeypatch.setenv("SSU_VAW_SPLIT", "1")   # every node on the posting lists
+    n, rng = 150, np.random.default_rng(3)
+    tree = synth.random_tree(200, 21)
+    obs, smp, ip, ix, data = synth.random_table(200, n, 0.15, 22)
+    data = rng.integers(1, 99, data.size).astype(float)
+    ix = np.asarray(ix)
+    if totals == "few":
+        data[:] = 1.0
+    elif totals in ("wide", "beyond"):   # one sample scaled up (the FP32 names then compute in FP64 past 2^24)
+        data[ix == 7] *= 3000 if totals == "wide" else 40000
+    table = [obs, smp, ip, ix, data]
+    if totals == "with_zero":
+        data[ix == 11] = 0.0
+    inp = ssu.Inputs(*tree, *table)
+    tot = np.bincount(ix, data, n)
+    kw = {"variance_adjust": True, "alpha": 0.4}
+    p = ssu.Plan(inp, name, **kw)
+    p.execute()
+    m = p.matrix()
+    monkeypatch.setenv("SSU_VAW_POINTS", "0")
+    q = ssu.Plan(inp, name, **kw)
+    q.execute()
+    ref = O.matrix(O.Tree(tree[0].astype(np.uint8), *tree[1:]), O.Table(*table), name.replace("_fp64", ""), **kw)
+    tol = TOL["fp64" if name.endswith("fp64") else "fp32"]
+    pos = tot[tot > 0]
+    assert (np.unique(tot).size <= 64) == (totals == "few")
+    print("[gpu-case]", name, totals, "distinct", np.unique(tot).size, "range", pos.max() / pos.min(), "err",
+          rel_err(m, ref), "against every total", rel_err(m, q.matrix()), flush=True)
+    assert rel_err(m, ref) <= tol and rel_err(m, q.matrix()) <= tol

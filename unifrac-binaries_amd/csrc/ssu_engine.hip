@@ -455,7 +455,9 @@ struct PlanImpl {
     // taken at the table's distinct totals tau_h (sample s at kidx_h[s])
     bool vsplit = false;
     std::vector<uint32_t> vdense_mask, vdense, kidx_h;
-    std::vector<double> tau_h;
+    std::vector<double> tau_h, vpts, vcos, vt;   // (one-sided sums at a few points: SparseNodesArgs::vpts)
+    uint32_t vN = 0;
+    void vaw_points();
     uint32_t split_thr = 0;          // FP32 shared-node path: nodes held by fewer samples use posting lists (0: off)
     double split_theta = 0.0;        // the occupancy split chosen (threshold / n; 0: none)
     uint32_t split_slots = 0;        // bound on their postings in any execution
@@ -550,7 +552,7 @@ struct PlanImpl {
         d_faith, d_stripes, d_smask, d_dmask, d_pc, d_pidx, d_pval, d_walked, d_rows, d_rcount, d_roff, d_rbsum,
         d_sp_node, d_sp_len, d_B, d_poff, d_pcnt, d_obsum, d_Ssp, d_out2, d_pspmax, d_urare, d_close,
         d_ridx, d_dlist, d_units, d_split, d_units_run, d_split_run, d_units_band, d_split_band, d_tws, d_udense,
-        d_order_run, d_order_band, d_vdense, d_tau, d_kidx, d_H, d_pcv, d_nbound;
+        d_order_run, d_order_band, d_vdense, d_tau, d_kidx, d_H, d_vpts, d_vcos, d_vt, d_Hc, d_pcv, d_nbound;
 
     hipStream_t own_st = nullptr;    // created with the plan; st may point at a caller's stream
     // per-execution inputs and output (nullptr: the plan's own table data / totals / result)
@@ -821,6 +823,37 @@ bool PlanImpl::upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std:
 // one-sided sums are taken at the table's distinct totals (an execution with
 // totals of its own takes them at every sample's).  The [n][D] sums must fit
 // VAW_H_BUDGET; SSU_VAW_SPLIT sets theta (0: off).
+// The totals the one-sided sums are taken at: the distinct totals where they are
+// few, Chebyshev points over their range where so many as hold the sums to FP64
+// rounding are at most VAW_POINTS - 1 (N terms leave 4 rho^-N / (rho - 1) of the
+// sums' size), otherwise (or where the terms are rounded to FP32, generalized
+// FP32) none: every total.  SSU_VAW_POINTS=0 turns them off.
+void PlanImpl::vaw_points() {
+    vpts.clear();
+    vcos.clear();
+    vt.clear();
+    vN = 0;
+    if (const char* env = getenv("SSU_VAW_POINTS"))
+        if (atoi(env) == 0) return;
+    if (spec.method == Method::generalized && !spec.fp64) return;
+    const size_t D = tau_h.size();
+    if (D <= VAW_POINTS) { vpts = tau_h; return; }
+    const bool zero = !(tau_h[0] > 0.0);
+    const double lo = tau_h[zero ? 1 : 0], hi = tau_h[D - 1];
+    if (!(lo > 0.0) || !std::isfinite(hi)) return;
+    const double mid = 0.5 * (std::log(hi) + std::log(lo)), L = 0.5 * (std::log(hi) - std::log(lo));
+    const double pi = 3.14159265358979323846, b = pi / L, rho = b + std::sqrt(1.0 + b * b);
+    const double terms = std::ceil(std::log(4.0 / ((rho - 1.0) * 1e-17)) / std::log(rho));
+    if (!(terms <= VAW_POINTS - 1)) return;
+    vN = (uint32_t)std::max(terms, 2.0);
+    for (uint32_t j = 0; j < vN; ++j) vpts.push_back(std::exp(mid + L * std::cos(pi * (j + 0.5) / vN)));
+    if (zero) vpts.push_back(tau_h[0]);
+    for (uint32_t k = 0; k < vN; ++k)
+        for (uint32_t j = 0; j < vN; ++j) vcos.push_back((k ? 2.0 : 1.0) / vN * std::cos(pi * k * (j + 0.5) / vN));
+    for (double x : tau_h)
+        vt.push_back(x > 0.0 ? std::min(1.0, std::max(-1.0, (std::log(x) - mid) / L)) : 2.0);
+}
+
 bool PlanImpl::split_vaw(std::string* err) {
     constexpr size_t VAW_H_BUDGET = (size_t)16 << 30;
     const char* env_theta = getenv("SSU_VAW_SPLIT");
@@ -835,11 +868,12 @@ bool PlanImpl::split_vaw(std::string* err) {
     kidx_h.resize(n);
     for (uint32_t s = 0; s < n; ++s)
         kidx_h[s] = (uint32_t)(std::lower_bound(tau_h.begin(), tau_h.end(), totals[s]) - tau_h.begin());
+    vaw_points();
     std::vector<uint32_t> cnt;
     if (!structural_counts(cnt, err)) return false;
     const SplitKind kind = spec.fp64 ? SplitKind::vaw64 : SplitKind::vaw32;
     uint32_t thr = env_theta ? (uint32_t)std::max(1.0, std::ceil(theta * n))
-                             : choose_split(kind, n, cnt, 1ull << 30, (uint32_t)tau_h.size()).thr;
+                             : choose_split(kind, n, cnt, 1ull << 30, (uint32_t)(vpts.empty() ? tau_h : vpts).size()).thr;
     if (thr == 0) return true;
     auto bound = [&](uint32_t t) {
         uint64_t b = 0;
@@ -862,7 +896,8 @@ bool PlanImpl::split_vaw(std::string* err) {
     vsplit = true;
     // (members: the host copies outlive the uploads)
     return upload(d_vdense, vdense_mask, st, err) && upload(d_dlist, vdense, st, err) &&
-           upload(d_tau, tau_h, st, err) && upload(d_kidx, kidx_h, st, err);
+           upload(d_tau, tau_h, st, err) && upload(d_kidx, kidx_h, st, err) && upload(d_vpts, vpts, st, err) &&
+           upload(d_vcos, vcos, st, err) && upload(d_vt, vt, st, err);
 }
 
 bool PlanImpl::embed_bits(DevMem& dst, uint32_t lb, bool structural, std::string* err) {
@@ -1324,6 +1359,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             (P.gen && !P.d_pspmax.ensure(sizeof(double), err)) ||
             (vsplit && !P.d_pcv.ensure((size_t)P.split_slots * (s.fp64 ? sizeof(double) : sizeof(float)), err)) ||
             (vsplit && !P.d_H.ensure(std::max<size_t>((size_t)P.n * vD, 1) * sizeof(double), err)) ||
+            (vsplit && !P.d_Hc.ensure(std::max<size_t>((size_t)P.n * P.vpts.size(), 1) * sizeof(double), err)) ||
             (vsplit && !P.d_nbound.ensure(kk * sizeof(double), err)) ||
             !P.d_obsum.ensure((offset_scan_blocks(K) + 1) * sizeof(uint32_t), err) ||
             !P.d_walked.ensure((size_t)sparse_rows_blocks(P.n) * sizeof(uint32_t), err) ||
@@ -1449,6 +1485,14 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             b.kidx = P.x_totals ? nullptr : P.d_kidx.as<uint32_t>();
             b.D = vD;
             b.H = P.d_H.as<double>();
+            if (!P.x_totals && !P.vpts.empty()) {
+                b.vpts = P.d_vpts.as<double>();
+                b.n_vpts = (uint32_t)P.vpts.size();
+                b.vN = P.vN;
+                b.vcos = P.d_vcos.as<double>();
+                b.vt = P.d_vt.as<double>();
+                b.Hc = P.d_Hc.as<double>();
+            }
             b.nbound = P.d_nbound.as<double>();
         }
         SSU_HIP(launch_sparse_nodes(b, P.st));

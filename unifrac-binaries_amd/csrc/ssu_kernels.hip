@@ -715,6 +715,11 @@ template <> __device__ __forceinline__ double dpow<double>(double x, double a) {
 // FP32 values none (the start's 5.2e-8 relative, measured on this GPU, is
 // below the FP32 rounding the reference's FP32 terms carry)
 template <class TV> constexpr int vaw_steps() { return sizeof(TV) == 8 ? 2 : 0; }
+// The one-sided terms (vaw_one), which the walk takes back out of sums that may
+// come from an interpolation: smooth in the total to FP64 rounding.  FP32 names
+// take one step (4.1e-15); their generalized terms round to FP32 (vaw_one_gen),
+// and are summed at every total.
+template <class TV, int VAW> constexpr int vaw_one_steps() { return sizeof(TV) == 8 ? 2 : VAW == 3 ? 0 : 1; }
 
 // x^alpha for x > 0 from the hardware log2 / exp2, as the generalized terms of
 // the shared-node path use them (0 <= alpha <= 1 there): exp2(a log2 x) carries
@@ -1375,7 +1380,7 @@ __device__ __forceinline__ double vaw_one_gen(double l, double u, double c, doub
 template <class TV, int VAW, uint32_t CW>
 __device__ __forceinline__ void vaw_row_term(unsigned long long* accb, const RowEntry<TV, true>& en, uint32_t b,
                                              TV v, TV cv, double Ta, double Tb, double scale, double alpha) {
-    constexpr int ST = vaw_steps<TV>();
+    constexpr int ST = vaw_steps<TV>(), OST = vaw_one_steps<TV, VAW>();
     const double l = __longlong_as_double((long long)en.q8);
     const double ua = (double)en.lu, ca = (double)en.uap, ub = (double)v, cb = (double)cv;
     const double ea = Ta - ca > 0.0 ? Ta - ca : 0.0, eb = Tb - cb > 0.0 ? Tb - cb : 0.0;
@@ -1384,9 +1389,9 @@ __device__ __forceinline__ void vaw_row_term(unsigned long long* accb, const Row
     const double rb = x > 0.0 ? r : 0.0;
     double one;
     if constexpr (VAW == 3)
-        one = vaw_one_gen<ST, TV>(l, ua, ca, ea, Tb, alpha) + vaw_one_gen<ST, TV>(l, ub, cb, eb, Ta, alpha);
+        one = vaw_one_gen<OST, TV>(l, ua, ca, ea, Tb, alpha) + vaw_one_gen<OST, TV>(l, ub, cb, eb, Ta, alpha);
     else
-        one = vaw_one<ST>(VAW == 2 ? l : l * ua, ca, ea, Tb) + vaw_one<ST>(VAW == 2 ? l : l * ub, cb, eb, Ta);
+        one = vaw_one<OST>(VAW == 2 ? l : l * ua, ca, ea, Tb) + vaw_one<OST>(VAW == 2 ? l : l * ub, cb, eb, Ta);
     double cn, cd;
     if constexpr (VAW == 2) {   // xor = 0, or = 1 for a node both hold
         cn = -one;
@@ -1849,7 +1854,7 @@ __global__ void __launch_bounds__(64) k_vaw_onesided(double* __restrict__ H, uin
                                                      const TV* __restrict__ pcv, const double* __restrict__ len,
                                                      const double* __restrict__ tot, uint32_t K, uint32_t n,
                                                      uint32_t slots, double alpha) {
-    constexpr int ST = vaw_steps<TV>();
+    constexpr int ST = vaw_one_steps<TV, VAW>();
     constexpr bool GEN = VAW == 3;
     const uint32_t a = blockIdx.x, lane = threadIdx.x;
     const uint32_t k0 = blockIdx.y * 64 * VH_COLS + lane;
@@ -1902,6 +1907,118 @@ __global__ void __launch_bounds__(64) k_vaw_onesided(double* __restrict__ H, uin
         const uint32_t k = k0 + 64 * j;
         if (k < D) H[(size_t)a * D + k] = acc[j];
     }
+}
+
+// The same sums without one pass per total.  As a function of the total t, a
+// one-sided term is (A + t)^(-1/2) (or -alpha/2) with A >= 0, analytic but for
+// t <= 0, so over totals from lo > 0 to hi a polynomial in log t of few degrees
+// holds H(a, .) to FP64 rounding: with 2L = log(hi / lo), the Chebyshev series
+// falls as rho^-N, rho = b + sqrt(1 + b^2), b = pi / L (totals within a factor of
+// 20: 27 terms).  k_vaw_points sums at the N Chebyshev points and forms the
+// coefficients (vN > 0), or sums at the totals themselves where those are few
+// (vN = 0); k_vaw_eval evaluates the series at every total by Clenshaw's
+// recurrence.  A zero total (an empty sample) is a point of its own, the last.
+// 1,500 samples (1,494 totals, 2.4e6 row entries): 1,149 us at every total, 85 us this way.
+//
+// k_vaw_points: one workgroup of four waves per sample, each wave a quarter of
+// the row's entries, staged 64 at a time in LDS; a lane holds point lane % p2 and
+// every (64 / p2)-th entry (p2: the points' number, up to a power of two).
+constexpr uint32_t VP_WAVES = 4;
+template <class TV, int VAW>
+__global__ void __launch_bounds__(64 * VP_WAVES) k_vaw_points(
+        double* __restrict__ out, uint32_t ldo, const double* __restrict__ pts, uint32_t np, uint32_t p2, uint32_t vN,
+        const double* __restrict__ vcos, const unsigned long long* __restrict__ rows,
+        const uint32_t* __restrict__ offsets, uint32_t nkc, const uint32_t* __restrict__ poff,
+        const TV* __restrict__ pval, const TV* __restrict__ pcv, const double* __restrict__ len,
+        const double* __restrict__ tot, uint32_t K, uint32_t n, uint32_t slots, double alpha) {
+    constexpr int ST = vaw_one_steps<TV, VAW>();
+    constexpr bool GEN = VAW == 3;
+    const uint32_t a = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __shared__ double sk[VP_WAVES][64], sc[VP_WAVES][64], se[VP_WAVES][64], su[GEN ? VP_WAVES : 1][64];
+    __shared__ double part[VP_WAVES][64], g[64];
+    const uint32_t pt = lane & (p2 - 1), grp = lane / p2, groups = 64 / p2;
+    const double tk = pt < np ? pts[pt] : 1.0;
+    double acc = 0.0;
+    if (poff[K] <= slots) {   // (never otherwise, by the plan's bound)
+        const double Ta = tot[a];
+        const uint32_t e0 = offsets[(size_t)a * nkc], e1 = offsets[(size_t)(a + 1) * nkc];
+        for (uint32_t q0 = e0 + 64 * w; q0 < e1; q0 += 64 * VP_WAVES) {   // uniform per wave
+            double kk = 0.0, cc = 0.0, ee = 0.0, uu = 0.0;
+            if (q0 + lane < e1) {
+                const unsigned long long ent = rows[q0 + lane];
+                const uint32_t r = (uint32_t)(ent >> 32);
+                const uint32_t slot = poff[r] + (uint32_t)ent;
+                const double l = len[r];
+                cc = (double)pcv[slot];
+                uu = (double)pval[slot];
+                kk = VAW == 1 ? l * uu : l;
+                ee = Ta - cc > 0.0 ? Ta - cc : 0.0;
+            }
+            sk[w][lane] = kk;
+            sc[w][lane] = cc;
+            se[w][lane] = ee;
+            if constexpr (GEN) su[w][lane] = uu;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const uint32_t cnt = min(64u, e1 - q0);
+#pragma unroll 2
+            for (uint32_t i = grp; i < cnt; i += groups) {
+                if constexpr (GEN) acc += vaw_one_gen<ST, TV>(sk[w][i], su[w][i], sc[w][i], se[w][i], tk, alpha);
+                else acc += vaw_one<ST>(sk[w][i], sc[w][i], se[w][i], tk);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    }
+    for (uint32_t d = p2; d < 64; d <<= 1) acc += __shfl_xor(acc, (int)d, 64);
+    part[w][lane] = acc;
+    __syncthreads();
+    if (threadIdx.x < np) {
+        double x = 0.0;
+        for (uint32_t q = 0; q < VP_WAVES; ++q) x += part[q][threadIdx.x];
+        g[threadIdx.x] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x < np) {
+        double x = g[threadIdx.x];
+        if (threadIdx.x < vN) {   // coefficient threadIdx.x of the series
+            x = 0.0;
+            for (uint32_t j = 0; j < vN; ++j) x = fma(vcos[threadIdx.x * vN + j], g[j], x);
+        }
+        out[(size_t)a * ldo + threadIdx.x] = x;
+    }
+}
+
+// H[a][k] = the series of sample a at t[k] in [-1, 1] (t[k] > 1: the zero total,
+// whose sum is entry vN).  Each thread one total, VE_ROWS samples.
+constexpr uint32_t VE_ROWS = 8;
+__global__ void __launch_bounds__(256) k_vaw_eval(double* __restrict__ H, uint32_t D, const double* __restrict__ t,
+                                                  const double* __restrict__ Hc, uint32_t ldc, uint32_t vN,
+                                                  uint32_t n) {
+    __shared__ double c[64][VE_ROWS];
+    const uint32_t a0 = blockIdx.y * VE_ROWS, k = blockIdx.x * 256 + threadIdx.x;
+    for (uint32_t q = threadIdx.x; q < ldc * VE_ROWS; q += 256) {
+        const uint32_t r = q / ldc, j = q % ldc;
+        c[j][r] = a0 + r < n ? Hc[(size_t)(a0 + r) * ldc + j] : 0.0;
+    }
+    __syncthreads();
+    if (k >= D) return;
+    const double x = t[k];
+    double b1[VE_ROWS], b2[VE_ROWS];
+#pragma unroll
+    for (uint32_t r = 0; r < VE_ROWS; ++r) b1[r] = b2[r] = 0.0;
+    for (uint32_t j = vN - 1; j > 0; --j)
+#pragma unroll
+        for (uint32_t r = 0; r < VE_ROWS; ++r) {
+            const double b = fma(2.0 * x, b1[r], c[j][r] - b2[r]);
+            b2[r] = b1[r];
+            b1[r] = b;
+        }
+#pragma unroll
+    for (uint32_t r = 0; r < VE_ROWS; ++r)
+        if (a0 + r < n) H[(size_t)(a0 + r) * D + k] = x > 1.0 ? c[vN][r] : fma(x, b1[r], c[0][r] - b2[r]);
 }
 
 // mx[0] = max of v[0..n): one workgroup
@@ -2419,7 +2536,17 @@ static void vaw_rows_t(uint32_t blocks, hipStream_t st, const SparseNodesArgs& a
                        a.tot, a.len, a.K, a.slots, a.alpha);
     hipLaunchKernelGGL(k_row_weights, dim3(a.n), dim3(64), 0, st, a.ssp, a.rows, a.roff, nkc, a.nbound,
                        (const uint32_t*)a.poff, a.K, a.n, a.slots);
-    hipLaunchKernelGGL((k_vaw_onesided<TV, VAW>), dim3(a.n, (a.D + 64 * VH_COLS - 1) / (64 * VH_COLS)), dim3(64), 0,
+    if (a.n_vpts) {   // at a few points (and the series at every total)
+        uint32_t p2 = 1;
+        while (p2 < a.n_vpts) p2 *= 2;
+        hipLaunchKernelGGL((k_vaw_points<TV, VAW>), dim3(a.n), dim3(64 * VP_WAVES), 0, st, a.vN ? a.Hc : a.H,
+                           a.n_vpts, a.vpts, a.n_vpts, p2, a.vN, a.vcos, a.rows, a.roff, nkc, (const uint32_t*)a.poff,
+                           (const TV*)a.pval, (const TV*)a.pcv, a.len, a.tot, a.K, a.n, a.slots, a.alpha);
+        if (a.vN)
+            hipLaunchKernelGGL(k_vaw_eval, dim3((a.D + 255) / 256, (a.n + VE_ROWS - 1) / VE_ROWS), dim3(256), 0, st,
+                               a.H, a.D, a.vt, (const double*)a.Hc, a.n_vpts, a.vN, a.n);
+    } else
+        hipLaunchKernelGGL((k_vaw_onesided<TV, VAW>), dim3(a.n, (a.D + 64 * VH_COLS - 1) / (64 * VH_COLS)), dim3(64), 0,
                        st, a.H, a.D, a.tau, a.rows, a.roff, nkc, (const uint32_t*)a.poff, (const TV*)a.pval,
                        (const TV*)a.pcv, a.len, a.tot, a.K, a.n, a.slots, a.alpha);
     pairs_rows_t<IX, false, TV, false, VAW>(blocks, st, a, nchunks, nkc, a0, na, mode);
@@ -2453,6 +2580,9 @@ hipError_t launch_sparse_rows(const SparseNodesArgs& a, hipStream_t st, uint32_t
     const bool whole = row0 == 0 && row1 == a.n;   // the per-sample sums are made for all rows at once
     if (a.vaw) {
         if (a.gram || a.gen || a.vaw < 1 || a.vaw > 3 || !a.ssp || !a.out2 || !a.pcv || !a.tot || !a.tau || !a.H ||
+            a.n_vpts > VAW_POINTS || (a.n_vpts && !a.vpts) || a.vN > a.n_vpts || a.vN == 1 ||
+            (a.vN ? !a.vcos || !a.vt || !a.Hc || a.n_vpts > a.vN + 1 : a.n_vpts && a.n_vpts != a.D) ||
+            (a.n + VE_ROWS - 1) / VE_ROWS > 65535 ||
             !a.nbound || !a.D || a.D > a.n || (!a.kidx && a.D != a.n) || !whole ||
             (a.vaw == 3 && !(a.alpha >= 0.0 && a.alpha <= 1.0)))
             return hipErrorInvalidValue;

@@ -257,8 +257,18 @@ struct SparseNodesArgs {
     const uint32_t* kidx = nullptr; // [n] sample -> its total's index in tau (nullptr: identity, D = n)
     uint32_t D = 0;
     double* H = nullptr;            // [n][D] one-sided sums
+    // with n_vpts > 0 they are summed at those totals only: the D totals themselves (vN = 0), or
+    // the vN Chebyshev points in log total, then the zero total if there is one; vcos [vN][vN]
+    // turns the sums at the points into a series' coefficients (Hc, [n][n_vpts]), vt [D] holds
+    // the totals' places in [-1, 1] (a zero total: above 1)
+    const double* vpts = nullptr;
+    uint32_t n_vpts = 0, vN = 0;
+    const double* vcos = nullptr;
+    const double* vt = nullptr;
+    double* Hc = nullptr;
     double* nbound = nullptr;       // [K] per-node correction bounds (ssp: their row sums)
 };
+constexpr uint32_t VAW_POINTS = 64;   // at most (a wave's lanes)
 // posting lists, per-panel prefix counts and row lists
 hipError_t launch_sparse_lists(const SparseNodesArgs& a, hipStream_t st);
 // each row's share over the posting lists (after launch_sparse_lists; in the

@@ -40,12 +40,14 @@ Rates rates_of(SplitKind k, double alpha) {
     case SplitKind::generalized64:
         if (alpha == 0.5) return {6.7e-13, 3.8e-12};
         return {alpha == 1.0 ? 2.0e-13 : 2.15e-12, 8.8e-12};
-    // VAW: the tiles' term (4,000 samples, theta 0.15 .. 0.6: 11.4 .. 3.3 ms; FP64, 2,000 samples:
-    // 7.7 .. 2.6); a posting (three FP64 reciprocal square roots) and a one-sided term at one
-    // total, fitted to the 8,192-sample workload at theta 0.25 / 0.5 / 1 (weighted and presence
-    // terms within 15% of each other; the weighted rates are used for both)
-    case SplitKind::vaw32: return {2.6e-13, 1.72e-12, 4.13e-13};
-    case SplitKind::vaw64: return {6.2e-13, 2.84e-12, 6.2e-13};
+    // VAW: the tiles' term; a posting (three FP64 reciprocal square roots); a one-sided term at
+    // one total (or point).  4,000 samples, theta 0.2 .. 0.8: tiles 9.37 .. 2.09 ms, posting phase
+    // 2.78 .. 14.3 (totals 14.3, 13.2 at 0.3, 13.5 at 0.4, 18.5); FP64, 2,000 samples: 6.42 .. 1.67
+    // and 1.28 .. 5.90 (8.63, 7.48 at 0.4, 8.49); the one-sided rate from the sums at every total
+    // of the 8,192-sample workload.  Weighted and presence terms are within 15% of each other; the
+    // weighted rates are used for both
+    case SplitKind::vaw32: return {2.65e-13, 2.37e-12, 4.13e-13};
+    case SplitKind::vaw64: return {6.7e-13, 3.8e-12, 6.2e-13};
     }
     return {1.0, 1.0};
 }

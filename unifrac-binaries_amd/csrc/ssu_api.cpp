@@ -410,7 +410,9 @@ ComputeStatus faith_common(const Table& t0, const PhyloTree& tree, r_vec** resul
     if (!degenerate) {
         std::string err;
         ssu::PostorderNodes nodes = synced_nodes(t, tree);
-        std::unique_ptr<Plan> plan = Plan::create(t, nodes, ComputeSpec{}, &err);
+        ComputeSpec spec;
+        spec.faith = true;
+        std::unique_ptr<Plan> plan = Plan::create(t, nodes, spec, &err);
         if (!plan || !plan->faith(r->values, &err)) {
             set_error(err);
             r_vec* rr = r;

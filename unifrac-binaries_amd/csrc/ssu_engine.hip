@@ -1162,7 +1162,7 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
 
     step("schedule");
     const bool unw = spec.method == Method::unweighted || spec.method == Method::unweighted_unnormalized;
-    P.gram = unw && !spec.vaw && spec.plain_kernel == 0;
+    P.gram = unw && !spec.vaw && spec.plain_kernel == 0 && !spec.faith;
     if (P.gram)   // non-finite lengths: VALU path
         for (size_t q = 0; q < P.knodes.size() && P.gram; ++q)
             P.gram = std::isfinite(spec.fp64 ? P.klen_d[q] : (double)P.klen_f[q]);
@@ -1174,8 +1174,9 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
     // Presence bits for the Gram path: with every value finite and >= 0 (and
     // positive totals), E[k][s] > 0 exactly when a stored value > 0 lies below
     // k, an OR up the tree.  SSU_GRAM_BITS=0 keeps the FP64 embedding.
-    if (P.gram && P.ldn / 32 <= BITS_MAX_WORDS) {
+    if ((P.gram || spec.faith) && P.ldn / 32 <= BITS_MAX_WORDS) {
         bool ok_vals = vals_nonneg;
+        for (size_t k = 0; k < P.len_all.size() && spec.faith && ok_vals; ++k) ok_vals = std::isfinite(P.len_all[k]);
         if (const char* env = getenv("SSU_GRAM_BITS")) ok_vals = ok_vals && atoi(env) != 0;
         if (ok_vals) {
             P.bits = true;
@@ -1998,7 +1999,12 @@ bool Plan::faith(double* host, std::string* err) {
     P.x_data = nullptr;    // the plan's own table
     P.x_totals = nullptr;
     if (!P.d_faith.ensure(std::max<uint32_t>(P.n, 1) * sizeof(double), err)) return false;
-    for (size_t c0 = 0; c0 < P.ldn && c0 < P.n; c0 += P.blk) {
+    if (P.spec.faith && P.bits) {   // present: a stored value > 0 lies below the node
+        if (!P.embed_bits(P.d_B, P.ldb, false, err)) return false;
+        SSU_HIP(launch_faith_bits(P.d_faith.as<double>(), P.d_B.as<uint32_t>(), P.ldb, P.d_len_all.as<double>(), P.m,
+                                  P.n, P.st));
+    }
+    for (size_t c0 = 0; c0 < P.ldn && c0 < P.n && !(P.spec.faith && P.bits); c0 += P.blk) {
         const size_t w = std::min(P.blk, P.ldn - c0);
         if (!P.embed(P.d_E, true, c0, w, err)) return false;
         SSU_HIP(launch_faith(P.d_faith.as<double>() + c0, P.d_E.as<double>(), w, P.d_len_all.as<double>(), P.m,

@@ -31,6 +31,7 @@ struct ComputeSpec {
     // per-sample sums S in segments that depend on the node count alone, so that a
     // sample's S does not depend on the other samples of the table (refinement sub-tables)
     bool fixed_segments = false;
+    bool faith = false;            // a plan for faith() alone: nothing prepared for the distances
 };
 
 // The spec a table's own values run with.  FP32 VAW terms hold the node counts

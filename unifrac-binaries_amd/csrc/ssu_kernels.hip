@@ -426,6 +426,72 @@ __global__ void __launch_bounds__(256) k_bits_smask(uint32_t* __restrict__ smask
     }
 }
 
+// Faith PD from presence bits: the sums of k_faith.  The ordered FP64 adds of a
+// sample are one serial chain, so the kernel is bound by the chain's length: a
+// node that none of a wave's 64 samples holds adds 0 to each and is left out
+// (every length finite).  One wave per 64 samples: lane l reads node k0 + l's two
+// words and length, the nodes held by a sample of the wave are compacted in order
+// into LDS, and each lane walks them, reading four nodes' words and lengths at a
+// time.  4,000 samples x 39,998 nodes: 543 us and 93 us for the bit rows, against 2.6 ms
+// from the FP64 embedding (1.3 GB written and read).
+constexpr uint32_t FB_LOADS = 4;   // nodes per round: 64 of them
+__global__ void __launch_bounds__(64) k_faith_bits(double* __restrict__ out, const uint32_t* __restrict__ B,
+                                                   uint32_t ldb, const double* __restrict__ len, uint32_t m,
+                                                   uint32_t n) {
+    __shared__ __attribute__((aligned(16))) uint32_t sw[2][64 * FB_LOADS + 4];
+    __shared__ __attribute__((aligned(16))) double sl[64 * FB_LOADS + 4];
+    const uint32_t lane = threadIdx.x, p0 = blockIdx.x * 2;   // (ldb is a multiple of 4)
+    const uint32_t* own = sw[lane >> 5];
+    const uint32_t sh = 31 - (lane & 31);
+    uint2 w[FB_LOADS];
+    double l[FB_LOADS];
+    auto fetch = [&](uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < FB_LOADS; ++u) {
+            const uint32_t k = k0 + 64 * u + lane;
+            w[u] = make_uint2(0u, 0u);
+            l[u] = 0.0;
+            if (k < m) {
+                w[u] = *reinterpret_cast<const uint2*>(B + (size_t)k * ldb + p0);
+                l[u] = len[k];
+            }
+        }
+    };
+    double acc = 0.0;
+    fetch(0);
+    for (uint32_t k0 = 0; k0 < m; k0 += 64 * FB_LOADS) {
+        uint32_t cnt = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < FB_LOADS; ++u) {
+            const uint64_t on = __ballot((w[u].x | w[u].y) != 0u);
+            if ((on >> lane) & 1u) {
+                const uint32_t at = cnt + __popcll(on & ((1ull << lane) - 1ull));
+                sw[0][at] = w[u].x;
+                sw[1][at] = w[u].y;
+                sl[at] = l[u];
+            }
+            cnt += (uint32_t)__popcll(on);
+        }
+        if (lane < 4) {   // the last four's remainder
+            sw[0][cnt + lane] = sw[1][cnt + lane] = 0u;
+            sl[cnt + lane] = 0.0;
+        }
+        __syncthreads();
+        fetch(k0 + 64 * FB_LOADS);   // in flight during the walk
+        for (uint32_t q = 0; q < cnt; q += 4) {
+            const uint4 b = *reinterpret_cast<const uint4*>(own + q);
+            const double2 l0 = *reinterpret_cast<const double2*>(sl + q), l1 = *reinterpret_cast<const double2*>(sl + q + 2);
+            const uint32_t bw[4] = {b.x, b.y, b.z, b.w};
+            const double lw[4] = {l0.x, l0.y, l1.x, l1.y};
+#pragma unroll
+            for (int z = 0; z < 4; ++z) acc += (int32_t)(bw[z] << sh) < 0 ? lw[z] : 0.0;
+        }
+        __syncthreads();
+    }
+    const uint32_t s = blockIdx.x * 64 + lane;
+    if (s < n) out[s] = acc;
+}
+
 // ------------------------------------------------------------------ Gram path
 
 // 64 K'-columns x 64 samples per workgroup: read node rows (coalesced over
@@ -2379,6 +2445,14 @@ hipError_t launch_faith(double* out, const double* E, size_t ldn, const double* 
                         hipStream_t st) {
     if (!n) return hipSuccess;
     hipLaunchKernelGGL(k_faith, dim3(grid1(n, 64)), dim3(64), 0, st, out, E, ldn, len, m, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_faith_bits(double* out, const uint32_t* B, uint32_t ldb, const double* len, uint32_t m, uint32_t n,
+                             hipStream_t st) {
+    if (!n) return hipSuccess;
+    if (ldb % 2 || (size_t)ldb * 32 < (size_t)(n + 63) / 64 * 64) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_faith_bits, dim3(grid1(n, 64)), dim3(64), 0, st, out, B, ldb, len, m, n);
     return hipGetLastError();
 }
 

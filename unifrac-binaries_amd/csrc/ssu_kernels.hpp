@@ -136,6 +136,9 @@ uint32_t fixed_rows_per_segment(uint32_t K);
 // Faith PD: out[s] = sum over all non-root nodes k in postorder of (E[k][s] > 0) * len[k]
 hipError_t launch_faith(double* out, const double* E, size_t ldn, const double* len, uint32_t m, uint32_t n,
                         hipStream_t st);
+// the same from presence bits (every length finite; ldb even, covering whole 64-sample groups)
+hipError_t launch_faith_bits(double* out, const uint32_t* B, uint32_t ldb, const double* len, uint32_t m, uint32_t n,
+                             hipStream_t st);
 
 // ---------------------------------------------------------------- Gram path
 // Pt[s][c] = 0xFF if E[col_node[c]][s] > 0 else 0 (col_node < 0 -> padding column)

@@ -230,6 +230,41 @@ ComputeStatus matrix_common(const Table& t0, const PhyloTree& tree, const char* 
     return run_full<TReal>(t, tree, make_spec(m, fp64, vaw, alpha, bypass, normalize), (*result)->matrix);
 }
 
+// The inputs of an in-memory call: the table's CSR on its way to the device from
+// the start; the tree sheared, collapsed and walked in postorder straight from its
+// arrays (src/api.cpp:90-100 SYNC_TREE_TABLE, VALIDATE_TREE_TABLE) on a second
+// thread, while this one borrows the table (sample totals) without an id map.
+struct InmemInputs {
+    std::shared_ptr<ssu::TableUpload> pre;
+    Table table;
+    ssu::PostorderNodes nodes;
+    uint32_t matched = 0, distinct = 0;   // table ids that name a leaf, of how many
+    bool tree_ok = false;
+    double input_ms = 0.0, tree_ms = 0.0;   // (overlapped)
+    InmemInputs(const support_biom_t* td, const support_bptree_t* tr) {
+        const auto t0 = Clock::now();
+        if (ssu::device_available(nullptr))
+            pre = ssu::TableUpload::start(td->indptr, td->indices, td->data, (uint32_t)td->n_obs);
+        std::thread tree_thread([&] {
+            const auto t1 = Clock::now();
+            ssu::NameIndex idx(td->obs_ids, (uint32_t)td->n_obs);
+            distinct = idx.distinct();
+            const double idx_ms = ms_since(t1);
+            tree_ok = tr->n_parens > 0 && ssu::synced_postorder(tr->structure, tr->lengths, tr->names,
+                                                                (uint32_t)tr->n_parens, idx, nodes, matched);
+            tree_ms = ms_since(t1);
+            static const bool timing = getenv("SSU_TIMING") && atoi(getenv("SSU_TIMING")) != 0;
+            if (timing)   // SSU_TIMING=1: the tree thread's two steps on stderr
+                fprintf(stderr, "[ssu tree] name index %7.2f ms, shear and postorder %7.2f ms\n", idx_ms,
+                        tree_ms - idx_ms);
+        });
+        table = Table::borrow(td->obs_ids, td->sample_ids, td->indptr, td->indices, td->data, (uint32_t)td->n_obs,
+                              (uint32_t)td->n_samples, false);
+        input_ms = ms_since(t0);
+        tree_thread.join();
+    }
+};
+
 template <class TReal, class TMat>
 ComputeStatus matrix_inmem(const support_biom_t* td, const support_bptree_t* tr, const char* method_name, bool vaw,
                            double alpha, bool bypass, bool normalize, unsigned depth, bool with_repl,
@@ -254,43 +289,17 @@ ComputeStatus matrix_inmem(const support_biom_t* td, const support_bptree_t* tr,
         g_call_ms[CP_TOTAL] = ms_since(t0);
         return v;
     }
-    // the table's CSR on its way to the device from the start; the tree sheared,
-    // collapsed and walked in postorder straight from its arrays (src/api.cpp:90-100
-    // SYNC_TREE_TABLE, VALIDATE_TREE_TABLE) on a second thread, while this one
-    // borrows the table (sample totals) without an id map
-    std::shared_ptr<ssu::TableUpload> pre;
-    if (ssu::device_available(nullptr))
-        pre = ssu::TableUpload::start(td->indptr, td->indices, td->data, (uint32_t)td->n_obs);
-    ssu::PostorderNodes nodes;
-    uint32_t matched = 0, distinct = 0;
-    bool tree_ok = false;
-    double tree_ms = 0.0;
-    std::thread tree_thread([&] {
-        const auto t1 = Clock::now();
-        ssu::NameIndex idx(td->obs_ids, (uint32_t)td->n_obs);
-        distinct = idx.distinct();
-        const double idx_ms = ms_since(t1);
-        tree_ok = tr->n_parens > 0 && ssu::synced_postorder(tr->structure, tr->lengths, tr->names,
-                                                            (uint32_t)tr->n_parens, idx, nodes, matched);
-        tree_ms = ms_since(t1);
-        static const bool timing = getenv("SSU_TIMING") && atoi(getenv("SSU_TIMING")) != 0;
-        if (timing)   // SSU_TIMING=1: the tree thread's two steps on stderr
-            fprintf(stderr, "[ssu tree] name index %7.2f ms, shear and postorder %7.2f ms\n", idx_ms,
-                    tree_ms - idx_ms);
-    });
-    Table t = Table::borrow(td->obs_ids, td->sample_ids, td->indptr, td->indices, td->data, (uint32_t)td->n_obs,
-                            (uint32_t)td->n_samples, false);
-    g_call_ms[CP_INPUT] = ms_since(t0);
-    tree_thread.join();
-    g_call_ms[CP_TREE] = tree_ms;   // (overlapped with the inputs)
-    if (!tree_ok) return tree_missing;
-    if (matched < distinct) return table_and_tree_do_not_overlap;
-    if (*result == nullptr && !init_full<TReal, TMat>(*result, t.sample_ids, mmap_dir)) {
+    InmemInputs in(td, tr);
+    g_call_ms[CP_INPUT] = in.input_ms;
+    g_call_ms[CP_TREE] = in.tree_ms;
+    if (!in.tree_ok) return tree_missing;
+    if (in.matched < in.distinct) return table_and_tree_do_not_overlap;
+    if (*result == nullptr && !init_full<TReal, TMat>(*result, in.table.sample_ids, mmap_dir)) {
         set_error("result allocation failed");
         return output_error;
     }
-    const ComputeStatus v =
-        run_full<TReal>(t, nodes, make_spec(m, fp64, vaw, alpha, bypass, normalize), (*result)->matrix, pre);
+    const ComputeStatus v = run_full<TReal>(in.table, in.nodes, make_spec(m, fp64, vaw, alpha, bypass, normalize),
+                                            (*result)->matrix, in.pre);
     g_call_ms[CP_TOTAL] = ms_since(t0);
     return v;
 }
@@ -394,6 +403,27 @@ ComputeStatus dense_pair(unsigned n_obs, const char** obs_ids, const double* s1,
     return st;
 }
 
+// Faith PD of a table whose every sample and row is kept
+ComputeStatus faith_result(const Table& t, const ssu::PostorderNodes& nodes,
+                           const std::shared_ptr<ssu::TableUpload>& pre, r_vec** result) {
+    r_vec* r = (r_vec*)malloc(sizeof(r_vec));
+    r->n_samples = t.n_samples;
+    r->values = (double*)calloc(t.n_samples ? t.n_samples : 1, sizeof(double));
+    r->sample_ids = dup_ids(t.sample_ids);
+    std::string err;
+    ComputeSpec spec;
+    spec.faith = true;
+    std::unique_ptr<Plan> plan = Plan::create(t, nodes, spec, &err, pre);
+    if (!plan || !plan->faith(r->values, &err)) {
+        set_error(err);
+        r_vec* rr = r;
+        destroy_results_vec(&rr);
+        return output_error;
+    }
+    *result = r;
+    return okay;
+}
+
 ComputeStatus faith_common(const Table& t0, const PhyloTree& tree, r_vec** result) {
     // src/api.cpp:569-604: drop zero-count samples (total < 1), shear, Faith PD
     if (t0.n_samples == 0 || t0.n_obs == 0) return table_empty;
@@ -402,24 +432,11 @@ ComputeStatus faith_common(const Table& t0, const PhyloTree& tree, r_vec** resul
     if (degenerate) fprintf(stderr, "WARNING: All samples had zero counts. Forcing zero result.\n");
     else if (nz.n_samples != t0.n_samples || nz.n_obs != t0.n_obs)
         fprintf(stderr, "WARNING: Some samples had zero counts and were filtered out.\n");
-    const Table& t = degenerate ? t0 : nz;
+    if (!degenerate) return faith_result(nz, synced_nodes(nz, tree), nullptr, result);
     r_vec* r = (r_vec*)malloc(sizeof(r_vec));
-    r->n_samples = t.n_samples;
-    r->values = (double*)calloc(t.n_samples ? t.n_samples : 1, sizeof(double));
-    r->sample_ids = dup_ids(t.sample_ids);
-    if (!degenerate) {
-        std::string err;
-        ssu::PostorderNodes nodes = synced_nodes(t, tree);
-        ComputeSpec spec;
-        spec.faith = true;
-        std::unique_ptr<Plan> plan = Plan::create(t, nodes, spec, &err);
-        if (!plan || !plan->faith(r->values, &err)) {
-            set_error(err);
-            r_vec* rr = r;
-            destroy_results_vec(&rr);
-            return output_error;
-        }
-    }
+    r->n_samples = t0.n_samples;
+    r->values = (double*)calloc(t0.n_samples ? t0.n_samples : 1, sizeof(double));
+    r->sample_ids = dup_ids(t0.sample_ids);
     *result = r;
     return okay;
 }
@@ -732,6 +749,23 @@ ComputeStatus faith_pd_one_off(const char* biom_filename, const char* tree_filen
 
 ComputeStatus ssu_faith_pd_inmem(const support_biom_t* td, const support_bptree_t* tr, r_vec** result) {
     if (!td || !tr || td->n_samples <= 0 || td->n_obs <= 0) return table_empty;
+    // The overlapped path of the in-memory matrices (the table's CSR and the tree on
+    // threads of their own, the table borrowed, no id maps or copies), for tables that
+    // the filter below leaves as they are: every total >= 1, an entry in every row.
+    // 4,000 samples x 20,000 tips (1.7e6 entries): 3.5 ms against 19 ms with the table
+    // filtered into a copy and the tree sheared and collapsed node by node.
+    bool rows_held = true;
+    for (int i = 0; i < td->n_obs && rows_held; ++i) rows_held = td->indptr[i + 1] > td->indptr[i];
+    if (rows_held) {
+        InmemInputs in(td, tr);
+        bool whole = in.table.index_ok;
+        for (uint32_t s = 0; s < in.table.n_samples && whole; ++s) whole = in.table.totals[s] >= 1.0;
+        if (whole) {
+            if (!in.tree_ok) return tree_missing;
+            if (in.matched < in.distinct) return table_and_tree_do_not_overlap;
+            return faith_result(in.table, in.nodes, in.pre, result);
+        }
+    }
     Table t = Table::borrow(td->obs_ids, td->sample_ids, td->indptr, td->indices, td->data, (uint32_t)td->n_obs,
                             (uint32_t)td->n_samples);
     PhyloTree tree = PhyloTree::from_arrays(tr->structure, tr->lengths, tr->names, tr->n_parens);

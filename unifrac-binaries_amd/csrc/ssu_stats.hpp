@@ -7,8 +7,8 @@
 //     B Q; two power levels here where scikit-bio uses one);
 //   * PERMANOVA pseudo-F (Anderson 2001) with a permutation p-value.
 // The reference reaches these through its third-party skbb library
-// (src/skbio_alt.cpp:144-233); the n x n products and the permutation sums
-// run here as HIP kernels, the (n x 3k) QR and the small SVD on the host.
+// (src/skbio_alt.cpp:144-233); the n x n products, the permutations and their sums
+// and the (n x 3k) QR run here as HIP kernels, the small SVD on the host.
 #pragma once
 
 #include <cstdint>

@@ -532,7 +532,7 @@ struct PlanImpl {
     std::vector<double> len_all;     // every non-root node, postorder (Faith PD)
     // exact Gram
     std::vector<int32_t> col_node;
-    std::vector<int8_t> digits;      // [4][Kp]
+    std::vector<int8_t> digits;      // 4 per Gram column, in the order of k_gram_i8r's reads
     std::vector<GramChunk> chunks;
     size_t Kp = 0, n_pad = 0;
 
@@ -659,9 +659,14 @@ bool PlanImpl::build_gram_columns() {
         b0 = b1;
     }
     Kp = col_node.size();
+    // as k_gram_i8r's lanes read them, 512 bytes per stage of 128 columns: [half of a
+    // 32-column step][digit * 4 + word of the half][step][byte of the word]
     digits.assign(4 * std::max<size_t>(Kp, 1), 0);
-    for (size_t c = 0; c < Kp; ++c)
-        for (int r = 0; r < 4; ++r) digits[(size_t)r * Kp + c] = dg[c][r];
+    for (size_t c = 0; c < Kp; ++c) {
+        const size_t in = c % GRAM_BK, half = in % 32 / 16, word = in % 16 / 4;
+        for (size_t r = 0; r < 4; ++r)
+            digits[c / GRAM_BK * 512 + half * 256 + (r * 4 + word) * 16 + in / 32 * 4 + in % 4] = dg[c][r];
+    }
     return true;
 }
 

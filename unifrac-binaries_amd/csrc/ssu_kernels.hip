@@ -576,6 +576,18 @@ __device__ __forceinline__ size_t gram_slot(uint32_t i, uint32_t j, uint32_t til
 constexpr int GLDA = GRAM_BK + 16;  // padded LDS row in bytes: ds_read_b128 stays conflict-free
 constexpr int GRAM_THREADS = 512;
 
+// b with its four words masked by words PLANE * 4 .. + 3 of dg's 16 lanes (each row of
+// 16 lanes has its own; a DPP broadcast within the AND)
+template <int PLANE>
+__device__ __forceinline__ v4i and_digits(v4i b, int dg) {
+    v4i r;
+    r.x = b.x & __builtin_amdgcn_update_dpp(0, dg, 0x150 + PLANE * 4, 0xf, 0xf, true);
+    r.y = b.y & __builtin_amdgcn_update_dpp(0, dg, 0x150 + PLANE * 4 + 1, 0xf, 0xf, true);
+    r.z = b.z & __builtin_amdgcn_update_dpp(0, dg, 0x150 + PLANE * 4 + 2, 0xf, 0xf, true);
+    r.w = b.w & __builtin_amdgcn_update_dpp(0, dg, 0x150 + PLANE * 4 + 3, 0xf, 0xf, true);
+    return r;
+}
+
 // Exact Gram on v_mfma_i32_32x32x32_i8.
 //   A operand: presence of the row samples, bytes 0x00 / 0xFF (0 / -1)
 //   B operand: presence of the column samples AND digit byte d_q of the column's length
@@ -583,11 +595,20 @@ constexpr int GRAM_THREADS = 512;
 // Workgroup: 8 waves on a 128x128 output tile.  Wave w owns rows (w>>2)*64 ..
 // +64 and columns (w&3)*32 .. +32 of the tile (two 32x32 MFMA blocks) for all
 // four digits: 128 accumulator registers, and per K step three operand
-// fragments for eight MFMAs.  At the end of each K-chunk the wave merges its
+// fragments from LDS for eight MFMAs; the digits of a step are one register (each
+// lane of a row of 16 holds a word) and reach the AND by DPP broadcast.  Read from
+// LDS as fragments they were 16 of 28 reads a stage, and LDS as busy as the matrix
+// cores.  Three stage buffers with the barrier in mid-stage: a wave goes from one
+// stage into the next without waiting, and a stage's global loads have a whole stage
+// to arrive.  At the end of each K-chunk the wave merges its
 // four digits exactly, acc_0 + 2^7 acc_1 + 2^14 acc_2 + 2^21 acc_3 (below
 // 2^45), and adds it times the chunk scale into its FP64 partial of the tile
 // held in registers (one FMA per chunk and element); G is written once, in the
 // fragment order of gram_slot.
+// Bound by the matrix cores: 8,000 samples x 8,580 columns 0.79 ms (2.9 POPS; two
+// buffers 0.89, one buffer and digits in LDS 1.03), 1,000 x 39.7k on 36 of the 256
+// CUs 0.35 ms (76% of those CUs' rate; 0.42, 0.49).  One wave per SIMD on 64 x 64 pairs
+// (a fragment fewer per eight MFMAs) took 1.6 times as long: nothing covers its waits.
 __global__ void __launch_bounds__(GRAM_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt, size_t ldp,
            const int8_t* __restrict__ digits, const GramChunk* __restrict__ chunks, uint32_t n_chunks,
@@ -595,104 +616,97 @@ k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt
     const uint32_t seq = (blockIdx.x % N_XCDS) * per_xcd + blockIdx.x / N_XCDS;
     if (seq >= n_tiles) return;
     const uint32_t bi = order[seq] >> 16, bj = order[seq] & 0xffffu;
-    __shared__ __attribute__((aligned(16))) int8_t sA[GRAM_BM * GLDA];
-    __shared__ __attribute__((aligned(16))) int8_t sB[GRAM_BM * GLDA];
-    __shared__ __attribute__((aligned(16))) int8_t sD[4 * GRAM_BK];
+    constexpr uint32_t SA = 0, SB = GRAM_BM * GLDA, SBUF = 2 * GRAM_BM * GLDA;
+    __shared__ __attribute__((aligned(16))) int8_t sm[3 * SBUF];   // three stages
 
     const uint32_t t = threadIdx.x;
     const uint32_t lane = t & 63, wave = t >> 6;
     const uint32_t rh = wave >> 2, cq = wave & 3;   // 64 rows, 32 columns
-    const size_t Kp = ldp;
 
     static_assert(GRAM_BK == 128 && GRAM_THREADS == 512, "staging below assumes 128-column stages, 512 threads");
-    const uint32_t lrow = t >> 3, lc16 = (t & 7) * 16;
+    const uint32_t lrow = t >> 3, lc16 = (t & 7) * 16;   // rows lrow and lrow + 64
     const int8_t* gA0 = Pt + ((size_t)bi * GRAM_BM + lrow) * ldp + lc16;
     const int8_t* gB0 = Pt + ((size_t)bj * GRAM_BM + lrow) * ldp + lc16;
     const size_t rstep = (size_t)64 * ldp;
-    int8_t* sA0 = sA + lrow * GLDA + lc16;
-    int8_t* sB0 = sB + lrow * GLDA + lc16;
-    const int8_t* gD0 = digits + (size_t)lrow * Kp + lc16;   // digit plane lrow, for t < 32
-    int8_t* sD0 = sD + lrow * GRAM_BK + lc16;
-    uint4 ra0, ra1, rb0, rb1, rd;
-#define SSU_GLOAD(stage)                                                              \
-    do {                                                                              \
-        const size_t k0_ = (size_t)(stage) * GRAM_BK;                                 \
-        ra0 = *reinterpret_cast<const uint4*>(gA0 + k0_);                             \
-        ra1 = *reinterpret_cast<const uint4*>(gA0 + rstep + k0_);                     \
-        rb0 = *reinterpret_cast<const uint4*>(gB0 + k0_);                             \
-        rb1 = *reinterpret_cast<const uint4*>(gB0 + rstep + k0_);                     \
-        if (t < 32) rd = *reinterpret_cast<const uint4*>(gD0 + k0_);                  \
-    } while (0)
-#define SSU_SSTORE()                                                                  \
-    do {                                                                              \
-        *reinterpret_cast<uint4*>(sA0) = ra0;                                         \
-        *reinterpret_cast<uint4*>(sA0 + 64 * GLDA) = ra1;                             \
-        *reinterpret_cast<uint4*>(sB0) = rb0;                                         \
-        *reinterpret_cast<uint4*>(sB0 + 64 * GLDA) = rb1;                             \
-        if (t < 32) *reinterpret_cast<uint4*>(sD0) = rd;                              \
-    } while (0)
-
-    v16i acc[4][2];   // [digit][mi]
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) acc[d][mi] = (v16i){0};
+    const int8_t* gD0 = digits + (lane >> 5) * 256 + (lane & 15) * 16;
+    int8_t* sw = sm + lrow * GLDA + lc16;
+    uint4 ra0, ra1, rb0, rb1, dn;
+    const auto gload = [&](uint32_t stage) __attribute__((always_inline)) {
+        const size_t k0 = (size_t)stage * GRAM_BK;
+        ra0 = *reinterpret_cast<const uint4*>(gA0 + k0);
+        ra1 = *reinterpret_cast<const uint4*>(gA0 + rstep + k0);
+        rb0 = *reinterpret_cast<const uint4*>(gB0 + k0);
+        rb1 = *reinterpret_cast<const uint4*>(gB0 + rstep + k0);
+    };
+    const auto sstore = [&](uint32_t off) __attribute__((always_inline)) {
+        int8_t* b = sw + off;
+        *reinterpret_cast<uint4*>(b + SA) = ra0;
+        *reinterpret_cast<uint4*>(b + SA + 64 * GLDA) = ra1;
+        *reinterpret_cast<uint4*>(b + SB) = rb0;
+        *reinterpret_cast<uint4*>(b + SB + 64 * GLDA) = rb1;
+    };
     double gacc[2][16];   // the wave's FP64 partial of G, C-fragment order
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
         for (int r = 0; r < 16; ++r) gacc[mi][r] = 0.0;
 
-    const uint32_t arow = rh * 64 + (lane & 31);
-    const uint32_t brow = cq * 32 + (lane & 31);
     const uint32_t khalf = (lane >> 5) * 16;
+    const int8_t* arow = sm + SA + (rh * 64 + (lane & 31)) * GLDA + khalf;
+    const int8_t* brow = sm + SB + (cq * 32 + (lane & 31)) * GLDA + khalf;
 
-    uint32_t ch = 0;
-    uint32_t ch_end_stage = n_chunks ? chunks[0].k1 / GRAM_BK : 0;
-    if (n_stages) { SSU_GLOAD(0); SSU_SSTORE(); }
-    __syncthreads();
-    for (uint32_t s = 0; s < n_stages; ++s) {
-        if (s + 1 < n_stages) SSU_GLOAD(s + 1);
-#pragma unroll
-        for (int kk = 0; kk < GRAM_BK / 32; ++kk) {
-            const uint32_t ko = kk * 32 + khalf;
-            const v4i a0 = *reinterpret_cast<const v4i*>(sA + arow * GLDA + ko);
-            const v4i a1 = *reinterpret_cast<const v4i*>(sA + (arow + 32) * GLDA + ko);
-            const v4i pb = *reinterpret_cast<const v4i*>(sB + brow * GLDA + ko);
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const v4i b = pb & *reinterpret_cast<const v4i*>(sD + d * GRAM_BK + ko);
-                acc[d][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b, acc[d][0], 0, 0, 0);
-                acc[d][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b, acc[d][1], 0, 0, 0);
-            }
-        }
-        if (s + 1 == ch_end_stage) {
-            // exact merge of the four digits (|acc| <= 127 * 2^17), then one FMA per element
-            const double sc = -chunks[ch].scale;   // A carries -1 for "present"
-#pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    double v = fma((double)acc[3][mi][r], 128.0, (double)acc[2][mi][r]);
-                    v = fma(v, 128.0, (double)acc[1][mi][r]);
-                    v = fma(v, 128.0, (double)acc[0][mi][r]);
-                    gacc[mi][r] = fma(v, sc, gacc[mi][r]);
-                }
-#pragma unroll
-            for (int d = 0; d < 4; ++d)
-#pragma unroll
-                for (int mi = 0; mi < 2; ++mi) acc[d][mi] = (v16i){0};
-            ++ch;
-            if (ch < n_chunks) ch_end_stage = chunks[ch].k1 / GRAM_BK;
-        }
-        __syncthreads();
-        if (s + 1 < n_stages) {
-            SSU_SSTORE();
-            __syncthreads();
-        }
+    if (n_stages) {
+        gload(0);
+        sstore(0);
+        dn = *reinterpret_cast<const uint4*>(gD0);
+        gload(min(1u, n_stages - 1));
     }
-#undef SSU_GLOAD
-#undef SSU_SSTORE
+    __syncthreads();
+    uint32_t s = 0, off = 0, off_n = SBUF;   // the stage's buffer, the next one's
+    for (uint32_t ch = 0; ch < n_chunks; ++ch) {
+        const uint32_t s_end = chunks[ch].k1 / GRAM_BK;
+        v16i acc[4][2];   // [digit][mi]
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi) acc[d][mi] = (v16i){0};
+        for (; s < s_end; ++s) {
+            const int dg[4] = {(int)dn.x, (int)dn.y, (int)dn.z, (int)dn.w};   // this stage's, one word per step
+            dn = *reinterpret_cast<const uint4*>(gD0 + (size_t)min(s + 1, n_stages - 1) * 512);
+            const auto step = [&](int kk) __attribute__((always_inline)) {
+                const v4i a0 = *reinterpret_cast<const v4i*>(arow + off + kk * 32);
+                const v4i a1 = *reinterpret_cast<const v4i*>(arow + off + 32 * GLDA + kk * 32);
+                const v4i pb = *reinterpret_cast<const v4i*>(brow + off + kk * 32);
+                const v4i b[4] = {and_digits<0>(pb, dg[kk]), and_digits<1>(pb, dg[kk]), and_digits<2>(pb, dg[kk]),
+                                  and_digits<3>(pb, dg[kk])};
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    acc[d][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b[d], acc[d][0], 0, 0, 0);
+                    acc[d][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b[d], acc[d][1], 0, 0, 0);
+                }
+            };
+            step(0);
+            step(1);
+            sstore(off_n);   // stage s + 1; its buffer was last read in stage s - 2
+            __syncthreads();
+            gload(min(s + 2, n_stages - 1));
+            step(2);
+            step(3);
+            off = off_n;
+            off_n = off_n == 2 * SBUF ? 0 : off_n + SBUF;
+        }
+        // exact merge of the four digits (|acc| <= 127 * 2^17), then one FMA per element
+        const double sc = -chunks[ch].scale;   // A carries -1 for "present"
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                double v = fma((double)acc[3][mi][r], 128.0, (double)acc[2][mi][r]);
+                v = fma(v, 128.0, (double)acc[1][mi][r]);
+                v = fma(v, 128.0, (double)acc[0][mi][r]);
+                gacc[mi][r] = fma(v, sc, gacc[mi][r]);
+            }
+    }
     // quadrant rh*2 + cq/2, block (mi, cq&1) of the fragment order of gram_slot
     double* gl = G + ((size_t)bi * tiles + bj) * (GRAM_BM * GRAM_BM) + lane;
 #pragma unroll

@@ -12,7 +12,7 @@ namespace {
 // (50k tips) workloads (total = fixed + terms * term + postings * posting); the
 // modelled optimum lands within the measured one for every kind (weighted
 // 0.193 vs 0.2, FP64 weighted 0.24 vs 0.23 - 0.3, generalized 0.38 vs 0.4,
-// Gram 0.075 vs 0.06 - 0.1).  The per-term cost includes the list building
+// Gram 0.07 vs 0.06 - 0.1).  The per-term cost includes the list building
 // and row lists, whose work follows the postings.
 struct Rates {
     double term;      // one (pair, node) term of the tiled kernel; Gram: one (pair, column) unit
@@ -32,7 +32,8 @@ Rates rates_of(SplitKind k, double alpha) {
     // square roots), 9.94 .. 3.74 (0.3: log2 and exp2), 3.14 .. 1.14 (1: no power), posting
     // phase 1.73 .. 6.20 ms; best totals at 0.4 (9.39 ms), 0.5 (10.5) and 0.2 - 0.3 (5.9)
     case SplitKind::generalized32: return {alpha == 1.0 ? 8.5e-14 : alpha == 0.5 ? 2.25e-13 : 2.65e-13, 1.57e-12};
-    case SplitKind::gram: return {3.4e-15, 6.1e-13};
+    // Gram: 0.82 ms for the 2.96e11 units of 8,000 samples, 3.73 for the 1.21e12 of 16,384
+    case SplitKind::gram: return {2.9e-15, 6.1e-13};
     // FP64 generalized, 1,200 samples, theta 0.2 .. 0.6: alpha 1/2 tiles 2.54 .. 0.90 ms, posting
     // phase 0.58 .. 1.55 (totals 3.51, 2.83 at 0.4 - 0.6); other alpha (an FP64 power per tile
     // term, two per posting) 8.07 .. 2.84 and 1.01 .. 3.28 (totals 9.47, 6.5 at 0.6); alpha 1

@@ -1391,7 +1391,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             !P.d_rbsum.ensure((row_list_scan_blocks(P.n, Ks) + 1) * sizeof(uint32_t), err))
             return false;
     }
-    if (P.gram && !P.d_G.ensure(P.n_pad * P.n_pad * sizeof(double), err)) return false;
+    if (P.gram && !P.d_G.ensure(P.n_pad * P.n_pad * sizeof(double) + gram_ws_bytes((uint32_t)P.n_pad, P.Kp), err))
+        return false;
     if (gather) {
         if (!P.d_U.ensure(std::max<size_t>(K, 1) * P.ldn * sizeof(float), err)) return false;
         if (s.vaw && !P.d_Cu.ensure(std::max<size_t>(K, 1) * P.ldn * sizeof(float), err)) return false;
@@ -1566,7 +1567,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             SSU_HIP(launch_gram_i8(P.d_G.as<double>(), P.d_Pt.as<int8_t>(), P.Kp, P.d_digits.as<int8_t>(),
                                    P.d_chunks.as<GramChunk>(), (uint32_t)P.chunks.size(), (uint32_t)P.n_pad,
                                    P.d_order_band.as<uint32_t>() + P.band_off[k], P.band_off[k + 1] - P.band_off[k],
-                                   P.st));
+                                   P.d_G.as<double>() + P.n_pad * P.n_pad, P.st));
             if (gsplit) {
                 if (k == 0) SSU_HIP(launch_sparse_rows(gb, P.st, 0, P.n, ROWS_DIAGONAL));
                 SSU_HIP(launch_sparse_rows(gb, P.st, r0, r1, ROWS_OFF_DIAGONAL));
@@ -1582,7 +1583,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             SSU_HIP(launch_gram_i8(P.d_G.as<double>(), P.d_Pt.as<int8_t>(), P.Kp, P.d_digits.as<int8_t>(),
                                    P.d_chunks.as<GramChunk>(), (uint32_t)P.chunks.size(), (uint32_t)P.n_pad,
                                    P.band_all ? P.d_order.as<uint32_t>() : P.d_order_run.as<uint32_t>(),
-                                   (uint32_t)P.order_used().size(), P.st));
+                                   (uint32_t)P.order_used().size(), P.d_G.as<double>() + P.n_pad * P.n_pad, P.st));
         } else {
             SSU_HIP(launch_fill(P.d_G.as<double>(), P.n_pad * P.n_pad, 0.0, P.st));   // no memset node in captures
         }

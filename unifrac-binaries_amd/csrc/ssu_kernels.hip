@@ -575,6 +575,7 @@ __device__ __forceinline__ size_t gram_slot(uint32_t i, uint32_t j, uint32_t til
 
 constexpr int GLDA = GRAM_BK + 16;  // padded LDS row in bytes: ds_read_b128 stays conflict-free
 constexpr int GRAM_THREADS = 512;
+constexpr size_t GRAM_TILE = (size_t)GRAM_BM * GRAM_BM;
 
 // b with its four words masked by words PLANE * 4 .. + 3 of dg's 16 lanes (each row of
 // 16 lanes has its own; a DPP broadcast within the AND)
@@ -612,10 +613,14 @@ __device__ __forceinline__ v4i and_digits(v4i b, int dg) {
 __global__ void __launch_bounds__(GRAM_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt, size_t ldp,
            const int8_t* __restrict__ digits, const GramChunk* __restrict__ chunks, uint32_t n_chunks,
-           uint32_t n_stages, const uint32_t* __restrict__ order, uint32_t n_tiles, uint32_t per_xcd) {
+           uint32_t all_stages, const uint32_t* __restrict__ order, uint32_t n_tiles, uint32_t parts,
+           double* __restrict__ ws, uint32_t per_xcd) {
     const uint32_t seq = (blockIdx.x % N_XCDS) * per_xcd + blockIdx.x / N_XCDS;
-    if (seq >= n_tiles) return;
-    const uint32_t bi = order[seq] >> 16, bj = order[seq] & 0xffffu;
+    if (seq >= n_tiles * parts) return;
+    const uint32_t part = seq / n_tiles, bij = order[seq - part * n_tiles];
+    const uint32_t bi = bij >> 16, bj = bij & 0xffffu;
+    uint32_t s = (uint32_t)((uint64_t)part * all_stages / parts);   // this part's stages
+    const uint32_t s1 = (uint32_t)((uint64_t)(part + 1) * all_stages / parts);
     constexpr uint32_t SA = 0, SB = GRAM_BM * GLDA, SBUF = 2 * GRAM_BM * GLDA;
     __shared__ __attribute__((aligned(16))) int8_t sm[3 * SBUF];   // three stages
 
@@ -655,16 +660,18 @@ k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt
     const int8_t* arow = sm + SA + (rh * 64 + (lane & 31)) * GLDA + khalf;
     const int8_t* brow = sm + SB + (cq * 32 + (lane & 31)) * GLDA + khalf;
 
-    if (n_stages) {
-        gload(0);
+    if (s < s1) {
+        gload(s);
         sstore(0);
-        dn = *reinterpret_cast<const uint4*>(gD0);
-        gload(min(1u, n_stages - 1));
+        dn = *reinterpret_cast<const uint4*>(gD0 + (size_t)s * 512);
+        gload(min(s + 1, s1 - 1));
     }
     __syncthreads();
-    uint32_t s = 0, off = 0, off_n = SBUF;   // the stage's buffer, the next one's
-    for (uint32_t ch = 0; ch < n_chunks; ++ch) {
-        const uint32_t s_end = chunks[ch].k1 / GRAM_BK;
+    uint32_t off = 0, off_n = SBUF;   // the stage's buffer, the next one's
+    uint32_t ch = 0;
+    while (ch < n_chunks && chunks[ch].k1 / GRAM_BK <= s) ++ch;
+    for (; ch < n_chunks && s < s1; ++ch) {
+        const uint32_t s_end = min(chunks[ch].k1 / GRAM_BK, s1);
         v16i acc[4][2];   // [digit][mi]
 #pragma unroll
         for (int d = 0; d < 4; ++d)
@@ -672,7 +679,7 @@ k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt
             for (int mi = 0; mi < 2; ++mi) acc[d][mi] = (v16i){0};
         for (; s < s_end; ++s) {
             const int dg[4] = {(int)dn.x, (int)dn.y, (int)dn.z, (int)dn.w};   // this stage's, one word per step
-            dn = *reinterpret_cast<const uint4*>(gD0 + (size_t)min(s + 1, n_stages - 1) * 512);
+            dn = *reinterpret_cast<const uint4*>(gD0 + (size_t)min(s + 1, s1 - 1) * 512);
             const auto step = [&](int kk) __attribute__((always_inline)) {
                 const v4i a0 = *reinterpret_cast<const v4i*>(arow + off + kk * 32);
                 const v4i a1 = *reinterpret_cast<const v4i*>(arow + off + 32 * GLDA + kk * 32);
@@ -689,7 +696,7 @@ k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt
             step(1);
             sstore(off_n);   // stage s + 1; its buffer was last read in stage s - 2
             __syncthreads();
-            gload(min(s + 2, n_stages - 1));
+            gload(min(s + 2, s1 - 1));
             step(2);
             step(3);
             off = off_n;
@@ -708,12 +715,28 @@ k_gram_i8r(double* __restrict__ G, uint32_t tiles, const int8_t* __restrict__ Pt
             }
     }
     // quadrant rh*2 + cq/2, block (mi, cq&1) of the fragment order of gram_slot
-    double* gl = G + ((size_t)bi * tiles + bj) * (GRAM_BM * GRAM_BM) + lane;
+    double* gl = (parts > 1 ? ws + (size_t)seq * GRAM_TILE : G + ((size_t)bi * tiles + bj) * GRAM_TILE) + lane;
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             gl[(size_t)(((((rh * 2 + (cq >> 1)) * 2 + mi) * 2 + (cq & 1)) * 16 + r) * 64)] = gacc[mi][r];
+}
+
+// G's tiles from their parts' sums, in order of the parts
+__global__ void __launch_bounds__(256) k_gram_sum(double* __restrict__ G, uint32_t tiles, const double* __restrict__ ws,
+                                                  const uint32_t* __restrict__ order, uint32_t n_tiles, uint32_t parts) {
+    const uint32_t bij = order[blockIdx.y];
+    const size_t e = blockIdx.x * 512 + threadIdx.x * 2;
+    const double* w = ws + (size_t)blockIdx.y * GRAM_TILE + e;
+    double2 v = make_double2(0.0, 0.0);
+#pragma unroll 8
+    for (uint32_t p = 0; p < parts; ++p) {
+        const double2 x = *reinterpret_cast<const double2*>(w + (size_t)p * n_tiles * GRAM_TILE);
+        v.x += x.x;
+        v.y += x.y;
+    }
+    *reinterpret_cast<double2*>(G + ((size_t)(bij >> 16) * tiles + (bij & 0xffffu)) * GRAM_TILE + e) = v;
 }
 
 template <class TOut>
@@ -2478,15 +2501,46 @@ hipError_t launch_presence_T(int8_t* Pt, size_t ldp, const double* E, size_t lde
     return hipGetLastError();
 }
 
+// A Gram of fewer tiles than CUs (T = tiles (tiles + 1) / 2) leaves CUs idle: its
+// stages are then split over `parts` workgroups per tile, whose sums k_gram_sum adds.
+// The choice minimises rounds of workgroups * (stages of a part * 1.1 us + 3) plus 64 ns
+// per part sum written and read, from T of the whole matrix, so that a pair's sum does
+// not depend on which tiles a launch computes.  1,000 samples x 39.7k columns (36 tiles):
+// 73 us in 7 parts, 345 in one; 256 samples (3 tiles): 14 us against 31.
+uint32_t gram_parts(uint32_t n_pad, size_t ldp) {
+    const uint64_t tiles = n_pad / GRAM_BM, T = tiles * (tiles + 1) / 2, S = ldp / GRAM_BK;
+    uint32_t best = 1;
+    double best_us = 0.0;
+    for (uint64_t p = 1; p <= 32 && (p == 1 || (T * p <= GRAM_MAX_PARTS && S >= 2 * p)); ++p) {
+        const double us = (double)((T * p + 255) / 256) * ((double)((S + p - 1) / p) * 1.1 + 3.0) +
+                          (p > 1 ? 4.0 + 0.064 * (double)(T * p) : 0.0);
+        if (p == 1 || us < best_us) {
+            best = (uint32_t)p;
+            best_us = us;
+        }
+    }
+    return best;
+}
+size_t gram_ws_bytes(uint32_t n_pad, size_t ldp) {
+    const size_t tiles = n_pad / GRAM_BM, parts = gram_parts(n_pad, ldp);
+    return parts > 1 ? tiles * (tiles + 1) / 2 * parts * GRAM_TILE * sizeof(double) : 0;
+}
+
 hipError_t launch_gram_i8(double* G, const int8_t* Pt, size_t ldp, const int8_t* digits, const GramChunk* chunks,
-                          uint32_t n_chunks, uint32_t n_pad, const uint32_t* order, uint32_t n_tiles, hipStream_t st) {
+                          uint32_t n_chunks, uint32_t n_pad, const uint32_t* order, uint32_t n_tiles, double* ws,
+                          hipStream_t st) {
     if (n_pad % GRAM_BM || ldp % GRAM_BK) return hipErrorInvalidValue;
     const uint32_t tiles = n_pad / GRAM_BM;
     if (tiles > 65535 || n_tiles > tiles * (tiles + 1) / 2 || !order) return hipErrorInvalidValue;
     if (!n_tiles) return hipSuccess;
-    const uint32_t per_xcd = (n_tiles + N_XCDS - 1) / N_XCDS;
+    const uint32_t parts = gram_parts(n_pad, ldp);
+    if (parts > 1 && !ws) return hipErrorInvalidValue;
+    const uint32_t per_xcd = (n_tiles * parts + N_XCDS - 1) / N_XCDS;
     hipLaunchKernelGGL(k_gram_i8r, dim3(per_xcd * N_XCDS), dim3(GRAM_THREADS), 0, st, G, tiles, Pt, ldp, digits,
-                       chunks, n_chunks, (uint32_t)(ldp / GRAM_BK), order, n_tiles, per_xcd);
+                       chunks, n_chunks, (uint32_t)(ldp / GRAM_BK), order, n_tiles, parts, ws, per_xcd);
+    if (parts > 1)
+        hipLaunchKernelGGL(k_gram_sum, dim3((uint32_t)(GRAM_TILE / 512), n_tiles), dim3(256), 0, st, G, tiles, ws, order,
+                           n_tiles, parts);
     return hipGetLastError();
 }
 

@@ -150,9 +150,13 @@ hipError_t launch_presence_T_bits(int8_t* Pt, size_t ldp, const uint32_t* B, uin
                                   uint32_t Kp, uint32_t n_pad, uint32_t n, hipStream_t st);
 // G = sum_c len_c * P[i][c] * P[j][c] for the upper-triangle 128x128 tiles, FP64,
 // stored tile by tile in MFMA fragment order (n_pad/128)^2 * 128^2 doubles;
-// order lists the tiles computed (every tile, or a subset)
+// order lists the tiles computed (every tile, or a subset); ws: gram_ws_bytes of scratch
+// (few tiles: their columns split over several workgroups each)
+constexpr uint32_t GRAM_MAX_PARTS = 512;   // tiles * parts
+size_t gram_ws_bytes(uint32_t n_pad, size_t ldp);
 hipError_t launch_gram_i8(double* G, const int8_t* Pt, size_t ldp, const int8_t* digits, const GramChunk* chunks,
-                          uint32_t n_chunks, uint32_t n_pad, const uint32_t* order, uint32_t n_tiles, hipStream_t st);
+                          uint32_t n_chunks, uint32_t n_pad, const uint32_t* order, uint32_t n_tiles, double* ws,
+                          hipStream_t st);
 // out[i][j] from G and T = diag(G): (T_i+T_j-2G)/(T_i+T_j-G) or T_i+T_j-2G, rows i in [row0, row1)
 template <class TOut>
 hipError_t launch_unweighted_combine(TOut* out, const double* G, uint32_t n_pad, uint32_t n, bool normalized,

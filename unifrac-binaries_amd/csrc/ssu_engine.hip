@@ -506,6 +506,9 @@ struct PlanImpl {
     // rows in the band (band 0 also every diagonal tile), the posting walk of its
     // rows (after band 0's tiles: the diagonal G(a, a) of every row) and the
     // banded combine of its rows, in order on st.
+    // (an embedding the 256 MB memory-side cache holds gains nothing: one-off weighted calls of 106
+    // and 266 MB 2 - 3% slower for the bits, of 492 MB equal or 3% faster, resident plans of 1 GB 6%)
+    static constexpr size_t HELD_MIN_BYTES = size_t(256) << 20;
     static constexpr uint32_t OUT_BANDS = 10, OUT_BANDS_GRAM = 16;
     std::vector<uint32_t> band_row0, band_off;   // rows [band_row0[k], band_row0[k + 1]); blocks [band_off[k], ..)
     std::vector<hipEvent_t> band_ev;
@@ -584,11 +587,24 @@ struct PlanImpl {
     bool split_weighted(std::string* err);
     bool split_vaw(std::string* err);
     bool structural_counts(std::vector<uint32_t>& cnt, std::string* err);
+    // The embedding of a split plan skips the blocks of samples that hold nothing below a
+    // node (d_held, from the structural bits) once the nodes that may be dense hold every block.
+    const uint32_t* held_ptr() const { return held_on ? d_held.as<uint32_t>() : nullptr; }
+    bool hold_dense(const DevMem& mask, std::string* err) {
+        if (!hw) return true;
+        SSU_HIP(launch_held_all(d_held.as<uint32_t>(), hw, d_knodes.as<int32_t>(), (uint32_t)knodes.size(),
+                                mask.as<uint32_t>(), st));
+        held_on = true;
+        return true;
+    }
+    uint32_t hw = 0;
+    bool held_on = false;
+    DevMem d_held;
     // presence bits of every node into dst, lb words per row (structural: every
     // stored entry counts as present)
     bool embed_bits(DevMem& dst, uint32_t lb, bool structural, std::string* err);
     // node-major FP64 embedding of sample columns [c0, c0 + w) into dst (row stride w)
-    bool embed(DevMem& dst, bool normalize, size_t c0, size_t w, std::string* err);
+    bool embed(DevMem& dst, bool normalize, size_t c0, size_t w, std::string* err, bool by_blocks = false);
     bool refine(const uint32_t* flags, std::string* err);
 };
 
@@ -686,6 +702,12 @@ bool PlanImpl::structural_counts(std::vector<uint32_t>& cnt, std::string* err) {
     if (lb <= BITS_MAX_WORDS) {
         DevMem& B = bits ? d_B : bits_tmp;   // the Gram path keeps its bit rows for the executions
         if (!embed_bits(B, lb, true, err)) return false;
+        const char* env = getenv("SSU_HELD_BLOCKS");   // 0: never, 1: always
+        if (!gram && use_paths && (env ? atoi(env) != 0 : (size_t)m * ldn * sizeof(double) >= HELD_MIN_BYTES)) {
+            hw = held_words(ldn);
+            if (!d_held.ensure((size_t)m * hw * sizeof(uint32_t), err)) return false;
+            SSU_HIP(launch_held_blocks(d_held.as<uint32_t>(), hw, B.as<uint32_t>(), lb, m, st));
+        }
         SSU_HIP(launch_count_bits(cnt_d.as<uint32_t>(), B.as<uint32_t>(), lb, d_knodes.as<int32_t>(), K, st));
     } else {
         if (!ones.ensure(std::max<uint64_t>(nnz, 1) * sizeof(double), err)) return false;
@@ -810,7 +832,7 @@ bool PlanImpl::split_weighted(std::string* err) {
         n_dense_max += cnt[q] >= thr;
     }
     // (members: the host copies outlive the uploads)
-    return upload(d_urare, urare, st, err) && upload(d_udense, udense, st, err);
+    return upload(d_urare, urare, st, err) && upload(d_udense, udense, st, err) && hold_dense(d_udense, err);
 }
 
 bool PlanImpl::upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std::string* err) {
@@ -902,7 +924,7 @@ bool PlanImpl::split_vaw(std::string* err) {
     // (members: the host copies outlive the uploads)
     return upload(d_vdense, vdense_mask, st, err) && upload(d_dlist, vdense, st, err) &&
            upload(d_tau, tau_h, st, err) && upload(d_kidx, kidx_h, st, err) && upload(d_vpts, vpts, st, err) &&
-           upload(d_vcos, vcos, st, err) && upload(d_vt, vt, st, err);
+           upload(d_vcos, vcos, st, err) && upload(d_vt, vt, st, err) && hold_dense(d_vdense, err);
 }
 
 bool PlanImpl::embed_bits(DevMem& dst, uint32_t lb, bool structural, std::string* err) {
@@ -923,15 +945,16 @@ bool PlanImpl::embed_bits(DevMem& dst, uint32_t lb, bool structural, std::string
     return true;
 }
 
-bool PlanImpl::embed(DevMem& dst, bool normalize, size_t c0, size_t w, std::string* err) {
+bool PlanImpl::embed(DevMem& dst, bool normalize, size_t c0, size_t w, std::string* err, bool by_blocks) {
     if (!dst.ensure(std::max<size_t>(m, 1) * blk * sizeof(double), err)) return false;
     double* E = dst.as<double>();
+    const uint32_t* held = by_blocks ? held_ptr() : nullptr;
     SSU_HIP(launch_embed_leaves(E, w, (uint32_t)c0, d_leaf_k.as<int32_t>(), d_leaf_row.as<int32_t>(),
                                 (uint32_t)leaf_k.size(), d_indptr.as<uint32_t>(), d_indices.as<uint32_t>(),
-                                data_ptr(), totals_ptr(), normalize, st));
+                                data_ptr(), totals_ptr(), normalize, st, held, hw));
     if (use_paths) {
         for (size_t r = 0; r + 1 < round_off.size(); ++r)
-            SSU_HIP(launch_embed_paths(E, w, hpaths(), round_off[r], round_off[r + 1], st));
+            SSU_HIP(launch_embed_paths(E, w, (uint32_t)c0, hpaths(), round_off[r], round_off[r + 1], st, held, hw));
         return true;
     }
     for (size_t h = 0; h + 1 < level_off.size(); ++h) {
@@ -1418,8 +1441,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
     const bool skip_rare = split && gather && single && !s.vaw && P.d_urare.p;
     for (size_t c0 = 0; c0 < P.ldn && !P.bits; c0 += P.blk) {
         const size_t w = std::min(P.blk, P.ldn - c0);
-        if (!P.embed(P.d_E, s.normalize, c0, w, err)) return false;
-        if (s.vaw && !P.embed(P.d_C, false, c0, w, err)) return false;  // raw counts, src/unifrac_cmp.cpp:250-251
+        if (!P.embed(P.d_E, s.normalize, c0, w, err, true)) return false;
+        if (s.vaw && !P.embed(P.d_C, false, c0, w, err, true)) return false;  // raw counts, src/unifrac_cmp.cpp:250-251
         if (single) SSU_HIP(P.mark(1));
         if (P.gram) {
             if (P.Kp)
@@ -1434,10 +1457,11 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                        P.d_Spart.as<double>(), split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
                                        split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.sparse && gather && !P.gen));
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.sparse && gather && !P.gen, P.held_ptr(), P.hw));
             if (gather && s.vaw)
                 SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
-                                           (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st));
+                                           (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st, nullptr, 0u, false,
+                                           false, P.held_ptr(), P.hw));
         }
     }
     if (!single && !P.bits) SSU_HIP(P.mark(1));   // blocked: embed and prep share one phase

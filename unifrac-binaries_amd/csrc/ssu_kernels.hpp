@@ -74,7 +74,8 @@ hipError_t launch_gather_square(float* sub, const float* out, uint32_t n, const 
 // E holds the sample columns [col0, col0 + ld) of the node-major embedding
 hipError_t launch_embed_leaves(double* E, size_t ld, uint32_t col0, const int32_t* leaf_k, const int32_t* leaf_row,
                                uint32_t n_leaves, const uint32_t* indptr, const uint32_t* indices, const double* data,
-                               const double* totals, bool normalize, hipStream_t st);
+                               const double* totals, bool normalize, hipStream_t st, const uint32_t* held = nullptr,
+                               uint32_t hw = 0);
 hipError_t launch_embed_level(double* E, size_t ldn, const int32_t* nodes, uint32_t n_nodes, const int32_t* child_ptr,
                               const int32_t* child_idx, hipStream_t st);
 
@@ -92,7 +93,16 @@ struct HeavyPaths {
     const int32_t* child_ptr;
     const int32_t* child_idx;
 };
-hipError_t launch_embed_paths(double* E, size_t ldn, const HeavyPaths& hp, uint32_t p0, uint32_t p1, hipStream_t st);
+hipError_t launch_embed_paths(double* E, size_t ldn, uint32_t col0, const HeavyPaths& hp, uint32_t p0, uint32_t p1,
+                              hipStream_t st, const uint32_t* held = nullptr, uint32_t hw = 0);
+// held: the blocks of 16 samples of each of m nodes that hold something, hw = held_words
+// words per node, from the nodes' presence bits; with it, launch_embed_leaves, _paths and
+// launch_gather_sums skip the other blocks (E is not written there).  launch_held_all
+// sets every bit of the rows r with bit r of mask.
+uint32_t held_words(size_t ldn);
+hipError_t launch_held_blocks(uint32_t* held, uint32_t hw, const uint32_t* B, uint32_t ldb, uint32_t m, hipStream_t st);
+hipError_t launch_held_all(uint32_t* held, uint32_t hw, const int32_t* knodes, uint32_t K, const uint32_t* mask,
+                           hipStream_t st);
 hipError_t launch_bits_paths(uint32_t* B, uint32_t ldb, const HeavyPaths& hp, uint32_t p0, uint32_t p1,
                              hipStream_t st);
 
@@ -130,7 +140,8 @@ hipError_t launch_gather_sums(float* U, size_t ldu, double* S, double* Spart, ui
                               const double* E,
                               size_t lde, uint32_t col0, const int32_t* knodes, const double* klen, uint32_t K,
                               uint32_t n, hipStream_t st, const uint32_t* rare_u = nullptr, uint32_t rps_fixed = 0,
-                              bool write_rare = false, bool scale_u = false);
+                              bool write_rare = false, bool scale_u = false, const uint32_t* held = nullptr,
+                              uint32_t hw = 0);
 // rows per segment that depends on K alone (for launch_gather_sums)
 uint32_t fixed_rows_per_segment(uint32_t K);
 // Faith PD: out[s] = sum over all non-root nodes k in postorder of (E[k][s] > 0) * len[k]

@@ -372,14 +372,18 @@ __global__ void __launch_bounds__(ST_T) k_coordinates(double* __restrict__ sampl
 
 // PERMANOVA permutations: row p > 0 of the labels is the p-th Fisher-Yates shuffle
 // of the grouping (row 0 the grouping itself), written sample major, Lt[i * ldp + p]
-// (columns past the rows: labels of no group).  One wave per row: its labels in LDS
-// as bytes, 64 draws at a time by its lanes, the exchanges in order by lane 0.
-// Bound by the exchanges' LDS round trips, every row at once: 999 shuffles of 2,500
-// labels 243 us, on the host 7 ms.
-constexpr uint32_t SHUF_MAX_N = 65536, SHUF_MAX_GROUPS = 256;
+// (columns past the rows: labels of no group).  One wave per row, its labels in LDS
+// as bytes, 64 exchanges at a time: a lane whose positions no earlier lane of the
+// batch touches is independent of those, so the lanes up to the first that is not
+// exchange at once, the rest in further rounds (`tag`: the first lane to touch a
+// position, by its low bits).  999 shuffles of 2,500 labels 90 us, 243 with the
+// exchanges one after another (their LDS round trips), on the host 7 ms.
+constexpr uint32_t SHUF_TAGS = 4096;
+constexpr uint32_t SHUF_MAX_N = 65536 - 4 * SHUF_TAGS, SHUF_MAX_GROUPS = 256;   // (64 KB of LDS)
 __global__ void __launch_bounds__(64) k_shuffles(uint32_t* __restrict__ Lt, const uint32_t* __restrict__ grouping,
                                                  uint32_t n, uint32_t n_lab, uint32_t ldp, uint64_t seed) {
-    extern __shared__ uint8_t lab[];
+    extern __shared__ uint32_t tag[];
+    uint8_t* lab = reinterpret_cast<uint8_t*>(tag + SHUF_TAGS);
     const uint32_t p = blockIdx.x, lane = threadIdx.x;
     if (p >= n_lab) {
         for (uint32_t i = lane; i < n; i += 64) Lt[(size_t)i * ldp + p] = 0xffffffffu;
@@ -392,13 +396,25 @@ __global__ void __launch_bounds__(64) k_shuffles(uint32_t* __restrict__ Lt, cons
         for (uint32_t top = n - 1; top > 0; top = top > 64 ? top - 64 : 0) {   // exchanges i = top .. max(1, top - 63)
             const uint32_t cnt = min(64u, top), i_l = top - min(lane, cnt - 1);
             const uint32_t j_l = (uint32_t)(mix64(key + i_l) % (i_l + 1));
-            for (uint32_t s = 0; s < cnt; ++s) {
-                const uint32_t i = top - s, j = (uint32_t)__builtin_amdgcn_readlane((int)j_l, (int)s);
-                if (lane == 0) {
-                    const uint8_t a = lab[i], b = lab[j];
-                    lab[i] = b;
-                    lab[j] = a;
+            for (uint32_t done = 0; done < cnt;) {   // (uniform)
+                const bool on = lane >= done && lane < cnt;
+                uint32_t *ti = tag + i_l % SHUF_TAGS, *tj = tag + j_l % SHUF_TAGS;
+                if (on) *ti = *tj = 64;
+                __syncthreads();
+                if (on) {
+                    atomicMin(ti, lane);
+                    atomicMin(tj, lane);
                 }
+                __syncthreads();
+                const uint64_t wait = __ballot(on && (*ti != lane || *tj != lane));   // (never the lane `done`)
+                const uint32_t end = wait ? (uint32_t)__builtin_ctzll(wait) : cnt;
+                if (on && lane < end) {
+                    const uint8_t a = lab[i_l], b = lab[j_l];
+                    lab[i_l] = b;
+                    lab[j_l] = a;
+                }
+                __syncthreads();
+                done = end;
             }
         }
         __syncthreads();
@@ -708,7 +724,7 @@ bool permanova_t(const void* mat, uint32_t n, const uint32_t* grouping, uint32_t
     if (n <= SHUF_MAX_N && groups <= SHUF_MAX_GROUPS) {
         if (!alloc(dg, (size_t)n * 4, err)) return false;
         ST_HIP(hipMemcpy(dg.p, grouping, (size_t)n * 4, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(k_shuffles, dim3(ldp), dim3(64), n, 0, dL.as<uint32_t>(), dg.as<const uint32_t>(), n, n_lab,
+        hipLaunchKernelGGL(k_shuffles, dim3(ldp), dim3(64), SHUF_TAGS * 4 + n, 0, dL.as<uint32_t>(), dg.as<const uint32_t>(), n, n_lab,
                            ldp, seed);
         ST_HIP(hipGetLastError());
     } else {   // more samples or groups than bytes in LDS hold

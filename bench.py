@@ -43,7 +43,7 @@ sys.path.insert(0, os.path.join(ROOT, "oracle"))
 
 PEAK_FP32_TFLOPS = 157.3    # MI355X published FP32 vector peak (packed FP32)
 PEAK_FP64_TFLOPS = 78.6     # MI355X published FP64 vector peak
-FLOPS_PER_TERM_SPARSE = 4   # sub, abs, fused multiply-add (the pair-node count of the stripe-kernel model)
+FLOPS_PER_TERM_SPARSE = 3   # FP32: sub, abs, add (the lengths are in the values); FP64: min, multiply-add
 PEAK_INT8_TOPS = 5000.0     # MI355X published dense INT8 MFMA peak, TOP/s
 PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth, GB/s
 GRAM_TILE = 128             # Gram output tile edge
@@ -453,7 +453,7 @@ def main():
         roofline = {"kernel": dom_kernel, "bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS,
                     "unit": "GB/s", "frac": achieved / PEAK_HBM_GBS, "traffic": None}
     elif dom_kernel in ("k_pairs_sparse", "k_pairs_sparse32"):
-        # executed work: the (pair, shared node) terms the kernel evaluated, 4 flops each (sub, abs, FMA)
+        # executed work: the (pair, dense node) terms the kernel evaluated
         peak = PEAK_FP64_TFLOPS if dom_kernel == "k_pairs_sparse" else PEAK_FP32_TFLOPS
         achieved = FLOPS_PER_TERM_SPARSE * dk["kernel_terms"] / (dom_ms / 1000.0) / 1e12
         roofline = {"kernel": dom_kernel, "bound": "valu", "achieved": achieved, "peak": peak,

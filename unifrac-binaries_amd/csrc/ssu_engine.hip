@@ -449,6 +449,10 @@ struct PlanImpl {
     bool gram = false;
     bool sparse = false;             // weighted (or generalized) through the shared-node kernels
     bool gen = false;                // generalized on the shared-node path
+    bool neg_len = false;            // (shared-node path) some length < 0
+    // FP32 weighted operand rows of the tiles hold l u: not with a negative length,
+    // whose l |u - v| is not |l u - l v|
+    bool scaled_rows() const { return sparse && !gen && !spec.fp64 && !neg_len; }
     // VAW on the shared-node path: nodes held by at least split_thr samples of the
     // plan's table (vdense_mask) stay with the pair tiles (vdense: their number, then
     // their indices), the others go to the posting lists; the one-sided sums are
@@ -801,10 +805,8 @@ bool PlanImpl::split_gram(std::string* err) {
 bool PlanImpl::split_weighted(std::string* err) {
     const char* env_theta = getenv("SSU_SPARSE_SPLIT");
     const double theta = env_theta ? atof(env_theta) : 1.0;
-    bool nonneg = true;
-    for (size_t q = 0; q < knodes.size(); ++q) nonneg = nonneg && (spec.fp64 ? klen_d[q] >= 0.0 : klen_f[q] >= 0.0f);
     const uint32_t K = (uint32_t)knodes.size();
-    if (!nonneg || !(theta > 0.0) || K == 0 || n < 2) return true;
+    if (neg_len || !(theta > 0.0) || K == 0 || n < 2) return true;
     std::vector<uint32_t> cnt;
     if (!structural_counts(cnt, err)) return false;
     // the threshold: SSU_SPARSE_SPLIT * n, or the cost model's choice on these
@@ -1220,8 +1222,11 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
             spec.alpha >= 0.0 && spec.alpha <= 1.0 && !(getenv("SSU_GEN_SPARSE") && atoi(getenv("SSU_GEN_SPARSE")) == 0);
     P.sparse = (weighted && !spec.vaw && spec.plain_kernel == 0) || P.gen;
     if (P.sparse) {
-        for (size_t q = 0; q < P.klen_d.size() && P.sparse; ++q)
-            if (!std::isfinite(spec.fp64 ? P.klen_d[q] : (double)P.klen_f[q])) P.sparse = false;
+        for (size_t q = 0; q < P.klen_d.size() && P.sparse; ++q) {
+            const double l = spec.fp64 ? P.klen_d[q] : (double)P.klen_f[q];
+            if (!std::isfinite(l)) P.sparse = false;
+            if (l < 0.0) P.neg_len = true;
+        }
         P.sparse = P.sparse && vals_nonneg;
     }
     P.gen = P.gen && P.sparse;
@@ -1457,7 +1462,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
                                        P.d_Spart.as<double>(), split ? P.d_smask.as<uint32_t>() : nullptr, P.d_E.as<double>(), w, (uint32_t)c0, P.d_knodes.as<int32_t>(),
                                        P.d_klen_sum.as<double>(), K, P.n, P.st,
                                        split && gather && P.d_urare.p ? P.d_urare.as<uint32_t>() : nullptr,
-                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.sparse && gather && !P.gen, P.held_ptr(), P.hw));
+                                       s.fixed_segments ? fixed_rows_per_segment(K) : 0u, !skip_rare, P.scaled_rows(), P.held_ptr(), P.hw));
             if (gather && s.vaw)
                 SSU_HIP(launch_gather_sums(P.d_Cu.as<float>(), P.ldn, nullptr, nullptr, nullptr, P.d_C.as<double>(), w,
                                            (uint32_t)c0, P.d_knodes.as<int32_t>(), nullptr, K, P.n, P.st, nullptr, 0u, false,
@@ -1623,6 +1628,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         a.U = s.fp64 ? P.d_E.p : P.d_U.p;
         a.rows = s.fp64 ? P.d_knodes.as<int32_t>() : nullptr;
         a.len = P.d_klen_sum.as<double>();
+        a.scaled = P.scaled_rows();
         a.ldn = P.ldn;
         a.dlist = P.d_dlist.as<uint32_t>();
         a.n = P.n;

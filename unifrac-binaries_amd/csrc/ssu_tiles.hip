@@ -56,14 +56,18 @@ __device__ __forceinline__ double ratio(double nm, double dn, double share, doub
 // Bound by VALU issue: 16,384 samples x 9,790 dense nodes in 44.9 ms, 2.94e13
 // terms/s of the 3.1e13 that sub + add reach in registers at two waves per SIMD;
 // 32 x 64 pairs per wave with lengths in the term, three LDS reads for 32 terms,
-// took 70.4 ms.
-struct OpW32 {
+// took 70.4 ms.  SCALED = false: l |u - v| of plain rows, for trees with a negative
+// length, whose sign |l u - l v| would lose.
+template <bool SCALED> struct OpW32 {
     typedef float V;
     static constexpr int RL = 8, CL = 8, WAVES = 2, EB = 16, UNROLL = 16;
-    static constexpr bool TWO = false, LEN = false, COUNTS = false, FLAGS = false;
+    static constexpr bool TWO = false, LEN = !SCALED, COUNTS = false, FLAGS = false;
     static constexpr uint32_t PANELS = 1;
     static __device__ __forceinline__ float prep(float u) { return u; }
-    static __device__ __forceinline__ void term(float u, float v, float, float& num) { num += __builtin_fabsf(u - v); }
+    static __device__ __forceinline__ void term(float u, float v, float l, float& num) {
+        if constexpr (SCALED) num += __builtin_fabsf(u - v);
+        else num = __builtin_fmaf(__builtin_fabsf(u - v), l, num);
+    }
     // d from the tile's sums x, y and the rare nodes' shares of them
     static __device__ __forceinline__ double distance(double x, double, double share, double, double tot,
                                                       bool normalized) {
@@ -558,7 +562,8 @@ template <class OP> static hipError_t launch_tiles(const TileArgs& a, hipStream_
 }
 
 hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st) {
-    return fp64 ? launch_tiles<OpW64>(a, st) : launch_tiles<OpW32>(a, st);
+    if (fp64) return launch_tiles<OpW64>(a, st);
+    return a.scaled ? launch_tiles<OpW32<true>>(a, st) : launch_tiles<OpW32<false>>(a, st);
 }
 
 template <class T> static hipError_t launch_gen(const TileArgs& a, hipStream_t st) {

@@ -51,7 +51,8 @@ struct TileArgs {
     const void* U;            // operand rows
     const int32_t* rows;      // FP64: operand row of processed node r (nullptr: r itself)
     size_t ldn;               // their stride, a multiple of the tile's edge
-    const double* len;        // [K] lengths (FP64 operands)
+    const double* len;        // [K] lengths
+    bool scaled;              // FP32 weighted: U's rows hold l u
     const uint32_t* dlist;    // dlist[0] = dense nodes, then their processed-node indices
     uint32_t n;
     const double* S;          // per-sample sums
@@ -71,7 +72,8 @@ struct TileArgs {
     uint32_t n_split;
 };
 // Weighted.  FP32: out_ij = (sum over the dense nodes of |x_i - x_j| + the rare
-// share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (U's rows are scaled).
+// share) / (S_i + S_j) (or the sum itself), x = l u in FP32 (scaled rows), or of
+// l |u_i - u_j| (plain rows).
 // FP64: x = S_i + S_j - 2 M in its place, M = sum of l min(u_i, u_j) + the rare
 // share, U the embedding (row rows[r] for processed node r).
 hipError_t launch_tiles_weighted(bool fp64, const TileArgs& a, hipStream_t st);

@@ -1438,7 +1438,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             SSU_HIP(launch_bits_smask(P.d_smask.as<uint32_t>(), P.d_B.as<uint32_t>(), P.ldb,
                                       P.d_sp_node.as<int32_t>(), Ks, npan, P.st));
     }
-    if (P.tiled && ((split && !P.d_dlist.ensure(((size_t)K + 1) * sizeof(uint32_t), err)) ||
+    // (VAW: the list uploaded with the plan stays; a larger request would drop it)
+    if (P.tiled && ((split && P.sparse && !P.d_dlist.ensure(((size_t)K + 1) * sizeof(uint32_t), err)) ||
                     !P.d_tws.ensure(std::max<size_t>(P.tset.slots * tile_slot_bytes(P.tile_rows()), 1), err)))
         return false;
     // one embedding block (E holds every sample): the postings of the FP32 split take their

@@ -42,8 +42,7 @@ def check(name, m, ref):
 
 
 CASES = [(m + p, kw) for m in METHODS for p in ("", "_fp64")
-         for kw in ({}, {"variance_adjust": True}, {"normalize": False})
-         if m + p != "generalized" or "variance_adjust" not in kw]
+         for kw in ({}, {"variance_adjust": True}, {"normalize": False})]
 
 
 @pytest.mark.parametrize("name,kw", CASES, ids=["-".join([m, *k]) for m, k in CASES])

@@ -97,3 +97,45 @@ def test_negative_lengths_rarefied(ssu, synth, O):
         for k, name in enumerate(names):
             check(name, b.matrix(k, rep), oracle_matrix(O, tree, drawn, name))
     b.close()
+
+
+@pytest.mark.parametrize("theta", ["0", "0.3", "1"])
+@pytest.mark.parametrize("name", ["weighted_normalized", "weighted_unnormalized", "generalized",
+                                  "weighted_normalized_fp64", "weighted_unnormalized_fp64", "generalized_fp64"])
+def test_negative_lengths_split(ssu, synth, O, monkeypatch, theta, name):
+    """Nodes of negative length stay on the tiles at any threshold of the split."""
+    monkeypatch.setenv("SSU_SPARSE_SPLIT", theta)
+    tree, table = negative_case(synth, 900, 200, 0.08, 6)
+    p = ssu.Plan(ssu.Inputs(*tree, *table), name, alpha=0.4)
+    p.execute()
+    check(name, p.matrix(), oracle_matrix(O, tree, table, name, alpha=0.4))
+    assert (p.sparse_terms() > 0) == (theta != "0")
+    p.close()
+
+
+@pytest.mark.parametrize("name,tol", [("weighted_unnormalized", 1e-6), ("weighted_unnormalized_fp64", 1e-11)])
+def test_negative_length_larger_than_the_rest(ssu, synth, O, monkeypatch, name, tol):
+    """A tip that holds half of every sample, with a negative length that takes away
+    most of the samples' sums (which then bound no sum of the other nodes) and
+    leaves the distances alone.  Rounding errors against the terms' magnitudes."""
+    monkeypatch.setenv("SSU_SPARSE_SPLIT", "1")   # every other node on the posting lists
+    (st, le, nm), (obs, smp, ip, ix, data) = synth.random_tree(400, 3), synth.random_table(400, 90, 0.1, 4)
+    tot = np.bincount(ix, data, 90)
+    one = oracle_matrix(O, (st, le, nm), (obs, smp, ip, ix, data), "weighted_unnormalized")
+    with np.errstate(invalid="ignore"):
+        pair = one / oracle_matrix(O, (st, le, nm), (obs, smp, ip, ix, data), "weighted_normalized")   # S_i + S_j
+    i, j, k = (np.arange(90) + s for s in range(3))
+    sums = (pair[i % 90, j % 90] + pair[i % 90, k % 90] - pair[j % 90, k % 90]) / 2
+    st = np.concatenate([[True], st, [True, False, False]])
+    le = np.concatenate([[0.0], le, [-0.95 * sums.min(), 0.0, 0.0]])
+    nm = [""] + list(nm) + ["half", "", ""]
+    table = (list(obs) + ["half"], smp, np.concatenate([ip, [ip[-1] + 90]]), np.concatenate([ix, np.arange(90)]),
+             np.concatenate([data, tot]))
+    ref = oracle_matrix(O, (st, le, nm), table, "weighted_unnormalized")
+    assert np.abs(ref - one / 2).max() < 1e-12
+    p = ssu.Plan(ssu.Inputs(st, le, nm, *table), name)
+    p.execute()
+    err = np.abs(p.matrix() - ref).max() / one.max()
+    print("[gpu-case] negative tip", name, "max err of the magnitudes", err, flush=True)
+    assert err <= tol
+    p.close()

@@ -797,8 +797,11 @@ bool PlanImpl::split_gram(std::string* err) {
 }
 
 // Shared-node weighted path: nodes held by fewer than theta * n samples are summed
-// from posting lists instead of the 32 x 64 tiles (decided per execution from
-// the actual occupancy).  Their postings at any execution number at most the
+// from posting lists instead of the pair tiles (decided per execution from
+// the actual occupancy).  A node of negative length stays on the tiles (the walk's
+// fixed point needs terms >= 0, and then S bounds nothing and the sums over the
+// listed nodes do): 8,000 samples x 50k tips, one length in 50 negative, 129 ms
+// (FP64 233) with every node on the tiles, 20.3 (32.5) this way.  Their postings at any execution number at most the
 // sum over nodes of min(structural occupancy, thr - 1); that bound sizes the
 // posting and row-list arrays and must stay below 2^30 (32-bit slot offsets in
 // the kernels): theta is lowered to fit.  SSU_SPARSE_SPLIT sets theta (0: off).
@@ -806,9 +809,13 @@ bool PlanImpl::split_weighted(std::string* err) {
     const char* env_theta = getenv("SSU_SPARSE_SPLIT");
     const double theta = env_theta ? atof(env_theta) : 1.0;
     const uint32_t K = (uint32_t)knodes.size();
-    if (neg_len || !(theta > 0.0) || K == 0 || n < 2) return true;
+    if (!(theta > 0.0) || K == 0 || n < 2) return true;
     std::vector<uint32_t> cnt;
     if (!structural_counts(cnt, err)) return false;
+    const auto listable = [&](uint32_t q) { return (spec.fp64 ? klen_d[q] : (double)klen_f[q]) >= 0.0; };
+    if (neg_len)   // (no choice there: left out of the model and of the slots)
+        for (uint32_t q = 0; q < K; ++q)
+            if (!listable(q)) cnt[q] = 0;
     // the threshold: SSU_SPARSE_SPLIT * n, or the cost model's choice on these
     // occupancies (generalized terms cost several times the weighted ones on the
     // tiles, which moves the balance)
@@ -830,8 +837,9 @@ bool PlanImpl::split_weighted(std::string* err) {
     udense.assign((K + 31) / 32, 0u);
     n_dense_max = 0;
     for (uint32_t q = 0; q < K; ++q) {
-        (cnt[q] < thr ? urare : udense)[q >> 5] |= 1u << (q & 31);
-        n_dense_max += cnt[q] >= thr;
+        const bool rare = cnt[q] < thr && (!neg_len || listable(q));
+        (rare ? urare : udense)[q >> 5] |= 1u << (q & 31);
+        n_dense_max += !rare;
     }
     // (members: the host copies outlive the uploads)
     return upload(d_urare, urare, st, err) && upload(d_udense, udense, st, err) && hold_dense(d_udense, err);
@@ -1485,7 +1493,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.src_fp64 = s.fp64 || skip_rare;
         b.ldu = P.ldn;
         b.len = P.d_klen_sum.as<double>();
-        b.S = P.S_ptr();
+        b.S = P.neg_len && !P.gen ? nullptr : P.S_ptr();
         b.out = P.out_ptr();
         b.out_fp64 = s.fp64;
         b.walked = P.d_walked.as<uint32_t>();
@@ -1509,7 +1517,8 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
         b.band = P.band;
         if (P.sparse) {
             b.dlist = P.d_dlist.as<uint32_t>();
-            if (gather && !P.gen && !skip_rare) b.fixed_dense = P.d_udense.as<uint32_t>();   // (their operand rows are scaled)
+            // (their operand rows are scaled; or some are dense for their length)
+            if ((gather && !P.gen && !skip_rare) || P.neg_len) b.fixed_dense = P.d_udense.as<uint32_t>();
         }
         if (vsplit) {
             const bool unw = s.method == Method::unweighted || s.method == Method::unweighted_unnormalized;

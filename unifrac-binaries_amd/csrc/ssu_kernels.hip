@@ -1483,8 +1483,8 @@ constexpr uint32_t SR_WALK = 1, SR_DIAG = 2;   // k_pairs_rows modes: the column
 // are accumulated in fixed point, integers in units of 2^(e - 51) (FP32
 // values: the FP64 product rounded to nearest by one FMA) or 2^(e - 61) (FP64
 // weighted values: l_r * min, and GRAM: l_r, truncated) where 2^e bounds the
-// row's sum of term magnitudes (S[a] weighted; 3 (ssp[a] + max ssp) GEN; the
-// FP64 sum of the row list's lengths unweighted).  Weighted partial sums go out in the value type.  Integer
+// row's sum of term magnitudes (weighted S[a], or ssp[a] where some length is
+// below 0; 3 (ssp[a] + max ssp) GEN; the FP64 sum of the row list's lengths unweighted).  Weighted partial sums go out in the value type.  Integer
 // adds make the result independent of the order in which waves and lanes add,
 // and two samples holding the same nodes get bit-equal G(a, b) and G(a, a).
 // Posting slots are addressed with 32-bit offsets (fewer than 2^30 slots).
@@ -2717,7 +2717,7 @@ static bool sparse_args_ok(const SparseNodesArgs& a) {
                         a.rbsum && a.npan == (a.n + 31) / 32 && a.slots < (1u << 30);
     if (!common) return false;
     if (a.gram) return a.n_pad >= a.n && a.n_pad % GRAM_BM == 0;   // unweighted: values, sums and out unused
-    return a.pcnt && a.obsum && a.thr && a.pval && a.U && (a.S || a.vaw) && a.out && a.out_fp64 == a.values_fp64 &&
+    return a.pcnt && a.obsum && a.thr && a.pval && a.U && (a.S || a.ssp || a.vaw) && a.out && a.out_fp64 == a.values_fp64 &&
            a.ldu >= (size_t)a.npan * 32 && (!a.vaw || (a.Cv && a.pcv));
 }
 
@@ -2785,9 +2785,10 @@ hipError_t launch_sparse_lists(const SparseNodesArgs& a, hipStream_t st) {
 template <class IX, bool GRAM, class TV, bool GEN = false, int VAW = 0>
 static void pairs_rows_t(uint32_t blocks, hipStream_t st, const SparseNodesArgs& a, uint32_t nchunks, uint32_t nkc,
                          uint32_t a0, uint32_t na, uint32_t mode) {
+    const double* bounds = a.S ? a.S : a.ssp;   // (weighted; a length below 0: S bounds nothing)
     hipLaunchKernelGGL((k_pairs_rows<TV, IX, GRAM, TV, GEN, VAW>), dim3(blocks), dim3(64 * SR_WAVES), 0, st,
                        GRAM ? nullptr : (TV*)a.out, a.walked, a.rows, a.roff, a.pc, (const IX*)a.pidx,
-                       GRAM ? nullptr : (const TV*)a.pval, a.len, GRAM ? nullptr : a.S, a.K, a.n, a.npan,
+                       GRAM ? nullptr : (const TV*)a.pval, a.len, GRAM ? nullptr : bounds, a.K, a.n, a.npan,
                        (const uint32_t*)a.poff, a.slots, nchunks, nkc, a.gram, a.n_pad / GRAM_BM, a.ssp,
                        (TV*)a.out2, a.pspmax, a.alpha, a.band, a0, na, mode, (const TV*)a.pcv, a.tot, a.H, a.D,
                        a.kidx);
@@ -2876,6 +2877,11 @@ hipError_t launch_sparse_rows(const SparseNodesArgs& a, hipStream_t st, uint32_t
         if (narrow) pairs_rows_t<uint16_t, true, float>((uint32_t)blocks, st, a, nchunks, nkc, row0, na, mode);
         else pairs_rows_t<uint32_t, true, float>((uint32_t)blocks, st, a, nchunks, nkc, row0, na, mode);
     } else if (a.values_fp64) {
+        if (!a.S) {   // the rows' bounds: their sums over the sparse nodes
+            if (!whole) return hipErrorInvalidValue;
+            hipLaunchKernelGGL((k_sparse_sums<double, false>), dim3(a.n), dim3(64), 0, st, a.ssp, a.rows, a.roff, nkc,
+                               (const uint32_t*)a.poff, (const double*)a.pval, a.len, a.K, a.n, a.slots, 0.0);
+        }
         if (narrow) pairs_rows_t<uint16_t, false, double>((uint32_t)blocks, st, a, nchunks, nkc, row0, na, mode);
         else pairs_rows_t<uint32_t, false, double>((uint32_t)blocks, st, a, nchunks, nkc, row0, na, mode);
     } else {

@@ -243,7 +243,7 @@ struct SparseNodesArgs {
     bool src_fp64 = false;  // (weighted) U holds FP64 rows (FP32 values: rounded when copied)
     size_t ldu;
     const double* len;      // [K]
-    const double* S;        // [n] (weighted)
+    const double* S;        // [n] (weighted) bounds of the rows' sums; nullptr: their sums over the sparse nodes (ssp)
     void* out;              // (weighted)
     bool out_fp64;
     uint32_t* walked;       // optional [sparse_rows_blocks(n)]: postings walked per wave
@@ -252,7 +252,7 @@ struct SparseNodesArgs {
     uint32_t* roff;         // [n * row_list_chunks(n, K) + 1]
     uint32_t* rbsum;        // [row_list_scan_blocks(n, K) + 1]
     uint32_t K, n, npan;
-    double* ssp = nullptr;  // (weighted, FP32 values) [n]: per-sample sum of l * u (GEN: l * u^alpha) over its sparse nodes
+    double* ssp = nullptr;  // (weighted, FP32 values or no S) [n]: per-sample sum of l * u (GEN: l * u^alpha) over its sparse nodes
     bool gen = false;       // generalized: numerator shares to out, denominator shares to out2
     double alpha = 1.0;
     void* out2 = nullptr;

@@ -241,9 +241,9 @@ struct InmemInputs {
     uint32_t matched = 0, distinct = 0;   // table ids that name a leaf, of how many
     bool tree_ok = false;
     double input_ms = 0.0, tree_ms = 0.0;   // (overlapped)
-    InmemInputs(const support_biom_t* td, const support_bptree_t* tr) {
+    InmemInputs(const support_biom_t* td, const support_bptree_t* tr, bool upload = true) {
         const auto t0 = Clock::now();
-        if (ssu::device_available(nullptr))
+        if (upload && ssu::device_available(nullptr))
             pre = ssu::TableUpload::start(td->indptr, td->indices, td->data, (uint32_t)td->n_obs);
         std::thread tree_thread([&] {
             const auto t1 = Clock::now();
@@ -424,21 +424,27 @@ ComputeStatus faith_result(const Table& t, const ssu::PostorderNodes& nodes,
     return okay;
 }
 
-ComputeStatus faith_common(const Table& t0, const PhyloTree& tree, r_vec** result) {
-    // src/api.cpp:569-604: drop zero-count samples (total < 1), shear, Faith PD
-    if (t0.n_samples == 0 || t0.n_obs == 0) return table_empty;
-    Table nz = t0.filtered(1.0);
+// Faith PD of t0 without its zero-count samples (total < 1, src/api.cpp:569-604): nz
+// is what the filter leaves, nodes() its sheared tree.
+template <class F>
+ComputeStatus faith_filtered(const Table& t0, const Table& nz, F nodes, r_vec** result) {
     const bool degenerate = nz.n_samples == 0 || nz.n_obs == 0;
     if (degenerate) fprintf(stderr, "WARNING: All samples had zero counts. Forcing zero result.\n");
     else if (nz.n_samples != t0.n_samples || nz.n_obs != t0.n_obs)
         fprintf(stderr, "WARNING: Some samples had zero counts and were filtered out.\n");
-    if (!degenerate) return faith_result(nz, synced_nodes(nz, tree), nullptr, result);
+    if (!degenerate) return faith_result(nz, nodes(), nullptr, result);
     r_vec* r = (r_vec*)malloc(sizeof(r_vec));
     r->n_samples = t0.n_samples;
     r->values = (double*)calloc(t0.n_samples ? t0.n_samples : 1, sizeof(double));
     r->sample_ids = dup_ids(t0.sample_ids);
     *result = r;
     return okay;
+}
+
+ComputeStatus faith_common(const Table& t0, const PhyloTree& tree, r_vec** result) {
+    if (t0.n_samples == 0 || t0.n_obs == 0) return table_empty;
+    const Table nz = t0.filtered(1.0);
+    return faith_filtered(t0, nz, [&] { return synced_nodes(nz, tree); }, result);
 }
 
 }  // namespace
@@ -750,28 +756,30 @@ ComputeStatus faith_pd_one_off(const char* biom_filename, const char* tree_filen
 ComputeStatus ssu_faith_pd_inmem(const support_biom_t* td, const support_bptree_t* tr, r_vec** result) {
     if (!td || !tr || td->n_samples <= 0 || td->n_obs <= 0) return table_empty;
     // The overlapped path of the in-memory matrices (the table's CSR and the tree on
-    // threads of their own, the table borrowed, no id maps or copies), for tables that
-    // the filter below leaves as they are: every total >= 1, an entry in every row.
-    // 4,000 samples x 20,000 tips (1.7e6 entries): 3.5 ms against 19 ms with the table
-    // filtered into a copy and the tree sheared and collapsed node by node.
+    // threads of their own, the table borrowed, no id maps).  A table that the filter
+    // leaves as it is (every total >= 1, an entry in every row) needs no copy: 4,000
+    // samples x 20,000 tips (1.7e6 entries) 3.7 ms.  Otherwise its entries are filtered
+    // and, where rows went too, the tree's arrays are walked once more for those left.
     bool rows_held = true;
     for (int i = 0; i < td->n_obs && rows_held; ++i) rows_held = td->indptr[i + 1] > td->indptr[i];
-    if (rows_held) {
-        InmemInputs in(td, tr);
-        bool whole = in.table.index_ok;
-        for (uint32_t s = 0; s < in.table.n_samples && whole; ++s) whole = in.table.totals[s] >= 1.0;
-        if (whole) {
-            if (!in.tree_ok) return tree_missing;
-            if (in.matched < in.distinct) return table_and_tree_do_not_overlap;
-            return faith_result(in.table, in.nodes, in.pre, result);
-        }
-    }
-    Table t = Table::borrow(td->obs_ids, td->sample_ids, td->indptr, td->indices, td->data, (uint32_t)td->n_obs,
-                            (uint32_t)td->n_samples);
-    PhyloTree tree = PhyloTree::from_arrays(tr->structure, tr->lengths, tr->names, tr->n_parens);
-    ComputeStatus st = validate(t, tree);
-    if (st != okay) return st;
-    return faith_common(t, tree, result);
+    InmemInputs in(td, tr, rows_held);
+    if (!in.tree_ok) return tree_missing;
+    if (in.matched < in.distinct) return table_and_tree_do_not_overlap;
+    bool whole = rows_held && in.table.index_ok;
+    for (uint32_t s = 0; s < in.table.n_samples && whole; ++s) whole = in.table.totals[s] >= 1.0;
+    if (whole) return faith_result(in.table, in.nodes, in.pre, result);
+    std::vector<uint32_t> rows;
+    const Table nz = in.table.filtered(1.0, &rows);
+    return faith_filtered(in.table, nz, [&] {
+        if (rows.size() == in.table.n_obs) return std::move(in.nodes);   // (the same rows)
+        std::vector<const char*> ids;
+        for (uint32_t i : rows) ids.push_back(td->obs_ids[i]);
+        ssu::NameIndex idx(ids.data(), (uint32_t)ids.size());
+        ssu::PostorderNodes nodes;
+        uint32_t matched = 0;   // (the tree was seen to be whole)
+        (void)ssu::synced_postorder(tr->structure, tr->lengths, tr->names, (uint32_t)tr->n_parens, idx, nodes, matched);
+        return nodes;
+    }, result);
 }
 
 // =================================================================== partial

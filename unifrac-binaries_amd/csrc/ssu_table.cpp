@@ -166,26 +166,41 @@ Table Table::dense_pair(const char* const* oids, const double* s1, const double*
     return own(std::move(o), std::move(s), std::move(ip), std::move(ix), std::move(d));
 }
 
-Table Table::filtered(double min_total) const {
+Table Table::filtered(double min_total, std::vector<uint32_t>* rows) const {
     std::vector<int64_t> new_index(n_samples, -1);
-    std::vector<std::string> sids;
+    Table t;
     for (uint32_t s = 0; s < n_samples; ++s)
-        if (totals[s] >= min_total) { new_index[s] = (int64_t)sids.size(); sids.push_back(sample_ids[s]); }
-    std::vector<std::string> oids;
-    std::vector<uint32_t> ip{0}, ix;
-    std::vector<double> d;
-    if (!sids.empty()) {
+        if (totals[s] >= min_total) {
+            new_index[s] = (int64_t)t.sample_ids.size();
+            t.sample_ids.push_back(sample_ids[s]);
+        }
+    std::vector<uint32_t>&ip = t.own_indptr_, &ix = t.own_indices_;
+    std::vector<double>& d = t.own_data_;
+    if (rows) rows->clear();
+    ip.push_back(0);
+    if (!t.sample_ids.empty()) {
+        ix.reserve(nnz());
+        d.reserve(nnz());
         for (uint32_t i = 0; i < n_obs; ++i) {
-            const size_t before = ix.size();
             for (uint32_t j = indptr[i]; j < indptr[i + 1]; ++j) {
                 const int64_t ni = indices[j] < n_samples ? new_index[indices[j]] : -1;
                 if (ni >= 0) { ix.push_back((uint32_t)ni); d.push_back(data[j]); }
             }
-            if (ix.size() > before) { oids.push_back(obs_ids[i]); ip.push_back((uint32_t)ix.size()); }
+            if (ix.size() > ip.back()) {
+                if (rows) rows->push_back(i);
+                else t.obs_ids.push_back(obs_ids[i]);
+                ip.push_back((uint32_t)ix.size());
+            }
         }
     }
-    if (oids.empty()) sids.clear();  // degenerate: nothing left (src/biom_inmem.cpp:332-337)
-    return own(std::move(oids), std::move(sids), std::move(ip), std::move(ix), std::move(d));
+    t.n_obs = (uint32_t)ip.size() - 1;
+    if (t.n_obs == 0) t.sample_ids.clear();  // degenerate: nothing left (src/biom_inmem.cpp:332-337)
+    t.n_samples = (uint32_t)t.sample_ids.size();
+    t.indptr = ip.data();
+    t.indices = ix.data();
+    t.data = d.data();
+    t.finish(!rows);
+    return t;
 }
 
 }  // namespace ssu

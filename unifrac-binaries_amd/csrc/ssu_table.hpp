@@ -35,8 +35,9 @@ struct Table {
     static Table dense_pair(const char* const* obs_ids, const double* s1, const double* s2, uint32_t n_obs);
 
     // Drop samples whose total is below min_total, then observations left
-    // without entries (src/biom_inmem.cpp:83-128, 284-338).
-    Table filtered(double min_total) const;
+    // without entries (src/biom_inmem.cpp:83-128, 284-338).  rows (a table borrowed
+    // without its ids): takes the kept observations' row numbers in place of their ids.
+    Table filtered(double min_total, std::vector<uint32_t>* rows = nullptr) const;
 
     Table() = default;
     Table(const Table&) = delete;             // the CSR pointers may point into own storage

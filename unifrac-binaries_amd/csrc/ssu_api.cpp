@@ -763,7 +763,7 @@ ComputeStatus ssu_faith_pd_inmem(const support_biom_t* td, const support_bptree_
     bool rows_held = true;
     for (int i = 0; i < td->n_obs && rows_held; ++i) rows_held = td->indptr[i + 1] > td->indptr[i];
     InmemInputs in(td, tr, rows_held);
-    if (!in.tree_ok) return tree_missing;
+    if (!in.tree_ok) return tr->n_parens > 0 ? tree_missing : table_and_tree_do_not_overlap;   // (no node at all: no leaf)
     if (in.matched < in.distinct) return table_and_tree_do_not_overlap;
     bool whole = rows_held && in.table.index_ok;
     for (uint32_t s = 0; s < in.table.n_samples && whole; ++s) whole = in.table.totals[s] >= 1.0;

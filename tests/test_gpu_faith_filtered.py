@@ -60,3 +60,21 @@ def test_faith_nothing_left(ssu, synth):
     obs, smp, ip, ix, data = synth.random_table(50, 20, 0.2, 2)
     status, vals, ids = ssu.faith_pd_inmem(ssu.Inputs(st, le, nm, obs, smp, ip, ix, np.full(len(data), 1e-3)))
     assert status == ssu.OKAY and ids == list(smp) and not vals.any()
+
+
+@pytest.mark.parametrize("values", [(5e-324, 1e8), (1e-310, 1e20), (1e308, 1.7e308)], ids=["least", "subnormal", "overflow"])
+def test_faith_of_proportions_that_vanish(ssu, synth, O, values):
+    """A value whose proportion underflows to 0, or of a total that overflows, does not
+    count as present: a node held only through it adds nothing."""
+    st, le, nm = synth.random_tree(60, 5)
+    obs, smp, ip, ix, data = synth.random_table(60, 30, 0.2, 6)
+    ip, ix, data = np.asarray(ip), np.asarray(ix), np.array(data, float)
+    own = np.nonzero(ix == ix[0])[0]
+    data[own] = 2.0
+    data[own[::2]], data[own[1::2]] = values
+    table = (obs, smp, ip, ix, data)
+    status, vals, _ = ssu.faith_pd_inmem(ssu.Inputs(st, le, nm, *table))
+    ref = O.faith_pd(O.Tree(st.astype(np.uint8), le, nm), O.Table(*table))
+    assert status == ssu.OKAY and np.array_equal(vals, ref)
+    full = O.faith_pd(O.Tree(st.astype(np.uint8), le, nm), O.Table(obs, smp, ip, ix, np.ones(data.size)))
+    assert ref[ix[0]] < full[ix[0]]

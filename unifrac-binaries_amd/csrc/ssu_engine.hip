@@ -1079,6 +1079,19 @@ ComputeSpec spec_for_table(const Table& t, ComputeSpec s) {
     return s;
 }
 
+// Whether every positive value of the table (all of them finite and >= 0) is a
+// positive proportion of its sample in FP64 too: no total overflows, and the
+// smallest value (at least 1 where all are whole) over the largest total does not
+// underflow.
+static bool proportions_positive(const Table& t) {
+    double most = 0.0, least = 1.0;
+    for (double x : t.totals) most = std::max(most, x);
+    if (!t.values_integral)
+        for (uint64_t j = t.indptr[0]; j < t.indptr[t.n_obs]; ++j)
+            if (t.data[j] > 0.0 && t.data[j] < least) least = t.data[j];
+    return std::isfinite(most) && least / std::max(most, 1.0) > 0.0;
+}
+
 std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nodes, const ComputeSpec& spec,
                                    std::string* err, const std::shared_ptr<TableUpload>& pre) {
     if (!device_available(err)) return nullptr;
@@ -1215,6 +1228,7 @@ std::unique_ptr<Plan> Plan::create(const Table& table, const PostorderNodes& nod
     if ((P.gram || spec.faith) && P.ldn / 32 <= BITS_MAX_WORDS) {
         bool ok_vals = vals_nonneg;
         for (size_t k = 0; k < P.len_all.size() && spec.faith && ok_vals; ++k) ok_vals = std::isfinite(P.len_all[k]);
+        if (spec.faith && ok_vals) ok_vals = proportions_positive(table);
         if (const char* env = getenv("SSU_GRAM_BITS")) ok_vals = ok_vals && atoi(env) != 0;
         if (ok_vals) {
             P.bits = true;

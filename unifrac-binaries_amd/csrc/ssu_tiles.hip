@@ -481,7 +481,7 @@ __global__ void __launch_bounds__(DL_T) k_dense_list(uint32_t* __restrict__ dlis
 // whole; the tiles left over, which would leave most of the XCD idle for one
 // more round, are cut into np parts over the nodes, np the cheapest of
 // ceil(left * np / resident) rounds of 1 / np of a tile each plus the cost of
-// writing and reading the parts' sums.
+// writing and reading the parts' sums, of those whose slots fit TILE_WS_BYTES.
 TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes) {
     const uint32_t resident = tile_resident(rows), cols = rows;
     TileSet t;
@@ -498,6 +498,7 @@ TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes) {
     // a part is at least 64 nodes; writing and reading one costs about as much as 24 nodes' terms
     const uint32_t most = std::max<uint32_t>(1, std::min<uint32_t>(TILE_MAX_PARTS, max_nodes / 64));
     const double part_cost = max_nodes ? 24.0 / max_nodes : 1.0;
+    const size_t most_slots = TILE_WS_BYTES / N_XCDS / tile_slot_bytes(rows);   // of an XCD
     std::vector<std::vector<TileUnit>> xcd(N_XCDS);
     size_t at = 0;
     for (uint32_t x = 0; x < N_XCDS; ++x) {
@@ -505,7 +506,7 @@ TileSet tile_set(uint32_t n, uint32_t rows, uint32_t max_nodes) {
         const size_t left = count % resident, whole = count - left;
         uint32_t np = 1;
         double best = left ? 1.0 : 0.0;
-        for (uint32_t q = 2; q <= most && left; ++q) {
+        for (uint32_t q = 2; q <= most && left && left * q <= most_slots; ++q) {
             const double cost = (double)((left * q + resident - 1) / resident) * (1.0 / q + part_cost);
             if (cost < 0.97 * best) { best = cost; np = q; }
         }

@@ -45,6 +45,7 @@ bool alloc(Buf& b, size_t bytes, std::string* err) {
 }
 
 constexpr uint32_t ST_T = 256;
+constexpr uint32_t MAX_GRID_Y = 65535;
 
 // Sum over the workgroup, the same order every time.
 __device__ __forceinline__ double block_sum(double v, double* part) {
@@ -164,16 +165,17 @@ __host__ __device__ uint64_t mix64(uint64_t z) {
 
 // X[i][c] = a standard normal from two counter-based uniforms (Box-Muller), index i k + c; 0 past k
 __global__ void __launch_bounds__(64) k_probes(double* __restrict__ X, uint32_t k, uint32_t ld, uint64_t seed) {
-    const uint32_t i = blockIdx.x, c = blockIdx.y * 64 + threadIdx.x;
-    if (c >= ld) return;
-    double x = 0.0;
-    if (c < k) {
-        const uint64_t idx = (uint64_t)i * k + c;
-        const double u1 = ((mix64(seed ^ mix64(2 * idx)) >> 11) + 1) * 0x1.0p-53;   // (0, 1]
-        const double u2 = (mix64(seed ^ mix64(2 * idx + 1)) >> 11) * 0x1.0p-53;
-        x = sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
+    const uint32_t i = blockIdx.x;
+    for (uint32_t c = blockIdx.y * 64 + threadIdx.x; c < ld; c += gridDim.y * 64) {
+        double x = 0.0;
+        if (c < k) {
+            const uint64_t idx = (uint64_t)i * k + c;
+            const double u1 = ((mix64(seed ^ mix64(2 * idx)) >> 11) + 1) * 0x1.0p-53;   // (0, 1]
+            const double u2 = (mix64(seed ^ mix64(2 * idx + 1)) >> 11) * 0x1.0p-53;
+            x = sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
+        }
+        X[(size_t)i * ld + c] = x;
     }
-    X[(size_t)i * ld + c] = x;
 }
 
 // R (q x q, column major, zero below its diagonal r) from above the diagonal of the n x q matrix A
@@ -361,13 +363,15 @@ __global__ void __launch_bounds__(QR_T) k_qr_small(double* __restrict__ A, doubl
 __global__ void __launch_bounds__(ST_T) k_coordinates(double* __restrict__ samples, const double* __restrict__ Q,
                                                       const double* __restrict__ W, uint32_t n, uint32_t q,
                                                       uint32_t used, uint32_t dims) {
-    const uint32_t i = blockIdx.x * ST_T + threadIdx.x, d = blockIdx.y;
+    const uint32_t i = blockIdx.x * ST_T + threadIdx.x;
     if (i >= n) return;
-    double u = 0.0;
-    if (d < used)
+    for (uint32_t d = blockIdx.y; d < dims; d += gridDim.y) {
+        double u = 0.0;
+        if (d < used)
 #pragma unroll 8
-        for (uint32_t c = 0; c < q; ++c) u += Q[(size_t)c * n + i] * W[(size_t)d * q + c];
-    samples[(size_t)i * dims + d] = u;
+            for (uint32_t c = 0; c < q; ++c) u += Q[(size_t)c * n + i] * W[(size_t)d * q + c];
+        samples[(size_t)i * dims + d] = u;
+    }
 }
 
 // PERMANOVA permutations: row p > 0 of the labels is the p-th Fisher-Yates shuffle
@@ -616,8 +620,9 @@ bool center_on_device(Buf& dB, const void* mat, uint32_t n, std::vector<double>&
 // Y = B X, X and Y n x ld row major (device)
 template <class T>
 bool symm_mult(double* Y, const Buf& dB, const double* X, uint32_t n, uint32_t ld, std::string* err) {
-    hipLaunchKernelGGL((k_symm_mult<T>), dim3((n + 15) / 16, ld / 16), dim3(64 * SM_WAVES), 0, 0, Y, dB.as<const T>(),
-                       X, n, ld);
+    for (uint32_t c0 = 0; c0 < ld; c0 += MAX_GRID_Y * 16)
+        hipLaunchKernelGGL((k_symm_mult<T>), dim3((n + 15) / 16, std::min(MAX_GRID_Y, (ld - c0) / 16)),
+                           dim3(64 * SM_WAVES), 0, 0, Y + c0, dB.as<const T>(), X + c0, n, ld);
     ST_HIP(hipGetLastError());
     return true;
 }
@@ -667,7 +672,7 @@ bool pcoa_t(const void* mat, uint32_t n, uint32_t dims, uint64_t seed, double* e
         return false;
     double *X = dX.as<double>(), *Y = dY.as<double>(), *H = dH.as<double>(), *V = dV.as<double>(), *Q = dQ.as<double>();
     double* r = dr.as<double>();
-    hipLaunchKernelGGL(k_probes, dim3(n, (ldk + 63) / 64), dim3(64), 0, 0, X, k, ldk, seed);
+    hipLaunchKernelGGL(k_probes, dim3(n, std::min(MAX_GRID_Y, (ldk + 63) / 64)), dim3(64), 0, 0, X, k, ldk, seed);
     ST_HIP(hipGetLastError());
     for (uint32_t level = 0; level <= PCOA_LEVELS; ++level) {
         // level 0: Y = B G; then Y = B (B Y_prev)
@@ -707,7 +712,7 @@ bool pcoa_t(const void* mat, uint32_t n, uint32_t dims, uint64_t seed, double* e
     if (!alloc(dW, W.size() * 8, err)) return false;
     ST_HIP(hipMemcpy(dW.p, W.data(), W.size() * 8, hipMemcpyHostToDevice));
     if (!alloc(dS, (size_t)n * dims * 8, err)) return false;
-    hipLaunchKernelGGL(k_coordinates, dim3(nb, dims), dim3(ST_T), 0, 0, dS.as<double>(), Q, dW.as<const double>(), n, q,
+    hipLaunchKernelGGL(k_coordinates, dim3(nb, std::min(MAX_GRID_Y, dims)), dim3(ST_T), 0, 0, dS.as<double>(), Q, dW.as<const double>(), n, q,
                        used, dims);
     ST_HIP(hipGetLastError());
     ST_HIP(hipMemcpy(samples, dS.p, (size_t)n * dims * 8, hipMemcpyDeviceToHost));

@@ -861,10 +861,13 @@ bool PlanImpl::upload_tiles(const TileSet& t, DevMem& units, DevMem& split, std:
 // totals of its own takes them at every sample's).  The [n][D] sums must fit
 // VAW_H_BUDGET; SSU_VAW_SPLIT sets theta (0: off).
 // The totals the one-sided sums are taken at: the distinct totals where they are
-// few, Chebyshev points over their range where so many as hold the sums to FP64
-// rounding are at most VAW_POINTS - 1 (N terms leave 4 rho^-N / (rho - 1) of the
-// sums' size), otherwise (or where the terms are rounded to FP32, generalized
-// FP32) none: every total.  SSU_VAW_POINTS=0 turns them off.
+// few; for FP32 names Chebyshev points over their range where so many as hold the sums
+// to FP64 rounding of their largest value are at most VAW_POINTS - 1 (N terms leave
+// 4 rho^-N / (rho - 1) of it); otherwise (or where the terms are rounded to FP32,
+// generalized FP32) none: every total.  A series' rounding does not leave the small
+// distances as the sums' own does (terms the walk takes back out bit for bit): entries
+// of FP64 names were up to 4.6e-12 off with one, 1.1e-14 at every total, so they take
+// none.  SSU_VAW_POINTS=0 turns them off.
 void PlanImpl::vaw_points() {
     vpts.clear();
     vcos.clear();
@@ -875,6 +878,7 @@ void PlanImpl::vaw_points() {
     if (spec.method == Method::generalized && !spec.fp64) return;
     const size_t D = tau_h.size();
     if (D <= VAW_POINTS) { vpts = tau_h; return; }
+    if (spec.fp64) return;
     const bool zero = !(tau_h[0] > 0.0);
     const double lo = tau_h[zero ? 1 : 0], hi = tau_h[D - 1];
     if (!(lo > 0.0) || !std::isfinite(hi)) return;

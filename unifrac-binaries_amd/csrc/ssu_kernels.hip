@@ -2121,7 +2121,7 @@ __global__ void __launch_bounds__(64) k_vaw_onesided(double* __restrict__ H, uin
 // The same sums without one pass per total.  As a function of the total t, a
 // one-sided term is (A + t)^(-1/2) (or -alpha/2) with A >= 0, analytic but for
 // t <= 0, so over totals from lo > 0 to hi a polynomial in log t of few degrees
-// holds H(a, .) to FP64 rounding: with 2L = log(hi / lo), the Chebyshev series
+// holds H(a, .) to FP64 rounding of its largest value (FP32 names): with 2L = log(hi / lo), the Chebyshev series
 // falls as rho^-N, rho = b + sqrt(1 + b^2), b = pi / L (totals within a factor of
 // 20: 27 terms).  k_vaw_points sums at the N Chebyshev points and forms the
 // coefficients (vN > 0), or sums at the totals themselves where those are few

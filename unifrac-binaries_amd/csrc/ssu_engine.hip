@@ -1673,6 +1673,7 @@ bool Plan::execute_into(const double* d_data, const double* d_totals, void* d_ou
             a.C = s.fp64 ? P.d_C.p : P.d_Cu.p;
             a.totals = P.totals_ptr();
         }
+        a.band = P.band;
         if (!mark_vaw(a)) return false;
         a.ws = P.d_tws.as<double>();
         const uint32_t nbands = P.banded_run ? (uint32_t)P.band_ev.size() : 1;

@@ -229,7 +229,7 @@ __device__ __forceinline__ void write_pair(const TileArgs& g, size_t i, size_t j
     if constexpr (OP::FLAGS) {
         // unnormalised: near-duplicates (distance below flag_tau of the pair's VAW
         // denominator) marked for the FP64 recomputation
-        if (g.flags && d < (double)g.flag_tau * (y + share2)) {
+        if (g.flags && g.band.has((uint32_t)(j - i)) && d < (double)g.flag_tau * (y + share2)) {
             g.flags[1 + i] = 1u;
             g.flags[1 + j] = 1u;
             atomicAdd(g.flags, 1u);

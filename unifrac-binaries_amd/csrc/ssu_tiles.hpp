@@ -3,6 +3,8 @@
 // and the launchers.
 #pragma once
 
+#include "ssu_kernels.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -69,7 +71,8 @@ struct TileArgs {
     const void* C;            // VAW: count rows, as U
     const double* totals;     // VAW: the samples' totals
     uint32_t* flags;          // unnormalised VAW weighted: marks of near-duplicates (below
-    float flag_tau;           //   flag_tau of the pair's VAW denominator), as launch_flag_close's
+    float flag_tau;           //   flag_tau of the pair's VAW denominator), as launch_flag_close's,
+    GapBand band;             //   among the pairs of the band (the others' shares are not there)
     double* ws;               // workspace slots of tile_slot_bytes
     const TileUnit* units;
     uint32_t n_units, per_xcd;

@@ -453,11 +453,14 @@ def main():
         roofline = {"kernel": dom_kernel, "bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS,
                     "unit": "GB/s", "frac": achieved / PEAK_HBM_GBS, "traffic": None}
     elif dom_kernel in ("k_pairs_sparse", "k_pairs_sparse32"):
-        # executed work: the (pair, dense node) terms the kernel evaluated
+        # executed work: the (pair, dense node) terms the kernel evaluated, two instructions each
+        # (the absolute value is an operand's modifier, counted as the third operation)
         peak = PEAK_FP64_TFLOPS if dom_kernel == "k_pairs_sparse" else PEAK_FP32_TFLOPS
         achieved = FLOPS_PER_TERM_SPARSE * dk["kernel_terms"] / (dom_ms / 1000.0) / 1e12
         roofline = {"kernel": dom_kernel, "bound": "valu", "achieved": achieved, "peak": peak,
-                    "unit": "TFLOP/s", "frac": achieved / peak, "traffic": None}
+                    "unit": "TFLOP/s", "frac": achieved / peak, "traffic": None,
+                    "device_kernel": "k_tiles<OpW64>" if dom_kernel == "k_pairs_sparse" else "k_tiles<OpW32<true>>",
+                    "flops_per_term": FLOPS_PER_TERM_SPARSE, "instructions_per_term": 2}
     else:
         achieved = FLOPS_PER_PAIR_NODE_W * pair_nodes[dom] / (dom_ms / 1000.0) / 1e12
         roofline = {"kernel": dom_kernel, "bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS,

@@ -510,9 +510,6 @@ struct PlanImpl {
     // rows in the band (band 0 also every diagonal tile), the posting walk of its
     // rows (after band 0's tiles: the diagonal G(a, a) of every row) and the
     // banded combine of its rows, in order on st.
-    // (an embedding the 256 MB memory-side cache holds gains nothing: one-off weighted calls of 106
-    // and 266 MB 2 - 3% slower for the bits, of 492 MB equal or 3% faster, resident plans of 1 GB 6%)
-    static constexpr size_t HELD_MIN_BYTES = size_t(256) << 20;
     static constexpr uint32_t OUT_BANDS = 10, OUT_BANDS_GRAM = 16;
     std::vector<uint32_t> band_row0, band_off;   // rows [band_row0[k], band_row0[k + 1]); blocks [band_off[k], ..)
     std::vector<hipEvent_t> band_ev;
@@ -601,6 +598,9 @@ struct PlanImpl {
         held_on = true;
         return true;
     }
+    // (an embedding that the 256 MB memory-side cache holds gains nothing: one-off weighted calls of 106
+    // and 266 MB 2 - 3% slower for the bits, of 492 MB equal or 3% faster, resident plans of 1 GB 6%)
+    static constexpr size_t HELD_MIN_BYTES = size_t(256) << 20;
     uint32_t hw = 0;
     bool held_on = false;
     DevMem d_held;
@@ -1791,8 +1791,8 @@ bool Plan::refine(const double* d_data, const double* d_totals, void* d_out, con
 
 bool Plan::refines() const { return p_->refine_on; }
 
-// Bands of about equal row counts, in whole block rows (32 FP32 / 64 FP64
-// samples; Gram: 128-sample tile rows, band 0 holding every diagonal tile).
+// Bands of about equal row counts, in whole tile rows (tile_rows(): 128 samples
+// weighted, 64 generalized and VAW; Gram: 128, band 0 holding every diagonal tile).
 bool PlanImpl::prepare_bands(std::string* err) {
     if (!band_ev.empty()) return true;
     const uint32_t ei = gram ? GRAM_BM : tile_rows();
@@ -2119,7 +2119,8 @@ double Plan::split_theta() const {
     if (P.gram) return P.gsplit_slots ? P.split_theta : 0.0;
     return P.split_thr ? (double)P.split_thr / std::max<uint32_t>(P.n, 1) : 0.0;
 }
-// (the names of the paths; programs compare them)
+// The names of the paths, which programs compare: "k_pairs_sparse32", "k_pairs_sparse",
+// "k_pairs_gen32" and "k_pairs_gen64" are those whose dense nodes run on k_tiles.
 const char* Plan::main_kernel() const {
     if (p_->gram) return "k_gram_i8r";
     if (p_->sparse)

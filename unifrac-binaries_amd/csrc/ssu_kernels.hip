@@ -27,9 +27,6 @@ inline unsigned grid1(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b)
 
 // ------------------------------------------------------------------ embedding
 
-// One workgroup per leaf: clear the row (16-byte stores; ld is even), then
-// scatter the leaf's CSR row (src/biom_inmem.cpp:473-497: value / total, or
-// the raw value).  E holds the sample columns [col0, col0 + ld) of the embedding.
 // what lanes with nothing to load read, so that a batch's loads need no branches
 static __device__ __align__(128) double2 zero_line;
 
@@ -74,6 +71,9 @@ __global__ void __launch_bounds__(256) k_held_all(uint32_t* __restrict__ held, u
     for (uint32_t w = 0; w < hw; ++w) held[(size_t)knodes[r] * hw + w] = 0xffffffffu;
 }
 
+// One workgroup per leaf: clear the row (16-byte stores; ld is even), then
+// scatter the leaf's CSR row (src/biom_inmem.cpp:473-497: value / total, or
+// the raw value).  E holds the sample columns [col0, col0 + ld) of the embedding.
 __global__ void __launch_bounds__(EMB_THREADS) k_embed_leaves(double* __restrict__ E, size_t ld, uint32_t col0,
                                                               const int32_t* __restrict__ leaf_k,
                                                               const int32_t* __restrict__ leaf_row,

@@ -3,10 +3,15 @@
 // Every dense node is held by a sizeable share of the samples, so every pair
 // block visits it: the kernels are dense contractions with |x_i - x_j| in
 // place of the product, which no matrix instruction forms.  They are laid out
-// like a vector-ALU GEMM: a tile is a workgroup of 2 x 2 waves, a lane holding its rows and columns in groups of 16 bytes, a group
-// apart from the next lane's, so that its operands are ds_read_b128 of 8
-// distinct contiguous pieces (no bank conflicts, each piece broadcast to 8 lanes).  Node rows go from memory
-// to LDS by global_load_lds, 16 bytes per lane, a stage of nodes ahead.
+// like a vector-ALU GEMM: a tile is a workgroup of 2 x 2 waves, a lane holding its
+// rows and columns in groups of 16 bytes, a group apart from the next lane's, so that
+// its operands are ds_read_b128 of 8 distinct contiguous pieces (no bank conflicts,
+// each piece broadcast to 8 lanes).  Node rows go from memory to LDS by
+// global_load_lds, 16 bytes per lane, a stage of nodes ahead.  Only the scaled FP32
+// weighted kernel waits for them at the barrier: in the others the next nodes' indices
+// and lengths (or, with a rolled node loop, the first read of a stage buffer that the
+// compiler cannot tell from the other one) have a wave wait before its terms, and what
+// overlaps the loads are the terms of the CU's other waves.
 #include "ssu_devmath.hpp"
 #include "ssu_tiles.hpp"
 
@@ -79,9 +84,11 @@ template <bool SCALED> struct OpW32 {
 
 // FP64 weighted: M = sum of l min(u, v), of which the distance is S_i + S_j - 2 M
 // (u, v >= 0; v_min_f64 without the NaN quieting the compiler adds for values it
-// does not see produced).  Bound by FP64 issue (half the FP32 rate): 3,001
-// samples x 3,700 dense nodes in 1.62 ms, against 2.66 ms in 64 x 64 blocks of one
-// wave; 131 samples 0.37 -> 0.04 ms, the parts filling the device.
+// does not see produced).  3,001 samples x 3,700 dense nodes in 1.62 ms, 1.1e13
+// terms/s: 58% of the 1.9e13 at which the two instructions issue (half the FP32 rate);
+// the rest are the waits for a v_min's result in the instruction after it and for the
+// next stage.  64 x 64 blocks of one wave took 2.66 ms; 131 samples 0.37 -> 0.04 ms,
+// the parts filling the device.
 struct OpW64 {
     typedef double V;
     static constexpr int RL = 8, CL = 8, WAVES = 2, EB = 8, UNROLL = 8;

@@ -44,7 +44,8 @@ Rates rates_of(SplitKind k, double alpha) {
     // VAW: the tiles' term; a posting (three FP64 reciprocal square roots); a one-sided term at
     // one total (or point).  4,000 samples, theta 0.2 .. 0.8: tiles 9.37 .. 2.09 ms, posting phase
     // 2.78 .. 14.3 (totals 14.3, 13.2 at 0.3, 13.5 at 0.4, 18.5); FP64, 2,000 samples: 6.42 .. 1.67
-    // and 1.28 .. 5.90 (8.63, 7.48 at 0.4, 8.49); the one-sided rate from the sums at every total
+    // and 1.28 .. 5.90 (sums at few points: 8.63, 7.48 at 0.4, 8.49; 1,500 samples at every total:
+    // 5.42 at 0.2, 5.19 at the model's 0.29, 5.43 at 0.42); the one-sided rate from the sums at every total
     // of the 8,192-sample workload.  Weighted and presence terms are within 15% of each other; the
     // weighted rates are used for both
     case SplitKind::vaw32: return {2.65e-13, 2.37e-12, 4.13e-13};
